@@ -66,25 +66,19 @@ def kernel_model(kname, info, D, sweeps, family=None, nqc=0):
         # reads the cell's origin, Jacobian and coefficient (the built-in
         # source is evaluated at the quadrature points); writes b_i
         return "hbm", 8 * (D + D * D + 1 + ni), "byte"
-    if kname == "flux_ref":
-        # writes R [nr][nr+1] and the kept block A_uu; reads the cell
-        # coefficients (72) and b_i
-        return "hbm", 8 * (nr * (nr + 1) + nu * nu + 72 + ni), "byte"
-    if kname == "reduced_rowlu" or (kname == "condense_grid" and family in (8, 10)):
-        # the reduced elimination of the flux families (row-per-lane, or the
-        # grid kernel for other sizes): reads R; writes S, g, U (packed),
-        # multipliers, pivot order, Y
-        return "hbm", 8 * (nr * (nr + 1) + nb * nb + nb + nu * (nu + 1) // 2 + nu * nu + nu
+    if kname == "condense_tile":
+        # the tile elimination of the flux families' reduced systems: reads the
+        # cell coefficients (72) and b_i; writes S, g, U (packed), the kept block
+        # A_uu of one potential component, R_uu^-1 and Y
+        nq = nu // (1 if nu * D == na else D)
+        return "hbm", 8 * (72 + ni + nb * nb + nb + nu * (nu + 1) // 2 + nq * nq + nu * nu
                            + (nb + 1) * nu), "byte"
     if kname == "recover_flux":
-        # reads A_uu, R_uu^-1, U^-1, Y (and, for the MFMA-product family, the
-        # kept A_qu and A_uq), the cell coefficients and b_i, the cell's trace
-        # values and ids; writes (q, u)
+        # reads A_uu, R_uu^-1 (and, for the MFMA-product family, the kept A_qu
+        # and A_uq), the cell coefficients and b_i, the cell's trace values and
+        # ids; writes (q, u)
         kept = 0 if family == 10 else 2 * na * nu
-        return "hbm", (8 * (3 * nu * nu + kept + (nb + 1) * nu + 72 + ni + nb + ni)
-                       + 4 * nb), "byte"
-    if kname == "flux_invert":
-        return "hbm", 8 * (nu * (nu + 1) // 2 + nu * nu + nu + 2 * nu * nu), "byte"
+        return "hbm", 8 * (2 * nu * nu + kept + 72 + ni + nb + ni) + 4 * nb, "byte"
     if kname == "assemble":
         # reads every S block once; writes the CSC values
         return "hbm", 8 * nb * nb + 8 * int(info.nnz) / nc, "byte"

@@ -740,7 +740,8 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
     // tables: one allocation, doubles first then bytes
     std::vector<const std::vector<double>*> dv = {&th.Mpp, &th.Gpq, &th.Gqp, &th.Fqp, &th.Fqq,
                                                    &th.Fpm, &th.Fqm, &th.Fmm, &th.Bp, &th.Bq,
-                                                   &th.xq, &th.fb_minv, &th.fr_P, &th.fr_G};
+                                                   &th.xq, &th.fb_minv, &th.fr_uu, &th.fr_ub,
+                                                   &th.fr_bb, &th.fr_qm, &th.fr_hm, &th.fr_G};
     size_t nd = 0;
     for (auto* v : dv) nd += v->size();
     size_t bytes = nd * sizeof(double) + th.prog_val.size() * sizeof(double) +
@@ -823,7 +824,8 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
     T.n = th.n;
     T.nqc = th.nqc;
     const double** ptrs[] = {&T.Mpp, &T.Gpq, &T.Gqp, &T.Fqp, &T.Fqq, &T.Fpm, &T.Fqm,
-                             &T.Fmm, &T.Bp,  &T.Bq,  &T.xq,  &T.fb_minv, &T.fr_P, &T.fr_G};
+                             &T.Fmm, &T.Bp,  &T.Bq,  &T.xq,  &T.fb_minv, &T.fr_uu, &T.fr_ub,
+                             &T.fr_bb, &T.fr_qm, &T.fr_hm, &T.fr_G};
     for (size_t i = 0; i < dv.size(); ++i) *ptrs[i] = reinterpret_cast<const double*>(base + offs[i]);
     T.pmask = reinterpret_cast<const uint8_t*>(base + off_pm);
     T.qmask = reinterpret_cast<const uint8_t*>(base + off_qm);
@@ -845,7 +847,6 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
     std::memcpy(T.fb_cid, th.fb_cid, sizeof(T.fb_cid));
     if (th.fb_minv.empty()) T.fb_minv = nullptr;
     T.fr_npair = th.fr_npair;
-    if (th.fr_npair == 0) T.fr_P = T.fr_G = nullptr;
   }
   m->x0.assign(desc->x0, desc->x0 + nc * D);
   m->jac.assign(desc->jac, desc->jac + nc * D * D);
@@ -858,11 +859,8 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
             J[6] * (J[1] * J[5] - J[2] * J[4]);
     }
     if (!(std::fabs(det) > 0.0)) return fail(ctx, HDG_ERR_ARG, "degenerate cell " + std::to_string(c));
-    // the reference flux decomposition assumes positively oriented cells
-    if (det < 0.0) {
-      m->tdev.fr_npair = 0;
-      m->tdev.fr_P = m->tdev.fr_G = nullptr;
-    }
+    // the Darcy reference flux decomposition assumes positively oriented cells
+    if (det < 0.0 && th.phys == kDarcy) m->tdev.fr_npair = 0;
   }
   std::vector<double> coef(desc->coef, desc->coef + nc);
   HIP_TRY(ctx, upload(m->d_x0, m->x0, st), "upload x0");
@@ -1580,8 +1578,8 @@ int recover_facet_major(hdg_mesh* m, const double* lam_free, double* free_values
   }
   if (m->used_family == kFamilyFluxSchur || m->used_family == kFamilyFluxRef) {
     const CellLayout L(m->th);
-    HIP_TRY(ctx, launch_recover_flux(m->tdev, m->meshdev(), m->pU, m->pY, (int64_t)L.U,
-                                     (int64_t)L.Y, m->used_family == kFamilyFluxRef,
+    HIP_TRY(ctx, launch_recover_flux(m->tdev, m->meshdev(), m->pU, (int64_t)L.U,
+                                     m->used_family == kFamilyFluxRef,
                                      m->d_cell_dofs.as<int32_t>(), lam_free,
                                      m->d_lam_dir.as<double>(), free_values, m->nfree,
                                      ctx->stream),

@@ -844,46 +844,57 @@ void detect_flux_sym(TablesHost& t) {
   t.fb_sym = 1 | (su < 0 ? 2 : 0) | (sb < 0 ? 4 : 0);
 }
 
-// Reference decomposition of the Darcy flux Schur complement (family 10).
-// The program's flux rows (a, i) of [A_qu A_qb] are
-//   A_qu: sum_e alpha[1 + e D + a] Gpq(e, i, j),  alpha[1 + e D + a] = -c_ea,
-//   A_qb: alpha[10 + 3F + a] Fpm(F, i, m),        alpha[10 + 3F + a] = aF nF_a,
-// and on an affine cell with det J > 0 the facet area times normal is the
-// cofactor image of the reference normal, aF nF_a = sum_e c_ea nhat_Fe.  So the
-// row block of component a is sum_e c_ea G_e with the reference matrices
-//   G_e[i][j] = -Gpq(e, i, j) (potential columns),
-//   G_e[i][(F, m)] = nhat_Fe Fpm(F, i, m) (trace columns),
-// and, C being (detJ/kappa) I = alpha_0 I, the flux Schur term
-//   [A_qu A_qb]^T (C^-1 (x) M^-1) [A_qu A_qb]
-//     = (1/alpha_0) sum_(e<=e') (sum_a c_ea c_e'a) P_(e,e').
-// Computed once here in long double.
+// Reference decomposition of the flux Schur complement (families 8 and 10).
+// With the cofactors c_ea = |det J| Ji(e, a) the program's flux rows are, per
+// flux component, combinations of the reference matrices G_e (scalar flux basis
+// against the scalar potential and trace bases):
+//   Darcy, component a:              [A_qu A_qb] = sum_e c_ea G_e,
+//     G_e[i][j] = -Gpq(e, i, j),  G_e[i][(F, m)] =  nhat_Fe Fpm(F, i, m);
+//   elasticity, stress component s = (p, q), displacement component d in s with
+//   partner a (the other one of p, q): sum_e c_ea G_e,
+//     G_e[i][j] =  Gpq(e, i, j),  G_e[i][(F, m)] = -nhat_Fe Fpm(F, i, m)
+// (on an affine cell the facet area times normal is the cofactor image of the
+// reference normal nhat; for Darcy the cells have det J > 0).  The flux block is
+// C (x) M, so the flux Schur term of two columns is a combination, with
+// per-cell weights W(e, e'), of the fixed matrices H_ee' = G_e^T M^-1 G_e', of
+// which a trace column meets only the direction its facet fixes.  Computed once
+// here in long double:
+//   fr_uu  H_ee' on the potential columns: Darcy (one component, symmetric
+//          weights) the sums over the pairs e <= e', else all (e, e');
+//   fr_ub  H_(e, fix(F)) on potential x trace columns [e][i][(F, m)];
+//   fr_bb  H_(fix(F), fix(F')) on the trace columns;
+//   fr_qm  Fqm as [i][(F, m)];
+//   fr_hm  (Darcy) H_e = M^-1 G_e [e][i][column], for a flux right-hand side;
+//   fr_G   G_e.
 void build_flux_ref(TablesHost& t) {
   t.fr_npair = 0;
-  t.fr_P.clear();
-  t.fr_G.clear();
-  const int D = t.D, np = t.np, nq = t.nq, nm = t.nm, nF = t.nF;
-  if (t.phys != kDarcy || t.fb_nc != D || (t.fb_sym & 1) == 0 || t.fb_minv.empty()) return;
-  // s_u = -1 (the integrated-by-parts u-q block), s_b = +1
-  if ((t.fb_sym & 6) != 2) return;
-  for (int a = 0; a < D; ++a)
-    for (int b = 0; b < D; ++b)
-      if (t.fb_cid[6 * a + b] != (a == b ? 0 : -1)) return;  // C = alpha_0 I
-  const int nr = nq + nF * nm;
-  // the kernel keeps at most three program terms per entry of R0 in registers
-  for (int c = t.na; c < t.n; ++c)
-    for (int r = t.na; r < t.n; ++r) {
-      const size_t e = (size_t)c * t.n + r;
-      if (t.prog_off[e + 1] - t.prog_off[e] > 3) return;
-    }
+  for (auto* v : {&t.fr_uu, &t.fr_ub, &t.fr_bb, &t.fr_qm, &t.fr_hm, &t.fr_G}) v->clear();
+  const int D = t.D, np = t.np, nq = t.nq, nm = t.nm, nF = t.nF, nbs = nF * nm;
+  const bool darcy = t.phys == kDarcy;
+  if ((t.fb_sym & 1) == 0 || t.fb_minv.empty()) return;
+  if (darcy) {
+    // s_u = -1 (the integrated-by-parts u-q block), s_b = +1, C = alpha_0 I
+    if (t.fb_nc != D || (t.fb_sym & 6) != 2) return;
+    for (int a = 0; a < D; ++a)
+      for (int b = 0; b < D; ++b)
+        if (t.fb_cid[6 * a + b] != (a == b ? 0 : -1)) return;
+  } else {
+    // s_u = s_b = -1, C the compliance in the first 36 coefficients
+    if (t.fb_nc != D * (D + 1) / 2 || (t.fb_sym & 6) != 6) return;
+    for (int a = 0; a < t.fb_nc; ++a)
+      for (int b = 0; b < t.fb_nc; ++b)
+        if (t.fb_cid[6 * a + b] != 6 * a + b) return;
+  }
+  const int nr = nq + nbs;
+  const long double sg = darcy ? -1.0L : 1.0L;
   std::vector<long double> G((size_t)D * np * nr, 0.0L);
   for (int e = 0; e < D; ++e)
     for (int i = 0; i < np; ++i) {
       for (int j = 0; j < nq; ++j)
-        G[((size_t)e * np + i) * nr + j] = -(long double)t.Gpq[((size_t)e * np + i) * nq + j];
+        G[((size_t)e * np + i) * nr + j] = sg * (long double)t.Gpq[((size_t)e * np + i) * nq + j];
       for (int F = 0; F < nF; ++F) {
-        const int fix = D - 1 - F / 2;
-        if (fix != e) continue;
-        const long double nh = (F % 2) ? 1.0L : -1.0L;
+        if (D - 1 - F / 2 != e) continue;
+        const long double nh = (F % 2) ? -sg : sg;
         for (int m = 0; m < nm; ++m)
           G[((size_t)e * np + i) * nr + nq + F * nm + m] =
               nh * (long double)t.Fpm[((size_t)F * np + i) * nm + m];
@@ -893,29 +904,45 @@ void build_flux_ref(TablesHost& t) {
   std::vector<long double> H((size_t)D * np * nr, 0.0L);
   for (int e = 0; e < D; ++e)
     for (int i = 0; i < np; ++i)
-      for (int c = 0; c < nr; ++c) {
-        long double v = 0.0L;
-        for (int k = 0; k < np; ++k)
-          v += (long double)t.fb_minv[(size_t)i * np + k] * G[((size_t)e * np + k) * nr + c];
-        H[((size_t)e * np + i) * nr + c] = v;
+      for (int k = 0; k < np; ++k) {
+        const long double m = t.fb_minv[(size_t)i * np + k];
+        for (int c = 0; c < nr; ++c)
+          H[((size_t)e * np + i) * nr + c] += m * G[((size_t)e * np + k) * nr + c];
       }
-  const int npair = D * (D + 1) / 2;
-  t.fr_P.assign((size_t)npair * nr * nr, 0.0);
+  auto dot = [&](int e, int r, int e2, int c) {
+    long double v = 0.0L;
+    for (int i = 0; i < np; ++i)
+      v += G[((size_t)e * np + i) * nr + r] * H[((size_t)e2 * np + i) * nr + c];
+    return v;
+  };
+  auto fix = [&](int b) { return D - 1 - (b / nm) / 2; };
+  t.fr_npair = darcy ? D * (D + 1) / 2 : D * D;
+  t.fr_uu.assign((size_t)t.fr_npair * nq * nq, 0.0);
   int p = 0;
   for (int e = 0; e < D; ++e)
-    for (int e2 = e; e2 < D; ++e2, ++p)
-      for (int r = 0; r < nr; ++r)
-        for (int c = 0; c < nr; ++c) {
-          long double v = 0.0L;
-          for (int i = 0; i < np; ++i) {
-            v += G[((size_t)e * np + i) * nr + r] * H[((size_t)e2 * np + i) * nr + c];
-            if (e2 != e) v += G[((size_t)e2 * np + i) * nr + r] * H[((size_t)e * np + i) * nr + c];
-          }
-          t.fr_P[((size_t)p * nr + r) * nr + c] = (double)v;
+    for (int e2 = darcy ? e : 0; e2 < D; ++e2, ++p)
+      for (int r = 0; r < nq; ++r)
+        for (int c = 0; c < nq; ++c) {
+          long double v = dot(e, r, e2, c);
+          if (darcy && e2 != e) v += dot(e2, r, e, c);
+          t.fr_uu[((size_t)p * nq + r) * nq + c] = (double)v;
         }
-  t.fr_G.resize(G.size());
+  t.fr_ub.assign((size_t)D * nq * nbs, 0.0);
+  for (int e = 0; e < D; ++e)
+    for (int r = 0; r < nq; ++r)
+      for (int b = 0; b < nbs; ++b)
+        t.fr_ub[((size_t)e * nq + r) * nbs + b] = (double)dot(e, r, fix(b), nq + b);
+  t.fr_bb.assign((size_t)nbs * nbs, 0.0);
+  for (int b = 0; b < nbs; ++b)
+    for (int b2 = 0; b2 < nbs; ++b2)
+      t.fr_bb[(size_t)b * nbs + b2] = (double)dot(fix(b), nq + b, fix(b2), nq + b2);
+  t.fr_qm.assign((size_t)nq * nbs, 0.0);
+  for (int r = 0; r < nq; ++r)
+    for (int b = 0; b < nbs; ++b)
+      t.fr_qm[(size_t)r * nbs + b] = t.Fqm[((size_t)(b / nm) * nq + r) * nm + b % nm];
+  t.fr_G.assign(G.size(), 0.0);
   for (size_t k = 0; k < G.size(); ++k) t.fr_G[k] = (double)G[k];
-  t.fr_npair = npair;
+  if (darcy) t.fr_hm.assign(H.begin(), H.end());
 }
 
 }  // namespace hdg

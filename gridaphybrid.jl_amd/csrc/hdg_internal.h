@@ -70,16 +70,16 @@ struct TablesHost {
   // A_uq = s_u A_qu^T and A_bq = s_b A_qb^T entry by entry, bit 1: s_u = -1,
   // bit 2: s_b = -1.
   int fb_sym = 0;
-  // Reference decomposition of the flux Schur complement for Darcy on affine
-  // cells (build_flux_ref): with c_ea = detJ Ji(e, a) the cofactor entries of
-  // the cell, [A_qu A_qb] row block of component a = sum_e c_ea G_e, so
-  //   [A_qu A_qb]^T (C^-1 (x) M^-1) [A_qu A_qb] = (1 / alpha_0) sum_p w_p P_p,
-  // w over the pairs (e, e') of sum_a c_ea c_e'a and P_(e,e) = G_e^T M^-1 G_e,
-  // P_(e,e') = G_e^T M^-1 G_e' + its transpose.  fr_npair = 0 when it does not
-  // apply (not Darcy, or no symmetric scalar flux block).
+  // Reference decomposition of the flux Schur complement on affine cells
+  // (build_flux_ref, which describes the matrices).  nbs = nF nm scalar trace
+  // functions.  fr_npair = 0 when it does not apply.
   int fr_npair = 0;
-  std::vector<double> fr_P;  // [npair][nr][nr] row-major, nr = nq + nb
-  std::vector<double> fr_G;  // [D][np][nr]  G_e
+  std::vector<double> fr_uu;  // [npair][nq][nq]
+  std::vector<double> fr_ub;  // [D][nq][nbs]
+  std::vector<double> fr_bb;  // [nbs][nbs]
+  std::vector<double> fr_qm;  // [nq][nbs]
+  std::vector<double> fr_hm;  // [D][np][nq + nbs] (Darcy)
+  std::vector<double> fr_G;   // [D][np][nq + nbs]
 };
 
 // Device view of the tables (pointers into one device allocation).
@@ -119,8 +119,12 @@ struct Tables {
   const double* fb_minv;  // [np][np] inverse of the scalar flux mass matrix
   int fb_sym;             // transpose symmetry of the flux coupling (TablesHost::fb_sym)
   int fr_npair;           // reference flux Schur decomposition (TablesHost::fr_*), 0: none
-  const double* fr_P;     // [npair][nr][nr]
-  const double* fr_G;     // [D][np][nr]
+  const double* fr_uu;
+  const double* fr_ub;
+  const double* fr_bb;
+  const double* fr_qm;
+  const double* fr_hm;
+  const double* fr_G;
 };
 
 // Device view of a mesh for the fused element generator.
@@ -151,12 +155,10 @@ struct CondenseOut {
   // (nb+1) ni); the flux-block path stores the reduced factors in the
   // per-cell slots of the full interior so every family shares one layout
   int64_t u_stride = 0, y_stride = 0;
-  // (grid elimination kernels) the multipliers and the pivot order, for
-  // solves with other right-hand sides: L[cell * u_stride + j * ni + r] =
-  // multiplier of interior row r at step j (rows pivoted later than j),
-  // P[cell * u_stride + k] = the row at LAPACK position k
-  double* L = nullptr;
-  double* P = nullptr;
+  // (tile elimination, per cell at cell * u_stride) A_ii^-1 and, from the
+  // reference products, the kept block A_uu, both [col][row]
+  double* Rinv = nullptr;
+  double* Auu = nullptr;
 };
 
 // Dense cell systems in HBM for the map-level API.
@@ -257,13 +259,14 @@ struct SysShape {
   int flux_na = 0;
   bool flux = false;
   bool ref = false;    // the reference decomposition applies (family 10)
+  int flux_keep = 0;   // flux unknowns of the kept blocks A_qu, A_uq (Darcy's family 8)
 };
 SysShape sys_shape(const Tables& T);
 SysShape sys_shape(const TablesHost& t);
 // Doubles per cell of the factor slot ("U"): ni(ni+1)/2 for the elimination
 // families; for classes where the flux-block path applies, room for its
 // reduced factors and the interior blocks its recovery refines with:
-//   [U m(m+1)/2][L m*m][P m][A_uu m*m][A_qu na*m][A_uq m*na],  m = ni - na.
+//   [U m(m+1)/2][A_uu m*m][A_qu na*m][A_uq m*na][R_uu^-1 m*m],  m = ni - na.
 size_t factor_slot(const SysShape& sh);
 // Family id of the flux-block Schur complement: the flux unknowns are
 // eliminated through C^-1 (x) M^-1 and the reduced system of the remaining
@@ -272,9 +275,10 @@ size_t factor_slot(const SysShape& sh);
 constexpr int kFamilyFluxSchur = 8;
 // (family 9, a fused variant of family 8 that never won a class, is removed;
 // its number stays reserved)
-// Family 10: the flux elimination of family 8 with the reduced system formed
-// from the reference decomposition (TablesHost::fr_*) instead of two MFMA
-// products per cell (Darcy on cells with det J > 0).
+// Family 10: the flux elimination of Darcy (cells with det J > 0) with the
+// reduced system formed from the reference decomposition (TablesHost::fr_*)
+// instead of family 8's two MFMA products per cell.  Elasticity's family 8 is
+// formed that way too.
 constexpr int kFamilyFluxRef = 10;
 // kernel families able to condense a class; returns their count
 int condense_variants(const SysShape& sh, int* fams, int max);
@@ -284,14 +288,12 @@ int condense_grid_options(int fam, int* gm, int max);
 size_t condense_workspace_bytes(const SysShape& sh, int fam, int64_t ncells);
 hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                 hipStream_t st, Workspace& ws, int gridmul, bool ref);
-// Recovery after a flux-block condensation (families 8 and 10): x_u =
-// U^-1 (y - Y lambda) from the reduced factors, x_q = (C^-1 (x) M^-1)(b_q -
-// A_qu x_u - A_qb lambda); then
-// FP64 refinement against the residual of the full interior system (the
-// reduced system is worse conditioned than A_ii).
-hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U,
-                               const double* Y, int64_t usz, int64_t ysz, bool ref,
-                               const int32_t* cell_dofs, const double* lam_free,
+// Recovery after a flux-block condensation (families 8 and 10): the structured
+// solve through R_uu^-1 and C^-1 (x) M^-1, refined in FP64 against the residual
+// of the full interior system (the reduced system is worse conditioned than
+// A_ii).
+hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, int64_t usz,
+                               bool ref, const int32_t* cell_dofs, const double* lam_free,
                                const double* lam_dir, double* out, int64_t nfree,
                                hipStream_t st);
 constexpr int kFluxRefineSteps = 2;  // FP64 refinement steps of the flux recovery (at most)

@@ -596,7 +596,6 @@ __global__ void __launch_bounds__(PR * PC)
           const bool use = ((act >> r) & 1u) && row != p;
           const double lv = use ? colv[r] * rinv : 0.0;
           s_lcol[buf][row] = lv;
-          if (out.L && use && row < ni) out.L[cell * out.u_stride + (int64_t)j * ni + row] = lv;
         }
         if (tr == 0) {
           s_piv[buf] = p;
@@ -641,8 +640,6 @@ __global__ void __launch_bounds__(PR * PC)
     }
     __syncthreads();  // last step's pivot row / multipliers fully consumed
     const int info = s_info;
-    if (out.P)
-      for (int k = tid; k < ni; k += NT) out.P[cell * out.u_stride + k] = (double)s_at[k];
 
     // ---------------- back substitution (backward map only) ---------------
     if (BACKSUB) {
@@ -902,6 +899,16 @@ __device__ inline int64_t wave_max_i64(int64_t x) {
 // max over the wavefront of nonnegative doubles (ordered like their bit patterns)
 __device__ inline double wave_max_f64(double x) {
   return __longlong_as_double(wave_max_i64(__double_as_longlong(x)));
+}
+__device__ inline int wave_max_i32(int x) {
+  int y;
+  y = __builtin_amdgcn_update_dpp(x, x, 0x121, 0xf, 0xf, false); x = max(x, y);
+  y = __builtin_amdgcn_update_dpp(x, x, 0x122, 0xf, 0xf, false); x = max(x, y);
+  y = __builtin_amdgcn_update_dpp(x, x, 0x124, 0xf, 0xf, false); x = max(x, y);
+  y = __builtin_amdgcn_update_dpp(x, x, 0x128, 0xf, 0xf, false); x = max(x, y);
+  y = __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false); x = max(x, y);
+  y = __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false); x = max(x, y);
+  return __builtin_amdgcn_readlane(x, 63);
 }
 __device__ inline int wave_min_i32(int x) {
   int y;
@@ -2005,6 +2012,8 @@ int clock_stop(std::vector<KernelTime>& out) {
   return bad;
 }
 
+#include "condense_tile.h"
+
 // --------------------------------------------------------------------------
 // Launchers
 // --------------------------------------------------------------------------
@@ -2291,7 +2300,8 @@ enum Family {
   kFamGrid16 = 7,
   kFamFlux = kFamilyFluxSchur,
   kFamRef = kFamilyFluxRef,
-  kFamCount = 11
+  kFamTile = 11,
+  kFamCount = 12
 };
 
 static bool wave_class(int ni, int nb) {
@@ -2309,26 +2319,35 @@ static bool family_ok(int fam, int ni, int nb) {
     case kFamLarge: return n > 64 && n <= kLargeMaxN;
     case kFamPanel: return n > 64 && n <= kPanelMaxN;
     case kFamGrid16: return n >= 48 && n + 1 <= 96;
+    case kFamTile: return n >= 48 && tile_ok(ni, nb);
   }
   return false;  // kFamFlux depends on the tables: launch_condense_fused
 }
 
 // default choice: the measured-fastest family for the size
-static int default_family(int ni, int nb) {
+static int default_family(int ni, int nb, bool fused) {
   const int n = ni + nb;
   if (wave_class(ni, nb)) return kFamWave;
   if (n + 1 <= 72) return kFamGrid8;
+  if (!fused && tile_ok(ni, nb)) return kFamTile;
   if (n > 128 && n <= 192 && n + 1 <= 176) return kFamGrid32;
   if (n <= 256) return kFamPanel;
   return kFamLarge;
 }
+
+// The entry program's generators have no tile instance: the classes the tile
+// kernel would take go through the flux families.
+template <class G>
+constexpr bool kGenFused = false;
+template <int PHYS>
+constexpr bool kGenFused<FusedGen<PHYS>> = true;
 
 template <class Gen, bool BACKSUB>
 static hipError_t launch_condense(const Gen& gen, const CondenseOut& out, int64_t ncells, int ni,
                                   int nb, hipStream_t st, Workspace& ws, int fam = -1,
                                   int gridmul = 0) {
   if (ncells <= 0) return hipSuccess;
-  if (fam < 0) fam = default_family(ni, nb);
+  if (fam < 0) fam = default_family(ni, nb, kGenFused<Gen>);
   if (!family_ok(fam, ni, nb)) return hipErrorInvalidValue;
   auto grid_of = [&](int per_cu_default) {
     const int64_t per = gridmul > 0 ? gridmul : per_cu_default;
@@ -2400,6 +2419,10 @@ static hipError_t launch_condense(const Gen& gen, const CondenseOut& out, int64_
 #undef HDG_WAVE
     return hipErrorInvalidValue;
   }
+  if (fam == kFamTile) {
+    if constexpr (kGenFused<Gen>) return hipErrorInvalidValue;
+    else return launch_tile<Gen, BACKSUB>(gen, out, ncells, ni, nb, st, gridmul);
+  }
   Bucket b;
   if (fam == kFamGrid32) {
     b = Bucket{32, 16, 6, 11};
@@ -2427,7 +2450,7 @@ static hipError_t launch_condense(const Gen& gen, const CondenseOut& out, int64_
 int condense_variants(const SysShape& sh, int* fams, int max) {
   int k = 0;
   for (int f = 0; f < kFamCount && k < max; ++f)
-    if (family_ok(f, sh.ni, sh.nb) || (f == kFamFlux && sh.flux) ||
+    if ((f != kFamTile && family_ok(f, sh.ni, sh.nb)) || (f == kFamFlux && sh.flux) ||
         (f == kFamRef && sh.ref))
       fams[k++] = f;
   return k;
@@ -2462,13 +2485,14 @@ int condense_default_family(const SysShape& sh) {
   // an 8x8 grid per cell), which no two-stage scheme beats
   if ((sh.flux || sh.ref) && !wave_class(sh.ni, sh.nb) && sh.ni + sh.nb > 96)
     return sh.ref ? kFamRef : kFamFlux;
-  return default_family(sh.ni, sh.nb);
+  return default_family(sh.ni, sh.nb, true);
 }
 
 size_t condense_workspace_bytes(const SysShape& sh, int fam, int64_t ncells) {
   const int ni = sh.ni, nb = sh.nb;
   if (fam < 0) fam = condense_default_family(sh);
-  if (fam == kFamFlux || fam == kFamRef) return flux_workspace_bytes(ni - sh.flux_na + nb, ncells);
+  if (fam == kFamFlux && sh.flux_keep)
+    return flux_workspace_bytes(ni - sh.flux_na + nb, ncells);
   if (fam == kFamPanel) {
     const int n = ni + nb;
     return panel_bytes(n, panel_grid(n, INT64_MAX, 0) * 2, nullptr);  // any grid multiplier <= 2x
@@ -2936,7 +2960,7 @@ void* scratch_address(int device) {
 int noalloc_family(int ni, int nb) {
   const int n = ni + nb;
   if (n > kNoAllocMaxN) return -1;
-  const int fam = default_family(ni, nb);
+  const int fam = default_family(ni, nb, false);
   if (fam != kFamLarge && fam != kFamPanel) return fam;  // no workspace
   if (family_ok(kFamGrid16, ni, nb)) return kFamGrid16;
   if (family_ok(kFamGrid32, ni, nb)) return kFamGrid32;
@@ -3150,7 +3174,7 @@ hipError_t launch_recover_mixed(const Tables& T, const MeshDev& M, const double*
 // --------------------------------------------------------------------------
 constexpr int kFluxWaves = 6;
 constexpr int kFluxMaxNp = 64;
-constexpr int kFusedMaxNb = 128;  // boundary values held in LDS by the flux recovery
+constexpr int kFusedMaxNb = 192;  // boundary values held in LDS by the flux recovery
 constexpr int kRecMaxNa = 192;    // flux rows of the flux recovery (three per lane)
 constexpr int kFluxTileLd = 17;  // leading dimension of a generated row tile
 
@@ -3204,9 +3228,9 @@ __device__ inline int flux_cinv(int ncomp, const int8_t* cid, const double* alph
   return 0;
 }
 
-template <int PHYS, int CT, int KSM, bool SYM>
+template <int CT, int KSM, bool SYM>
 __global__ void __launch_bounds__(64 * kFluxWaves, 3)  // two workgroups per CU
-    flux_schur_kernel(FusedGen<PHYS> gen, int64_t first,
+    flux_schur_kernel(FusedGen<kDarcy> gen, int64_t first,
                       int64_t count, double* __restrict__ R, FluxPlan fp,
                       double* __restrict__ blocks, int64_t bstride) {
   constexpr int NW = kFluxWaves, NT = 64 * NW, LT = kFluxTileLd;
@@ -3462,251 +3486,6 @@ __global__ void __launch_bounds__(64 * kFluxWaves, 3)  // two workgroups per CU
   }
 }
 
-// --------------------------------------------------------------------------
-// Darcy flux elimination from the reference decomposition (family 10).  With
-// C = alpha_0 I and the flux coupling [A_qu A_qb] = sum_e c_ea G_e per flux
-// component a (build_flux_ref), the reduced system of flux_schur is
-//   R[:, :nr] = R0 - s_r (1/alpha_0) sum_p w_p P_p,  w_(e,e') = sum_a c_ea c_e'a
-//   R[:, nr]  = r0 - s_r (1/alpha_0) sum_e G_e^T (sum_a c_ea M^-1 b_q,a)
-// (s_r = -1 on the potential rows, +1 on the trace rows: A_uq = -A_qu^T,
-// A_bq = A_qb^T).  No per-cell product of the flux block remains.  A
-// workgroup owns a band of BR rows of R and runs over the cells of the chunk;
-// each thread owns up to kRefEntries entries (row, column) of the band and
-// keeps, for all cells, their values of every P_p and their entry-program
-// terms (R0 has at most kRefTerms terms per entry) in registers, so a cell
-// costs the cell's coefficients, a few small products and one store per
-// entry.  Of the blocks kept for the recovery only A_uu is written (the
-// recovery applies A_qu and A_uq from the reference matrices as well).
-// --------------------------------------------------------------------------
-constexpr int kRefThreads = 256;
-// entries of R per thread: 3 keeps the kernel at 144 VGPRs, three wavefronts
-// per SIMD (5: 203 VGPRs, two).  Measured at 64^3 k=2: 9.4 ms per step
-// against 11.4 with 5; at 24^3 k=3: 3.5 against 4.0
-constexpr int kRefEntries = 3;
-constexpr int kRefTerms = 3;    // entry-program terms per entry of R0 kept in registers
-constexpr int kRefSplit = 16;   // threads per row of the rhs column's sum
-
-struct RefPlan {
-  int nr, np, na, nu, BR, nbands, npair;
-  size_t lds;  // dynamic LDS bytes
-};
-
-static bool ref_plan_sizes(int D, int np, int na, int ni, int nb, int npair, RefPlan* rp) {
-  if (ni > kRefThreads) return false;  // one right-hand-side value per thread
-  const int nu = ni - na, nr = nu + nb;
-  if (nr + 1 >= (1 << 23)) return false;  // entry columns packed above 8 bits of band row
-  int BR = std::min(nr, kRefEntries * kRefThreads / (nr + 1));
-  BR = std::min(BR, kRefThreads / kRefSplit);  // the rhs column: kRefSplit threads per row
-  if (BR < 1) return false;
-  const int nbands = (nr + BR - 1) / BR;
-  BR = (nr + nbands - 1) / nbands;  // balance the bands
-  // alpha, b_i, then M^-1 (prologue only) aliased with the rhs column, and
-  // the band's columns of every H_e = M^-1 G_e (rows of odd length D np | 1)
-  const size_t lds = (size_t)kMaxAlpha + ni + std::max<size_t>((size_t)np * np, BR) +
-                     (size_t)((D * np) | 1) * BR;
-  if (lds * sizeof(double) > 64 * 1024) return false;
-  if (rp) {
-    rp->nr = nr;
-    rp->np = np;
-    rp->na = na;
-    rp->nu = nu;
-    rp->BR = BR;
-    rp->nbands = nbands;
-    rp->npair = npair;
-    rp->lds = lds * sizeof(double);
-  }
-  return true;
-}
-
-static bool ref_plan(const Tables& T, RefPlan* rp) {
-  if (T.phys != kDarcy || T.fr_npair <= 0 || !T.fr_P || !T.fr_G || !T.fb_minv) return false;
-  return ref_plan_sizes(T.D, T.np, T.na, T.ni, T.nb, T.fr_npair, rp);
-}
-
-template <int D>
-__global__ void __launch_bounds__(kRefThreads, 2)
-    flux_ref_kernel(FusedGen<kDarcy> gen, int64_t first, int64_t count, double* __restrict__ R,
-                    RefPlan rp, double* __restrict__ blocks, int64_t bstride) {
-  constexpr int NT = kRefThreads, NE = kRefEntries, NK = kRefTerms, NPAIR = D * (D + 1) / 2;
-  constexpr int SPL = kRefSplit;
-  const Tables& T = gen.T;
-  const int nr = rp.nr, nc = nr + 1, np = rp.np, na = rp.na, nu = rp.nu, BR = rp.BR;
-  const int ni = T.ni, n = T.n, nk = D * np;
-  const int hld = nk | 1;  // odd row stride of s_H: the rows of a wavefront hit distinct banks
-  const int tid = threadIdx.x;
-  const int band = (int)(blockIdx.x % rp.nbands);
-  const int64_t group = blockIdx.x / rp.nbands, ngroups = gridDim.x / rp.nbands;
-  const int r0 = band * BR, rows = min(BR, nr - r0);
-  extern __shared__ double s_dyn[];
-  double* s_al = s_dyn;                      // [kMaxAlpha]
-  double* s_b = s_al + kMaxAlpha;            // [ni] interior right-hand side
-  double* s_minv = s_b + ni;                 // [np][np], prologue only
-  double* s_xr = s_minv;                     // [BR] rhs column of the Schur term
-  double* s_H = s_minv + max(np * np, BR);   // [BR][hld]: H_e[j][r0 + rl] at rl * hld + e * np + j
-  // ---- per-thread entries: P values and R0's program terms, for all cells ----
-  double pv[NE][NPAIR], tv[NE][NK];
-  int tid8[NE];  // term coefficient ids, 8 bits each; 0xff: no term
-  int ent[NE];   // (column << 8) | band row of the entry, -1: none
-#pragma unroll
-  for (int u = 0; u < NE; ++u) {
-    const int t = tid + NT * u;
-    const bool ok = t < rows * nc;
-    const int c = ok ? t / rows : 0, rl = ok ? t - c * rows : 0;
-    const int r = r0 + rl;
-    ent[u] = ok ? (c << 8) | rl : -1;
-#pragma unroll
-    for (int p = 0; p < NPAIR; ++p)
-      pv[u][p] = (ok && c < nr) ? T.fr_P[((size_t)p * nr + r) * nr + c] : 0.0;
-    int ids = 0xffffff;
-#pragma unroll
-    for (int k = 0; k < NK; ++k) tv[u][k] = 0.0;
-    if (ok && c < nr) {
-      const int e = (na + c) * n + na + r;
-      const uint32_t h = T.prog_head[e];
-      const int cnt = (h >> 8) & 15, x0 = (int)(h >> 12);
-      if (cnt >= 1) {
-        ids = (ids & ~0xff) | (int)(h & 255);
-        tv[u][0] = T.prog_val0[e];
-      }
-#pragma unroll
-      for (int k = 1; k < NK; ++k)
-        if (cnt > k) {
-          ids = (ids & ~(0xff << (8 * k))) | ((int)T.prog_xid[x0 + k - 1] << (8 * k));
-          tv[u][k] = T.prog_xval[x0 + k - 1];
-        }
-    }
-    tid8[u] = ids;
-  }
-  // H_e = M^-1 G_e on the band's columns (M^-1 is symmetric, so the rhs
-  // column's G_e^T M^-1 z_e is H_e^T z_e)
-  // M^-1 staged transposed (M^-1[j][i] at i * np + j): the threads of a
-  // wavefront take consecutive j, which the row-major copy put in one bank
-  // when np = 64
-  for (int t = tid; t < np * np; t += NT) {
-    const int i = t / np, j = t - i * np;
-    s_minv[t] = T.fb_minv[j * np + i];
-  }
-  __syncthreads();
-  for (int t = tid; t < nk * BR; t += NT) {
-    const int rl = t / nk, k = t - rl * nk, e = k / np, j = k - e * np;
-    double h = 0.0;
-    if (rl < rows)
-      for (int i = 0; i < np; ++i)
-        h = fma(s_minv[i * np + j], T.fr_G[((size_t)e * np + i) * nr + r0 + rl], h);
-    s_H[rl * hld + k] = h;
-  }
-  __syncthreads();  // s_minv is reused as s_xr
-  // the cell's coefficients and right-hand side are loaded one cell ahead
-  // (a thread holds at most one of each: kMaxAlpha, ni <= NT)
-  auto fetch = [&](int64_t lc, double& al, double& bv) {
-    const int64_t cell = first + lc;
-    al = (lc < count && tid < kMaxAlpha) ? gen.M.alpha[cell * kMaxAlpha + tid] : 0.0;
-    bv = (lc < count && tid < ni) ? gen.M.srcq[cell * srcq_stride(T) + tid] : 0.0;
-  };
-  // rhs column: thread (rl, part) sums the terms k = part, part + SPL, ... of
-  // sum_k H[k][rl] z[k], z_e[j] = sum_a c_ea b_q,a[j]; the SPL partial sums of
-  // a row sit in consecutive lanes of one wavefront
-  const int xrl = tid / SPL, xpart = tid - xrl * SPL;
-  int xe0 = 0, xj0 = xpart;  // the thread's first term k = xe0 * np + xj0
-  while (xj0 >= np) xj0 -= np, ++xe0;
-  double nal, nbv;
-  fetch(group, nal, nbv);
-  for (int64_t lc = group; lc < count; lc += ngroups) {
-    if (tid < kMaxAlpha) s_al[tid] = nal;
-    if (tid < ni) s_b[tid] = nbv;
-    fetch(lc + ngroups, nal, nbv);
-    __syncthreads();
-    // C = alpha_0 I, c_ea = -alpha[1 + e * D + a]; w_p = sum_a c_ea c_e'a / alpha_0
-    double c[D * D];
-#pragma unroll
-    for (int t = 0; t < D * D; ++t) c[t] = -s_al[1 + t];
-    const double a0 = s_al[0];
-    const bool bad = !(a0 != 0.0);  // a singular C leaves a zero system
-    const double inva = bad ? 0.0 : 1.0 / a0;
-    if (xrl < rows) {
-      // (c_ea read from LDS: a register array indexed by the runtime e would
-      // become a chain of selects; -z is exact, so z = -sum_a alpha b)
-      double x = 0.0;
-      int e = xe0, j = xj0;  // k = e * np + j
-      for (int k = xpart; k < nk; k += SPL) {
-        double zn = 0.0;
-#pragma unroll
-        for (int a = 0; a < D; ++a) zn = fma(s_al[1 + e * D + a], s_b[a * np + j], zn);
-        x = fma(s_H[xrl * hld + k], -zn, x);
-        j += SPL;
-        while (j >= np) j -= np, ++e;
-      }
-#pragma unroll
-      for (int off = SPL / 2; off >= 1; off >>= 1) x += __shfl_xor(x, off, SPL);
-      if (xpart == 0) s_xr[xrl] = x * inva;
-    }  // (a row group's SPL lanes take the same branch)
-    double w[NPAIR];
-    {
-      int p = 0;
-#pragma unroll
-      for (int e = 0; e < D; ++e)
-#pragma unroll
-        for (int e2 = e; e2 < D; ++e2, ++p) {
-          double v = 0.0;
-#pragma unroll
-          for (int a = 0; a < D; ++a) v = fma(c[e * D + a], c[e2 * D + a], v);
-          w[p] = v * inva;
-        }
-    }
-    __syncthreads();
-    double* Rc = R + lc * (int64_t)nc * nr;  // [nc][nr] column-major
-    double* Bk = blocks + lc * bstride;      // [A_uu] (A_qu, A_uq: not used by the recovery)
-#pragma unroll
-    for (int u = 0; u < NE; ++u) {
-      if (ent[u] < 0) continue;
-      const int cc = ent[u] >> 8, rl = ent[u] & 255, r = r0 + rl;
-      double r0v, x;
-      if (cc < nr) {  // the entry program's terms, in its order
-        r0v = 0.0;
-#pragma unroll
-        for (int k = 0; k < NK; ++k) {
-          const int id = (tid8[u] >> (8 * k)) & 0xff;
-          if (id != 0xff) r0v = fma(s_al[id], tv[u][k], r0v);
-        }
-        x = 0.0;
-#pragma unroll
-        for (int p = 0; p < NPAIR; ++p) x = fma(w[p], pv[u][p], x);
-      } else {  // the trace rows carry no source (the cell system's rhs is [b_i; 0])
-        r0v = r < nu ? s_b[na + r] : 0.0;
-        x = s_xr[rl];
-      }
-      // s_r = -1 on the potential rows, +1 on the trace rows
-      Rc[(int64_t)cc * nr + r] = bad ? 0.0 : (r < nu ? r0v + x : r0v - x);
-      if (r < nu && cc < nu) Bk[(int64_t)cc * nu + r] = r0v;  // A_uu
-    }
-    __syncthreads();  // LDS reuse by the next cell
-  }
-}
-
-static hipError_t launch_flux_ref(const Tables& T, const MeshDev& M, int64_t first, int64_t count,
-                                  double* R, const RefPlan& rp, double* blocks, int64_t bstride,
-                                  hipStream_t st) {
-  if (count <= 0) return hipSuccess;
-  // about 2048 workgroups over all bands (eight per CU, three resident); with
-  // np = 64 (k = 3) the per-workgroup set-up (P values, H_e) is four times
-  // dearer and 1024 do better.  Measured at 64^3 k=2: 9.36 ms per step with
-  // 2048, 9.37 with 2304, 11.5 with 1536, 14.3 with 768; at 24^3 k=3: 3.07
-  // with 1024, 3.16 with 2304, 3.30 with 1536, 3.82 with 768
-  const int target = rp.np >= 64 ? 1024 : 2048;
-  const int64_t groups = std::max<int64_t>(
-      1, std::min<int64_t>(count, (target + rp.nbands - 1) / rp.nbands));
-  const int grid = (int)(groups * rp.nbands);
-  FusedGen<kDarcy> gen{T, M};
-  ClockScope clk_(st, "flux_ref");
-  if (T.D == 3)
-    hipLaunchKernelGGL(flux_ref_kernel<3>, dim3(grid), dim3(kRefThreads), rp.lds, st, gen, first,
-                       count, R, rp, blocks, bstride);
-  else
-    hipLaunchKernelGGL(flux_ref_kernel<2>, dim3(grid), dim3(kRefThreads), rp.lds, st, gen, first,
-                       count, R, rp, blocks, bstride);
-  return hipGetLastError();
-}
-
 // The reduced augmented system R of a chunk of cells as an element generator
 // for the regular elimination kernels (rows and columns in reduced order, the
 // last column is the right-hand side).
@@ -3720,139 +3499,6 @@ struct ReducedGen {
   }
 };
 
-// Elimination family for the reduced system: the grid kernels (no workspace;
-// they also keep the multipliers and the pivot order for the recovery).
-static int reduced_family(int ni, int nb) {
-  const int n = ni + nb;
-  if (n + 1 <= 72) return kFamGrid8;
-  if (n + 1 <= 96) return kFamGrid16;
-  if (n <= 192 && n + 1 <= 176) return kFamGrid32;
-  return -1;
-}
-
-// Row-per-lane elimination of the reduced system [R_uu R_ub r_u; R_bu R_bb
-// r_b] (NU interior + NB boundary rows, column-major in the workspace, as
-// ReducedGen reads it) for the sizes of the flux family's 3D classes.  One
-// workgroup of two wavefronts per cell; lane r of wavefront w holds row
-// 64 w + r in registers, the unrolled steps giving every register index as a
-// constant.  Two passes keep the registers to one part of the row:
-//  1. the NU interior columns: all interior rows sit in wavefront 0, so the
-//     pivot search (largest magnitude, smallest LAPACK position on ties) is a
-//     DPP reduction and the LAPACK position bookkeeping lives in a register;
-//     every row's multiplier and the pivot row of each step go to LDS;
-//  2. the NB + 1 trailing columns, in chunks of CW: the same rank-1 updates
-//     replayed with the recorded multipliers, the pivot lane publishing its
-//     chunk in LDS each step.
-// One barrier per step separates the pivot row's publication from the
-// updates.  Every entry sees the same operations in the same order as in the
-// grid kernels.  Outputs as condense_kernel: S, g, U, Y = L^-1 P [R_ub r_u],
-// the multipliers L [step][row], the pivot order P and the singular-cell info.
-template <int NU, int NB>
-__global__ void __launch_bounds__(128)
-    reduced_rowlu_kernel(const double* __restrict__ R, CondenseOut out, int64_t ncells) {
-  constexpr int NR = NU + NB, NC = NR + 1, NT = NB + 1;
-  constexpr int CW = 28;  // trailing columns per pass
-  static_assert(NU <= 64 && NR <= 128, "interior rows in one wavefront, two wavefronts");
-  __shared__ double s_l[NU][NR];  // multiplier of each row at each step
-  __shared__ double s_prow[2][CW > NU ? CW : NU];
-  __shared__ double s_rinv[2];
-  __shared__ int s_piv[NU];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int row = 64 * w + lane;
-  const int64_t us = out.u_stride, ys = out.y_stride;
-  for (int64_t cell = blockIdx.x; cell < ncells; cell += gridDim.x) {
-    const double* Rc = R + cell * (int64_t)NC * NR;
-    int pos = row;  // LAPACK position of this interior row
-    int info = 0;
-    // ---- pass 1: the interior columns, with pivoting -------------------------
-    {
-      double a[NU];
-#pragma unroll
-      for (int c = 0; c < NU; ++c) a[c] = row < NR ? Rc[(int64_t)c * NR + row] : 0.0;
-#pragma unroll
-      for (int j = 0; j < NU; ++j) {
-        const int buf = j & 1;
-        double l = 0.0;
-        if (w == 0) {  // wave-uniform
-          const bool cand = lane < NU && pos >= j;
-          const int64_t key = cand ? dbits(fabs(a[j])) : (int64_t)-1;
-          const int64_t m = wave_max_i64(key);
-          const int ppos = wave_min_i32(key == m && cand ? pos : INT_MAX);
-          const int p = __builtin_ffsll(__ballot(cand && pos == ppos)) - 1;
-          const int q = __builtin_ffsll(__ballot(lane < NU && pos == j)) - 1;
-          const double pv = wave_readlane_f64(a[j], p);
-          const double rinv = pv != 0.0 ? 1.0 / pv : 0.0;
-          if (pv == 0.0 && info == 0) info = j + 1;
-          if (lane == q) pos = ppos;  // LAPACK interchange of positions j and ppos
-          if (lane == p) {
-            pos = j;
-#pragma unroll
-            for (int c = j + 1; c < NU; ++c) s_prow[buf][c] = a[c];
-          }
-          if (lane == 0) {
-            s_rinv[buf] = rinv;
-            s_piv[j] = p;
-          }
-          const bool use = lane < NU ? pos > j : row < NR;
-          l = use ? a[j] * rinv : 0.0;
-          if (lane < NU && use && out.L) out.L[cell * us + (int64_t)j * NU + lane] = l;
-        }
-        __syncthreads();
-        if (w != 0) l = row < NR ? a[j] * s_rinv[buf] : 0.0;
-        if (row < NR) s_l[j][row] = l;
-#pragma unroll
-        for (int c = j + 1; c < NU; ++c) a[c] = fma(-l, s_prow[buf][c], a[c]);
-      }
-      if (w == 0 && lane < NU && out.U) {  // U, packed by columns in LAPACK row order
-#pragma unroll
-        for (int c = 0; c < NU; ++c)
-          if (c >= pos) out.U[cell * us + c * (c + 1) / 2 + pos] = a[c];
-      }
-    }
-    __syncthreads();  // the last step's pivot row is read before pass 2 reuses it
-    // ---- pass 2: the trailing columns, replaying the updates ---------------
-#pragma unroll
-    for (int c0 = 0; c0 < NT; c0 += CW) {
-      double b[CW];
-#pragma unroll
-      for (int c = 0; c < CW; ++c)
-        b[c] = (row < NR && c0 + c < NT) ? Rc[(int64_t)(NU + c0 + c) * NR + row] : 0.0;
-#pragma unroll 1
-      for (int j = 0; j < NU; ++j) {
-        const int buf = j & 1;
-        if (row == s_piv[j]) {
-#pragma unroll
-          for (int c = 0; c < CW; ++c) s_prow[buf][c] = b[c];
-        }
-        __syncthreads();
-        const double l = row < NR ? s_l[j][row] : 0.0;
-#pragma unroll
-        for (int c = 0; c < CW; ++c) b[c] = fma(-l, s_prow[buf][c], b[c]);
-      }
-      if (w == 0 && lane < NU && out.Y) {
-#pragma unroll
-        for (int c = 0; c < CW; ++c)
-          if (c0 + c < NT) out.Y[cell * ys + (int64_t)(c0 + c) * NU + pos] = b[c];
-      }
-      if (row >= NU && row < NR) {
-        const int rb = row - NU;
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-          const int col = c0 + c;
-          if (col < NB) {
-            if (out.S) out.S[(cell * NB + col) * NB + rb] = b[c];
-          } else if (col == NB && out.g) {
-            out.g[cell * NB + rb] = b[c];
-          }
-        }
-      }
-      __syncthreads();  // the pivot-row buffers are reused by the next chunk
-    }
-    if (w == 0 && lane < NU && out.P) out.P[cell * us + pos] = (double)lane;
-    if (threadIdx.x == 0 && out.info) out.info[cell] = info;
-  }
-}
-
 // Register tiling of the flux kernel for a size: column tiles per wavefront
 // and the k-step bound of the unrolled loops.
 static bool flux_fits(int fb_nc, int na, int np, int ni, int nb, int* ct, int* ksm) {
@@ -3863,7 +3509,7 @@ static bool flux_fits(int fb_nc, int na, int np, int ni, int nb, int* ct, int* k
   // which keeps Z's registers within three wavefronts per SIMD)
   const int k = KS <= 8 ? 8 : KS <= 16 ? 16 : KS <= 21 ? 21 : KS <= 24 ? 24 : 0;
   if (k == 0 || c > 2 || c * k > 32) return false;
-  if (reduced_family(ni - na, nb) < 0) return false;
+  if (!tile_ok(ni - na, nb)) return false;
   const int nu = ni - na;
   if (nu > 64 || na > 128 || nb > 128) return false;  // one wavefront per cell in the recovery
   const size_t ncp = 16 * (size_t)((nr + 1 + 15) / 16);
@@ -3907,254 +3553,26 @@ static size_t flux_lds(const FluxPlan& fp, int np) {
 }
 
 // Regions of the flux family's per-cell factor slot (doubles from the slot's
-// start): the reduced factors U (packed by columns), the multipliers L
-// [step][row] and the pivot order P, then the kept interior blocks A_uu
-// [u col][u row], A_qu [u col][flux row], A_uq [flux col][u row], then
-// R_uu^-1 and U^-1, both [col][row].
+// start): the reduced factor U (packed by columns), then the kept interior
+// blocks A_uu [u col][u row] (reference decomposition: of one component),
+// A_qu [u col][flux row], A_uq [flux col][u row] (na = 0: not kept), then
+// R_uu^-1 [col][row].
 struct FluxSlot {
-  int64_t auu, aqu, auq, ri, uinv, size;
+  int64_t auu, aqu, auq, ri, size;
 };
 
 static FluxSlot flux_slot(int na, int nu) {
   FluxSlot o;
-  o.auu = (int64_t)nu * (nu + 1) / 2 + (int64_t)nu * nu + nu;
+  o.auu = (int64_t)nu * (nu + 1) / 2;
   o.aqu = o.auu + (int64_t)nu * nu;
   o.auq = o.aqu + (int64_t)na * nu;
   o.ri = o.auq + (int64_t)na * nu;
-  o.uinv = o.ri + (int64_t)nu * nu;
-  o.size = o.uinv + (int64_t)nu * nu;
+  o.size = o.ri + (int64_t)nu * nu;
   return o;
 }
 
-// R_uu^-1 = U^-1 L^-1 P and U^-1 from the reduced factors, one wavefront per
-// cell with a lane per column of the result held in registers (NUM >= nu).
-// U (column-major) and the multipliers (permuted to positions) are staged in
-// LDS as nu rows zero-padded to NUM, with 1 / diag(U) (0 for a zero pivot), so
-// the unrolled substitutions test bounds once per column (each column's
-// operands load together) and read them as broadcasts.  With NUM = 32 one pass does both inverses: lanes
-// [0, nu) solve for the columns of R_uu^-1, lanes [32, 32 + nu) for those of
-// U^-1, and the columns go out through LDS as one contiguous copy; with
-// NUM = 64 each inverse takes a pass.  The recovery then needs only products
-// with kept matrices.  A zero pivot of U gives a zero row, as in the
-// substitution (the condensation reports such cells as singular).
-constexpr int kInvWaves = 1;
-
-template <int NUM>
-__global__ void __launch_bounds__(64 * kInvWaves)
-    flux_invert_kernel(double* __restrict__ slot, int64_t usz, int64_t ncells, int nu,
-                       int64_t ri_off) {
-  extern __shared__ double s_inv[];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int nup = nu * (nu + 1) / 2, nn = nu * nu;
-  double* sU = s_inv + (int64_t)w * (2 * nu * NUM + 2 * NUM);  // U [col][row], rows padded
-  double* sL = sU + nu * NUM;  // multipliers [step][position], positions padded
-  double* sP = sL + nu * NUM;  // row at each position (-1 past nu)
-  double* sD = sP + NUM;        // 1 / U[c][c]
-  for (int64_t cell = (int64_t)blockIdx.x * kInvWaves + w; cell < ncells;
-       cell += (int64_t)gridDim.x * kInvWaves) {
-    double* Uc = slot + cell * usz;
-    const double* Lc = Uc + nup;
-    // multipliers as stored into sU's region first, then permuted into sL
-    for (int t = lane; t < nn; t += 64) sU[t] = Lc[t];
-    for (int t = lane; t < NUM; t += 64) sP[t] = t < nu ? Lc[nn + t] : -1.0;
-    wave_sync_lds();
-    for (int t = lane; t < nu * NUM; t += 64) {
-      const int i = t / NUM, k = t - i * NUM;
-      sL[t] = k < nu ? sU[i * nu + (int)sP[k]] : 0.0;
-    }
-    wave_sync_lds();
-    for (int t = lane; t < nu * NUM; t += 64) {
-      const int c = t / NUM, k = t - c * NUM;
-      sU[t] = k <= c ? Uc[c * (c + 1) / 2 + k] : 0.0;
-    }
-    for (int t = lane; t < NUM; t += 64) {
-      const double d = t < nu ? Uc[t * (t + 1) / 2 + t] : 0.0;
-      sD[t] = d != 0.0 ? 1.0 / d : 0.0;
-    }
-    wave_sync_lds();
-    // y <- U^-1 y
-    auto back_subst = [&](double (&y)[NUM]) {
-#pragma unroll
-      for (int c = NUM - 1; c >= 0; --c) {
-        if (c < nu) {  // one block per column: its operands load together
-          const double* col = sU + c * NUM;
-          y[c] *= sD[c];
-#pragma unroll
-          for (int k = 0; k < c; ++k) y[k] = fma(-col[k], y[c], y[k]);
-        }
-      }
-    };
-    // y <- L^-1 y (positions)
-    auto forward = [&](double (&y)[NUM]) {
-#pragma unroll
-      for (int i = 0; i < NUM - 1; ++i) {
-        if (i + 1 < nu) {
-          const double* li = sL + i * NUM;
-#pragma unroll
-          for (int k = i + 1; k < NUM; ++k) y[k] = fma(-li[k], y[i], y[k]);
-        }
-      }
-    };
-    double* out = Uc + ri_off;  // R_uu^-1 then U^-1, [col][row]
-    if (NUM == 32) {
-      const bool rinv = lane < 32;
-      const int j = lane & 31;
-      double y[NUM];
-#pragma unroll
-      for (int k = 0; k < NUM; ++k)
-        y[k] = rinv ? ((int)sP[k] == j ? 1.0 : 0.0) : (k == j ? 1.0 : 0.0);
-      if (rinv) forward(y);
-      back_subst(y);
-      wave_sync_lds();  // the staged factors are dead: their LDS takes the columns
-      if (j < nu) {
-        double* col = sU + (rinv ? 0 : nn) + j * nu;
-#pragma unroll
-        for (int k = 0; k < NUM; ++k)
-          if (k < nu) col[k] = y[k];
-      }
-      wave_sync_lds();
-      for (int t = lane; t < 2 * nn; t += 64) out[t] = sU[t];
-    } else {
-#pragma unroll 1
-      for (int pass = 0; pass < 2; ++pass) {
-        const int j = lane;
-        double y[NUM];
-#pragma unroll
-        for (int k = 0; k < NUM; ++k)
-          y[k] = pass == 0 ? ((int)sP[k] == j ? 1.0 : 0.0) : (k == j ? 1.0 : 0.0);
-        if (pass == 0) forward(y);
-        back_subst(y);
-        if (j < nu) {
-          double* col = out + (int64_t)pass * nn + (int64_t)j * nu;
-#pragma unroll
-          for (int k = 0; k < NUM; ++k)
-            if (k < nu) col[k] = y[k];
-        }
-      }
-    }
-    wave_sync_lds();
-  }
-}
-
-// flux_invert_kernel for 32 < nu <= 64 with the two inverses computed side by
-// side: a workgroup of two wavefronts per cell shares the staged factors,
-// wavefront 0 forming R_uu^-1 and wavefront 1 U^-1.  The factors are staged
-// packed (U by columns as the slot keeps it, the multipliers by steps over
-// the positions after the step), 34 KB per cell, so four cells fit a CU.
-// Each lane does exactly what the single-wavefront kernel does for its column
-// and pass, with the same operands, so the results are the same bit for bit.
-constexpr int kInv2Lds = 64 * 65 / 2 + 64 * 63 / 2 + 2 * 64;  // doubles per cell
-
-__global__ void __launch_bounds__(128)
-    flux_invert2_kernel(double* __restrict__ slot, int64_t usz, int64_t ncells, int nu,
-                        int64_t ri_off) {
-  constexpr int NUM = 64;
-  extern __shared__ double s_inv[];
-  const int lane = threadIdx.x & 63, pass = threadIdx.x >> 6;
-  const int nup = nu * (nu + 1) / 2, nn = nu * nu;
-  double* sU = s_inv;                   // U packed by columns: (k, c), k <= c, at c(c+1)/2 + k
-  double* sL = sU + NUM * (NUM + 1) / 2;  // multipliers: (i, k), k > i, at i(2 NUM - i - 1)/2 + k - i - 1
-  double* sP = sL + NUM * (NUM - 1) / 2;  // row at each position (-1 past nu)
-  double* sD = sP + NUM;                  // 1 / U[c][c]
-  for (int64_t cell = blockIdx.x; cell < ncells; cell += gridDim.x) {
-    double* Uc = slot + cell * usz;
-    const double* Lc = Uc + nup;
-    for (int t = threadIdx.x; t < NUM; t += 128) sP[t] = t < nu ? Lc[nn + t] : -1.0;
-    for (int t = threadIdx.x; t < nup; t += 128) sU[t] = Uc[t];
-    for (int t = threadIdx.x; t < NUM; t += 128) {
-      const double d = t < nu ? Uc[t * (t + 1) / 2 + t] : 0.0;
-      sD[t] = d != 0.0 ? 1.0 / d : 0.0;
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < NUM * (NUM - 1) / 2; t += 128) {
-      // t -> (i, k): row i of the packed strictly-upper layout
-      int i = 0, rem = t;
-      while (rem >= NUM - 1 - i) rem -= NUM - 1 - i, ++i;
-      const int k = i + 1 + rem;
-      sL[t] = (i < nu && k < nu) ? Lc[i * nu + (int)sP[k]] : 0.0;
-    }
-    __syncthreads();
-    double* out = Uc + ri_off;  // R_uu^-1 then U^-1, [col][row]
-    const int j = lane;
-    double y[NUM];
-#pragma unroll
-    for (int k = 0; k < NUM; ++k)
-      y[k] = pass == 0 ? ((int)sP[k] == j ? 1.0 : 0.0) : (k == j ? 1.0 : 0.0);
-    if (pass == 0) {  // y <- L^-1 y (positions)
-#pragma unroll
-      for (int i = 0; i < NUM - 1; ++i) {
-        if (i + 1 < nu) {
-          const double* li = sL + i * (2 * NUM - i - 1) / 2 - (i + 1);
-#pragma unroll
-          for (int k = i + 1; k < NUM; ++k) y[k] = fma(-li[k], y[i], y[k]);
-        }
-      }
-    }
-    // y <- U^-1 y
-#pragma unroll
-    for (int c = NUM - 1; c >= 0; --c) {
-      if (c < nu) {
-        const double* col = sU + c * (c + 1) / 2;
-        y[c] *= sD[c];
-#pragma unroll
-        for (int k = 0; k < c; ++k) y[k] = fma(-col[k], y[c], y[k]);
-      }
-    }
-    if (j < nu) {
-      double* col = out + (int64_t)pass * nn + (int64_t)j * nu;
-#pragma unroll
-      for (int k = 0; k < NUM; ++k)
-        if (k < nu) col[k] = y[k];
-    }
-    __syncthreads();  // the staged factors are reused by the next cell
-  }
-}
-
-static hipError_t launch_flux_invert(double* slot, int64_t usz, int64_t ncells, int na, int nu,
-                                     hipStream_t st) {
-  if (ncells <= 0) return hipSuccess;
-  const FluxSlot fs = flux_slot(na, nu);
-  const int num = nu <= 32 ? 32 : 64;
-  const size_t lds = kInvWaves * (size_t)(2 * nu * num + 2 * num) * sizeof(double);
-  const int64_t blocks = (ncells + kInvWaves - 1) / kInvWaves;
-  const int grid = (int)(blocks < 65536 ? blocks : 65536);
-  ClockScope clk_(st, "flux_invert");
-  if (nu <= 32)
-    hipLaunchKernelGGL((flux_invert_kernel<32>), dim3(grid), dim3(64 * kInvWaves), lds, st,
-                       slot, usz, ncells, nu, fs.ri);
-  else if (nu <= 64)
-    hipLaunchKernelGGL(flux_invert2_kernel, dim3((int)std::min<int64_t>(ncells, 65536)),
-                       dim3(128), (size_t)kInv2Lds * sizeof(double), st, slot, usz, ncells, nu,
-                       fs.ri);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-// Elimination of a chunk of reduced systems: the row-per-lane kernel for the
-// 3D flux classes, else the grid family of the size.
-static hipError_t launch_reduced(const double* R, int nr, const CondenseOut& o, int64_t count,
-                                 int nu, int nb, hipStream_t st, int rfam, int gridmul) {
-  // 32 row-per-lane workgroups per CU (about four times the resident eight):
-  // measured at 64^3 k=2, 12.3 ms per step against 13.2 with 16, 14.3 with 8
-  // and 12.4 with one cell per workgroup
-  const int grid = (int)std::min<int64_t>(count, 256 * (gridmul > 0 ? gridmul : 32));
-#define HDG_ROWLU(NU_, NB_)                                                                  \
-  if (nu == NU_ && nb == NB_) {                                                              \
-    ClockScope clk_(st, "reduced_rowlu");                                                    \
-    hipLaunchKernelGGL((reduced_rowlu_kernel<NU_, NB_>), dim3(grid), dim3(128), 0, st, R, o, \
-                       count);                                                               \
-    return hipGetLastError();                                                                \
-  }
-  HDG_ROWLU(27, 54)
-  HDG_ROWLU(18, 54)
-#undef HDG_ROWLU
-  ReducedGen rg{R, nr};
-  Workspace none;
-  return launch_condense<ReducedGen, false>(rg, o, count, nu, nb, st, none, rfam, gridmul);
-}
-
-// Cells per flux chunk: the reduced systems of one chunk live in the workspace.
+// Cells per chunk of family 8's MFMA products: the reduced systems of one chunk
+// live in the workspace.
 static int64_t flux_chunk(int nr) {
   const int64_t per = (int64_t)nr * (nr + 1) * (int64_t)sizeof(double);
   const int64_t c = ((int64_t)512 << 20) / per;
@@ -4166,53 +3584,36 @@ static size_t flux_workspace_bytes(int nr, int64_t ncells) {
   return (size_t)chunk * nr * (nr + 1) * sizeof(double);
 }
 
-
-template <int PHYS>
-static hipError_t launch_flux_phys(const Tables& T, const MeshDev& M, const CondenseOut& out,
-                                   hipStream_t st, Workspace& ws, int gridmul, bool ref) {
+// Darcy, family 8: R from two MFMA products per cell, chunk by chunk.
+static hipError_t launch_flux_schur(const Tables& T, const MeshDev& M, const CondenseOut& out,
+                                    const FluxSlot& fs, hipStream_t st, Workspace& ws,
+                                    int gridmul) {
   FluxPlan fp;
   int ct = 0, ksm = 0;
-  RefPlan rp;
-  if (ref) {
-    if (!sys_shape(T).ref || !ref_plan(T, &rp)) return hipErrorInvalidValue;
-  } else if (!flux_plan(T, fp, &ct, &ksm)) {
-    return hipErrorInvalidValue;
-  }
+  if (!flux_plan(T, fp, &ct, &ksm)) return hipErrorInvalidValue;
   const int nu = T.ni - T.na, nb = T.nb, nr = nu + nb;
-  const int rfam = reduced_family(nu, nb);
-  if (rfam < 0) return hipErrorInvalidValue;
-  const int64_t ncells = M.ncells;
-  if (ncells <= 0) return hipSuccess;
-  if (!out.U) return hipErrorInvalidValue;
+  const int64_t ncells = M.ncells, usz = out.u_stride, ysz = out.y_stride;
   const int64_t chunk = std::min<int64_t>(ncells, flux_chunk(nr));
   hipError_t e = workspace_reserve(ws, flux_workspace_bytes(nr, ncells));
   if (e != hipSuccess) return e;
-  const size_t lds = ref ? 0 : flux_lds(fp, T.np);
+  const size_t lds = flux_lds(fp, T.np);
   if (lds > 160 * 1024 - sizeof(FusedShared) - 1024) return hipErrorInvalidValue;
-  FusedGen<PHYS> gen{T, M};
-  // reduced factors and kept blocks in the per-cell slots of the class
-  const int64_t usz = out.u_stride, ysz = out.y_stride;
-  if (usz < (int64_t)factor_slot(sys_shape(T)) || ysz < (int64_t)(nb + 1) * nu)
-    return hipErrorInvalidValue;
-  const int64_t boff = (int64_t)nu * (nu + 1) / 2 + (int64_t)nu * nu + nu;  // after U, L, P
+  FusedGen<kDarcy> gen{T, M};
   for (int64_t first = 0; first < ncells; first += chunk) {
     const int64_t count = std::min<int64_t>(chunk, ncells - first);
     const int grid = (int)std::min<int64_t>(count, 256 * 4);
-    if (ref) {
-      e = launch_flux_ref(T, M, first, count, ws.p, rp, out.U + first * usz + boff, usz, st);
-      if (e != hipSuccess) return e;
-    } else {
+    {
       ClockScope clk_(st, "flux_schur");
-#define HDG_FLUX(CT_, KS_)                                                                   \
-  if (ct == CT_ && ksm == KS_) {                                                             \
-    if (PHYS == kDarcy && fp.sym)                                                            \
-      hipLaunchKernelGGL((flux_schur_kernel<PHYS, CT_, KS_, PHYS == kDarcy>), dim3(grid),    \
-                         dim3(64 * kFluxWaves), lds, st, gen, first, count, ws.p, fp,         \
-                         out.U + first * usz + boff, usz);                                    \
-    else                                                                                     \
-      hipLaunchKernelGGL((flux_schur_kernel<PHYS, CT_, KS_, false>), dim3(grid),             \
-                         dim3(64 * kFluxWaves), lds, st, gen, first, count, ws.p, fp,         \
-                         out.U + first * usz + boff, usz);                                    \
+#define HDG_FLUX(CT_, KS_)                                                                     \
+  if (ct == CT_ && ksm == KS_) {                                                               \
+    if (fp.sym)                                                                                \
+      hipLaunchKernelGGL((flux_schur_kernel<CT_, KS_, true>), dim3(grid), dim3(64 * kFluxWaves), \
+                         lds, st, gen, first, count, ws.p, fp, out.U + first * usz + fs.auu,    \
+                         usz);                                                                 \
+    else                                                                                       \
+      hipLaunchKernelGGL((flux_schur_kernel<CT_, KS_, false>), dim3(grid),                      \
+                         dim3(64 * kFluxWaves), lds, st, gen, first, count, ws.p, fp,           \
+                         out.U + first * usz + fs.auu, usz);                                    \
   }
       HDG_FLUX(1, 8)
       HDG_FLUX(1, 16)
@@ -4227,142 +3628,162 @@ static hipError_t launch_flux_phys(const Tables& T, const MeshDev& M, const Cond
     CondenseOut o;
     o.S = out.S ? out.S + first * nb * nb : nullptr;
     o.g = out.g ? out.g + first * nb : nullptr;
-    o.U = out.U ? out.U + first * usz : nullptr;
+    o.U = out.U + first * usz;
     o.Y = out.Y ? out.Y + first * ysz : nullptr;
     o.u_stride = usz;
     o.y_stride = ysz;
-    o.L = o.U ? o.U + (int64_t)nu * (nu + 1) / 2 : nullptr;
-    o.P = o.L ? o.L + (int64_t)nu * nu : nullptr;
+    o.Rinv = o.U + fs.ri;
     o.info = out.info ? out.info + first : nullptr;
-    e = launch_reduced(ws.p, nr, o, count, nu, nb, st, rfam, gridmul);
+    e = launch_tile<ReducedGen, false>(ReducedGen{ws.p, nr}, o, count, nu, nb, st, gridmul);
     if (e != hipSuccess) return e;
   }
-  return launch_flux_invert(out.U, usz, ncells, T.na, nu, st);
+  return hipSuccess;
 }
 
 hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                 hipStream_t st, Workspace& ws, int gridmul, bool ref) {
-  if (ref && (T.phys != kDarcy || T.fr_npair == 0)) return hipErrorInvalidValue;
-  return T.phys == kDarcy ? launch_flux_phys<kDarcy>(T, M, out, st, ws, gridmul, ref)
-                          : launch_flux_phys<kElasticity>(T, M, out, st, ws, gridmul, false);
+  const SysShape sh = sys_shape(T);
+  if (ref ? !sh.ref : !sh.flux) return hipErrorInvalidValue;
+  const int nu = T.ni - T.na;
+  if (M.ncells <= 0) return hipSuccess;
+  // reduced factors and kept blocks in the per-cell slots of the class
+  if (!out.U || out.u_stride < (int64_t)factor_slot(sh) ||
+      out.y_stride < (int64_t)(T.nb + 1) * nu)
+    return hipErrorInvalidValue;
+  const FluxSlot fs = flux_slot(sh.flux_keep, nu);
+  if (T.phys == kDarcy && !ref) return launch_flux_schur(T, M, out, fs, st, ws, gridmul);
+  CondenseOut o = out;
+  o.Auu = out.U + fs.auu;
+  o.Rinv = out.U + fs.ri;
+  if (T.phys == kDarcy)
+    return T.D == 2 ? launch_tile_ref<kDarcy, 2>(T, M, o, st, gridmul)
+                    : launch_tile_ref<kDarcy, 3>(T, M, o, st, gridmul);
+  return T.D == 2 ? launch_tile_ref<kElasticity, 2>(T, M, o, st, gridmul)
+                  : launch_tile_ref<kElasticity, 3>(T, M, o, st, gridmul);
 }
 
 size_t factor_slot(const SysShape& sh) {
   const size_t dense = (size_t)sh.ni * (sh.ni + 1) / 2;
   if (sh.flux_na <= 0) return dense;
-  const size_t m = (size_t)(sh.ni - sh.flux_na), na = (size_t)sh.flux_na;
-  size_t s = std::max(dense, (size_t)flux_slot((int)na, (int)m).size);
-  return s;
+  return std::max(dense, (size_t)flux_slot(sh.flux_keep, sh.ni - sh.flux_na).size);
 }
 
-// Family 10 has kernels for the sizes: the band kernel's plan, the reduced
-// elimination (row-per-lane or grid), the inverses (nu <= 64) and the
-// recovery (one wavefront per cell, at most kRecMaxNa flux rows).
-static bool ref_fits(int phys, int D, int fb_nc, int na, int np, int ni, int nb, int npair) {
-  if (phys != kDarcy || npair <= 0 || fb_nc != D || np > kFluxMaxNp || na <= 0 || na >= ni)
-    return false;
-  const int nu = ni - na;
-  if (nu > 64 || na > kRecMaxNa || nb > kFusedMaxNb) return false;
-  if (reduced_family(nu, nb) < 0) return false;
-  return ref_plan_sizes(D, np, na, ni, nb, npair, nullptr);
+// The reference decomposition has kernels for the sizes: the tile elimination
+// and the recovery (one wavefront per cell, at most kRecMaxNa flux rows).
+static bool ref_fits(int npair, int na, int np, int ni, int nb) {
+  if (npair <= 0 || na <= 0 || na >= ni || na > kRecMaxNa || nb > kFusedMaxNb) return false;
+  return ref_tile_ok(ni - na, nb, np);
 }
 
-SysShape sys_shape(const Tables& T) {
-  SysShape sh;
-  sh.ni = T.ni;
-  sh.nb = T.nb;
-  sh.flux = T.fb_minv && flux_fits(T.fb_nc, T.na, T.np, T.ni, T.nb, nullptr, nullptr);
-  sh.ref = T.fb_minv && T.fr_P && T.fr_G &&
-           ref_fits(T.phys, T.D, T.fb_nc, T.na, T.np, T.ni, T.nb, T.fr_npair);
-  sh.flux_na = sh.flux || sh.ref ? T.na : 0;
-  return sh;
-}
-
-SysShape sys_shape(const TablesHost& t) {
+template <class TT>
+static SysShape shape_of(const TT& t, bool minv) {
   SysShape sh;
   sh.ni = t.ni;
   sh.nb = t.nb;
-  sh.flux = !t.fb_minv.empty() && flux_fits(t.fb_nc, t.na, t.np, t.ni, t.nb, nullptr, nullptr);
-  sh.ref = !t.fb_minv.empty() && !t.fr_P.empty() &&
-           ref_fits(t.phys, t.D, t.fb_nc, t.na, t.np, t.ni, t.nb, t.fr_npair);
+  const bool ref = minv && ref_fits(t.fr_npair, t.na, t.np, t.ni, t.nb);
+  if (t.phys == kDarcy) {
+    sh.ref = ref;
+    sh.flux = minv && flux_fits(t.fb_nc, t.na, t.np, t.ni, t.nb, nullptr, nullptr);
+    sh.flux_keep = sh.flux ? t.na : 0;
+  } else {
+    sh.flux = ref;  // elasticity's family 8 is the reference decomposition
+  }
   sh.flux_na = sh.flux || sh.ref ? t.na : 0;
   return sh;
 }
 
+SysShape sys_shape(const Tables& T) { return shape_of(T, T.fb_minv != nullptr); }
+
+SysShape sys_shape(const TablesHost& t) { return shape_of(t, !t.fb_minv.empty()); }
+
 // Flux recovery, one wavefront per cell, for both flux families.  The cell's
-// slot holds R_uu^-1, the interior blocks A_uu, A_qu, A_uq and U^-1, the
-// inverse of the reduced system's upper factor; Y = L^-1 P [R_ub r_u] are the
-// reduced system's lower-factor rows (RecSlot gives where):
-//   c   = b_i - A_ib lambda                 (boundary columns of the program)
-//   x_u = U^-1 (y - Y lambda)
-//   x_q = A_qq^-1 (c_q - A_qu x_u)          (A_qq^-1 = C^-1 (x) M^-1)
-// then up to kFluxRefineSteps FP64 refinement steps against the residual of
-// the full interior system, r = c - A_ii x, with the structured solve as the
-// approximate inverse:
-//   z = A_qq^-1 r_q,  d_u = R_uu^-1 (r_u - A_uq z),  d_q = z - A_qq^-1 A_qu d_u.
-// The reduced system R_uu is worse conditioned than A_ii when the flux block
-// is small (large kappa): the first x_u can be off by cond(R_uu) eps in the
-// near-null mode of A_uq A_qq^-1 A_qu, and the refinement brings it to the
-// accuracy of a direct FP64 solve of A_ii.  Each step reads every kept block
-// once: A_qu x_u is carried from step to step (A_qu x_u + A_qu d_u), and
-// r_u - A_uq z is formed as c_u - A_uu x_u - A_uq (x_q + z), whose rounding is
-// that of the residual itself.  It stops once a correction is below 2^-48 of
-// the solution.
+// slot holds R_uu^-1 of the reduced system and the interior blocks A_uu, A_qu,
+// A_uq (RecSlot gives where).  With c = b_i - A_ib lambda (boundary columns of
+// the program), the structured solve of a right-hand side r is
+//   z = A_qq^-1 r_q (A_qq^-1 = C^-1 (x) M^-1),  d_u = R_uu^-1 (r_u - A_uq z),
+//   d_q = z - A_qq^-1 A_qu d_u,
+// applied to c and then, up to kFluxRefineSteps times, to the residual of the
+// full interior system, r = c - A_ii x.  The reduced system R_uu is worse
+// conditioned than A_ii when the flux block is small (large kappa): the first
+// x_u can be off by cond(R_uu) eps in the near-null mode of A_uq A_qq^-1 A_qu,
+// and the refinement brings it to the accuracy of a direct FP64 solve of A_ii.
+// Each step reads every kept block once: A_qu x_u is carried from step to step
+// (A_qu x_u + A_qu d_u), and r_u - A_uq z is formed as c_u - A_uu x_u -
+// A_uq (x_q + z), whose rounding is that of the residual itself.  It stops
+// once a correction is below 2^-48 of the solution.
 constexpr int kRecWaves = 4;      // cells (wavefronts) per workgroup of the flux recovery
 
-// doubles of LDS per wavefront of the flux recovery (the last na: the
-// reference variant's work vector)
-__host__ __device__ inline int rec_wave_lds(int na, int nu, int nb) {
-  return kMaxAlpha + 72 + nb + 5 * na + (na > 72 ? na : 72) + 2 * nu;
+// doubles of LDS per wavefront of the flux recovery (the last ng: the
+// reference variant's G_e products, ncq D np)
+__host__ __device__ inline int rec_wave_lds(int na, int nu, int nb, int ng) {
+  return kMaxAlpha + 72 + nb + 5 * na + 2 * nu + ng;
 }
 
 struct RecSlot {
   const double* slot;  // per-cell slots, stride usz
   int64_t usz;
   int64_t ri, auu, aqu, auq;  // R_uu^-1 [col][row], A_uu, A_qu, A_uq (offsets in the slot)
-  int64_t uinv;               // U^-1 [col][row]
-  const double* w;     // Y: w + cell * wsz + column * wld + u row
-  int64_t wsz;
-  int wld;
 };
 
-// REF (family 10): A_qu and A_uq are not read from the slot but applied from
-// the reference matrices G_e (potential columns) and the cell's cofactors
-// c_ea: A_qu[(a,i)][c] = sum_e c_ea G_e[i][c] and A_uq = -A_qu^T (the Darcy
-// coupling of build_flux_ref).  G_e is staged in LDS once per workgroup
-// (g_lds), or, where it does not fit (3D k=3), read from the table, which
-// every cell shares (L2-resident).
-template <int PHYS, int KQ, bool REF>
+// C^-1 (6 x 6, row-major) of a cell's flux block C (x) M, one entry per lane:
+// Darcy C = alpha_0 I; elasticity the compliance, k0 on the normal components,
+// k1 between them, ks on the shear ones (0 where C is singular).
+template <int PHYS>
+__device__ inline double flux_cinv_entry(const double* alpha, int D, int a, int b) {
+  if (PHYS == kDarcy) return a == b && a < D && alpha[0] != 0.0 ? 1.0 / alpha[0] : 0.0;
+  const int nc = D * (D + 1) / 2;
+  if (a >= nc || b >= nc) return 0.0;
+  int ia, ja, ib, jb;
+  sym_pair(D, a, ia, ja);
+  sym_pair(D, b, ib, jb);
+  const double k0 = alpha[0], k1 = alpha[D == 3 ? 3 : 2], ks = alpha[7];
+  const double dm = k0 - k1, dn = k0 + (D - 1) * k1;
+  if (dm == 0.0 || dn == 0.0 || ks == 0.0) return 0.0;
+  if (ia == ja && ib == jb) return (a == b ? k0 + (D - 2) * k1 : -k1) / (dm * dn);
+  return a == b ? 1.0 / ks : 0.0;
+}
+
+// REF (the reference decomposition): A_qu and A_uq are not read from the slot
+// but applied from the reference matrices G_e (potential columns) and the
+// cell's cofactors c_ea,
+//   Darcy:      (A_qu v)[(a, i)] = sum_e c_ea t_e[i],  t_e = G_e v;
+//   elasticity: (A_qu v)[(s, i)] = sum over the components d of s = (p, q) of
+//               sum_e c_e,partner t_de[i],  t_de = G_e v_d;
+// and A_uq = -A_qu^T; A_uu is kept for one potential component.  G_e is staged
+// in LDS once per workgroup (g_lds), or, where it does not fit (3D Darcy k=3),
+// read from the table, which every cell shares (L2-resident).
+template <int PHYS, int KQ, int KU, bool REF>
 __global__ void __launch_bounds__(256)
     recover_flux_kernel(FusedGen<PHYS> gen, RecSlot rs, const int32_t* __restrict__ cell_dofs,
                         const double* __restrict__ lam_free, const double* __restrict__ lam_dir,
                         double* __restrict__ out, bool g_lds) {
   constexpr int WPB = kRecWaves;
   // M^-1 and M transposed ([col][row]: lane i reads row i at stride 1, free of
-  // bank conflicts for any np), (REF with g_lds: G_e [D][np][nu]), then the
+  // bank conflicts for any np), (REF with g_lds: G_e [D][np][nq]), then the
   // wavefronts' vectors
   extern __shared__ double s_m[];
   const Tables& T = gen.T;
-  const int ni = T.ni, nb = T.nb, na = T.na, np = T.np, nu = ni - na, nqc = T.nqc;
+  const int ni = T.ni, nb = T.nb, na = T.na, np = T.np, nu = ni - na, nq = T.nq;
   const int ncomp = T.fb_nc, D = T.D;
+  const int nd = PHYS == kDarcy ? 1 : D, ng = nd * D * np;
   const int64_t ncells = gen.M.ncells;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int gsz = REF && g_lds ? D * np * nu : 0;
-  double* s_gu = s_m + 2 * np * np;  // REF with g_lds: G_e[i][c] at (e * np + i) * nu + c
+  const int gsz = REF && g_lds ? D * np * nq : 0;
+  double* s_gu = s_m + 2 * np * np;  // REF with g_lds: G_e[i][c] at (e * np + i) * nq + c
   // G_e[i][c] at gsrc[(e * np + i) * gld + c]
   const double* gsrc = g_lds ? s_gu : T.fr_G;
-  const int gld = g_lds ? nu : nu + nb;
-  double* alpha = s_m + 2 * np * np + gsz + (int64_t)w * rec_wave_lds(na, nu, nb);  // [kMaxAlpha]
+  const int gld = g_lds ? nq : nq + T.nF * T.nm;
+  double* alpha = s_m + 2 * np * np + gsz + (int64_t)w * rec_wave_lds(na, nu, nb, REF ? ng : 0);
   double* c6 = alpha + kMaxAlpha;  // C, then C^-1 [2][36]
   double* lam = c6 + 72;           // [nb]
   double* xq = lam + nb;           // x_q [na]
   double* cq = xq + na;            // c_q [na]
   double* aq = cq + na;            // A_qu x_u [na]
   double* qv = aq + na;            // flux work vector [na]
-  double* zv = qv + na;            // [max(na, 72)]; flux_cinv's scratch at a cell's start
-  double* xuv = zv + (na > 72 ? na : 72);  // x_u [nu]
+  double* zv = qv + na;            // [na]
+  double* xuv = zv + na;           // x_u [nu]
   double* uv = xuv + nu;           // reduced work vector [nu]
-  double* tv = uv + nu;            // REF: G_e products [D][np]
+  double* tv = uv + nu;            // REF: G_e products [nd][D][np]
   for (int t = threadIdx.x; t < np * np; t += 64 * WPB) {
     const int i = t / np, j = t - i * np;
     s_m[j * np + i] = T.fb_minv[t];
@@ -4370,12 +3791,20 @@ __global__ void __launch_bounds__(256)
   }
   if (REF && g_lds)
     for (int t = threadIdx.x; t < gsz; t += 64 * WPB) {
-      const int e = t / (np * nu), rem = t - e * np * nu, i = rem / nu, c = rem - i * nu;
-      s_gu[t] = T.fr_G[((size_t)e * np + i) * (nu + nb) + c];
+      const int k = t / nq, c = t - k * nq;
+      s_gu[t] = T.fr_G[(size_t)k * (nq + T.nF * T.nm) + c];
     }
   __syncthreads();
   const double* Minv = s_m;
   const double* Mm = s_m + np * np;
+  auto cof = [&](int e, int a) {
+    return PHYS == kDarcy ? -alpha[1 + e * D + a] : alpha[36 + e * D + a];
+  };
+  // stress component of the pair (d, a)
+  auto stress = [&](int d, int a) {
+    const int i = min(d, a), j = max(d, a);
+    return i * D - i * (i - 1) / 2 + j - i;
+  };
 
   // v <- (Cm (x) Mt) v over the flux rows (v in LDS): Mt = M^-1 with Cm = C^-1
   // for a solve, Mt = M with Cm = C for a product (Mt stored transposed)
@@ -4397,9 +3826,11 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int t = 0; t < KQ; ++t) {
       const int r = lane + 64 * t;
-      if (r < na) v[r] = y[t];
+      // (Darcy: C = alpha_0 I, no mixing of the components)
+      if (r < na) v[r] = PHYS == kDarcy ? y[t] * Cm[0] : y[t];
     }
     wave_sync_lds();
+    if (PHYS == kDarcy) return;
 #pragma unroll
     for (int t = 0; t < KQ; ++t) {
       const int r = lane + 64 * t;
@@ -4421,12 +3852,13 @@ __global__ void __launch_bounds__(256)
   // qv = A_qu v (v over the u unknowns, in LDS)
   auto aqu_apply = [&](const double* Aqu, const double* v) {
     if (REF) {
-      // t_e[i] = sum_c G_e[i][c] v[c]; qv[(a, i)] = sum_e c_ea t_e[i]
-      for (int t = lane; t < D * np; t += 64) {
-        const double* g = gsrc + (int64_t)t * gld;
+      for (int t = lane; t < ng; t += 64) {
+        const int d = PHYS == kDarcy ? 0 : t / (D * np);
+        const double* g = gsrc + (int64_t)(t - d * D * np) * gld;
+        const double* vd = v + d * nq;
         double acc = 0.0;
 #pragma unroll 4
-        for (int c = 0; c < nu; ++c) acc = fma(g[c], v[c], acc);
+        for (int c = 0; c < nq; ++c) acc = fma(g[c], vd[c], acc);
         tv[t] = acc;
       }
       wave_sync_lds();
@@ -4436,7 +3868,16 @@ __global__ void __launch_bounds__(256)
         if (r < na) {
           const int a = r / np, i = r - a * np;
           double acc = 0.0;
-          for (int e = 0; e < D; ++e) acc = fma(-alpha[1 + e * D + a], tv[e * np + i], acc);
+          if (PHYS == kDarcy) {
+            for (int e = 0; e < D; ++e) acc = fma(cof(e, a), tv[e * np + i], acc);
+          } else {
+            int p, q;
+            sym_pair(D, a, p, q);
+            for (int e = 0; e < D; ++e) {
+              acc = fma(cof(e, p), tv[(q * D + e) * np + i], acc);
+              if (p != q) acc = fma(cof(e, q), tv[(p * D + e) * np + i], acc);
+            }
+          }
           qv[r] = acc;
         }
       }
@@ -4466,90 +3907,71 @@ __global__ void __launch_bounds__(256)
       const int a = lane / 6, b = lane - 6 * (lane / 6);
       const int id = T.fb_cid[lane];
       c6[lane] = (a < ncomp && b < ncomp && id >= 0) ? alpha[id] : 0.0;
+      c6[36 + lane] = flux_cinv_entry<PHYS>(alpha, D, a, b);
     }
-    if (lane == 0 && flux_cinv(ncomp, T.fb_cid, alpha, zv, c6 + 36))
-      for (int t = 0; t < 36; ++t) c6[36 + t] = 0.0;
     wave_sync_lds();
     const double* base = rs.slot + cell * rs.usz;
     const double* Ri = base + rs.ri;
     const double* Auu = base + rs.auu;
     const double* Aqu = base + rs.aqu;
     const double* Auq = base + rs.auq;
-    const double* Wc = rs.w + cell * rs.wsz;
     const double* bi = gen.M.srcq + cell * srcq_stride(T);
-    // ---- c = b_i - A_ib lambda and y - Y lambda -----------------------------------
-    double cu = 0.0;
-#pragma unroll
-    for (int t = 0; t < KQ + 1; ++t) {
-      const int r = lane + 64 * t;
-      if (r < ni) {
-        double v = bi[r];
-        const int k1 = T.prog_rptr[r + 1];
-        for (int k = T.prog_rbsplit[r]; k < k1; ++k)
-          v = fma(-(alpha[T.prog_rid[k]] * T.prog_rval[k]), lam[T.prog_rcol[k] - ni], v);
-        if (r < na) {
-          cq[r] = v;
-        } else {
-          const int u = r - na;
-          double x = Wc[(int64_t)nb * rs.wld + u];
-#pragma unroll 4
-          for (int j = 0; j < nb; ++j) x = fma(-Wc[(int64_t)j * rs.wld + u], lam[j], x);
-          uv[u] = v;
-          xuv[u] = x;
-        }
-      }
-    }
-    wave_sync_lds();
-    if (lane < nu) cu = uv[lane];
-    {  // x_u = U^-1 (y - Y lambda)
-      const double* Ui = base + rs.uinv;
-      double x = 0.0;
-      if (lane < nu)
-#pragma unroll 4
-        for (int c = 0; c < nu; ++c) x = fma(Ui[(int64_t)c * nu + lane], xuv[c], x);
-      wave_sync_lds();
-      if (lane < nu) xuv[lane] = x;
-      wave_sync_lds();
-    }
-    // ---- x_q = A_qq^-1 (c_q - A_qu x_u) -------------------------------------------
-    aqu_apply(Aqu, xuv);
-#pragma unroll
-    for (int t = 0; t < KQ; ++t) {
-      const int r = lane + 64 * t;
+    // ---- c = b_i - A_ib lambda ------------------------------------------------------
+    double cu[KU];
+    for (int r = lane; r < ni; r += 64) {
+      double v = bi[r];
+      const int k1 = T.prog_rptr[r + 1];
+      for (int k = T.prog_rbsplit[r]; k < k1; ++k)
+        v = fma(-(alpha[T.prog_rid[k]] * T.prog_rval[k]), lam[T.prog_rcol[k] - ni], v);
       if (r < na) {
-        aq[r] = qv[r];
-        qv[r] = cq[r] - qv[r];
+        cq[r] = v;
+        xq[r] = 0.0;
+        aq[r] = 0.0;
+      } else {
+        uv[r - na] = v;
+        xuv[r - na] = 0.0;
       }
     }
     wave_sync_lds();
-    flux_apply(qv, Minv, c6 + 36);
 #pragma unroll
-    for (int t = 0; t < KQ; ++t) {
-      const int r = lane + 64 * t;
-      if (r < na) xq[r] = qv[r];
-    }
-    wave_sync_lds();
-    // ---- FP64 refinement against the full interior system ---------------------
+    for (int t = 0; t < KU; ++t) cu[t] = lane + 64 * t < nu ? uv[lane + 64 * t] : 0.0;
+    // ---- the structured solve of c, then of the residuals of the full interior system
 #pragma unroll 1
-    for (int it = 0; it < kFluxRefineSteps; ++it) {
-      // r_q = c_q - (C (x) M) x_q - A_qu x_u  (into zv)
+    for (int it = 0; it <= kFluxRefineSteps; ++it) {
+      double ru[KU];
 #pragma unroll
-      for (int t = 0; t < KQ; ++t) {
-        const int r = lane + 64 * t;
-        if (r < na) zv[r] = xq[r];
-      }
-      wave_sync_lds();
-      flux_apply(zv, Mm, c6);
+      for (int t = 0; t < KU; ++t) ru[t] = cu[t];
+      if (it == 0) {
 #pragma unroll
-      for (int t = 0; t < KQ; ++t) {
-        const int r = lane + 64 * t;
-        if (r < na) zv[r] = (cq[r] - zv[r]) - aq[r];
-      }
-      double ru = 0.0;
-      if (lane < nu) {
-        ru = cu;
+        for (int t = 0; t < KQ; ++t) {
+          const int r = lane + 64 * t;
+          if (r < na) zv[r] = cq[r];
+        }
+      } else {
+        // r_q = c_q - (C (x) M) x_q - A_qu x_u  (into zv)
+#pragma unroll
+        for (int t = 0; t < KQ; ++t) {
+          const int r = lane + 64 * t;
+          if (r < na) zv[r] = xq[r];
+        }
+        wave_sync_lds();
+        flux_apply(zv, Mm, c6);
+#pragma unroll
+        for (int t = 0; t < KQ; ++t) {
+          const int r = lane + 64 * t;
+          if (r < na) zv[r] = (cq[r] - zv[r]) - aq[r];
+        }
+#pragma unroll
+        for (int t = 0; t < KU; ++t) {
+          const int r = lane + 64 * t;
+          if (r < nu) {
+            const int d = REF && PHYS != kDarcy ? r / nq : 0, ld = REF ? nq : nu;
+            const double* av = Auu + (r - d * nq);
+            const double* xv = xuv + d * nq;
 #pragma unroll 4
-        for (int c = 0; c < nu; ++c) ru = fma(-Auu[(int64_t)c * nu + lane], xuv[c], ru);
+            for (int c = 0; c < ld; ++c) ru[t] = fma(-av[(int64_t)c * ld], xv[c], ru[t]);
+          }
+        }
       }
       wave_sync_lds();
       flux_apply(zv, Minv, c6 + 36);  // z = A_qq^-1 r_q
@@ -4561,31 +3983,53 @@ __global__ void __launch_bounds__(256)
       wave_sync_lds();
       // t = r_u - A_uq z = c_u - A_uu x_u - A_uq (x_q + z);  d_u = R_uu^-1 t
       if (REF) {
-        // A_uq = -A_qu^T: s_e[i] = sum_a c_ea qv[(a, i)]; ru += sum_(e,i) G_e[i][u] s_e[i]
-        for (int t = lane; t < D * np; t += 64) {
-          const int e = t / np, i = t - e * np;
+        // A_uq = -A_qu^T: s_de[i] = sum_a c_ea qv[(component of d, a; i)],
+        // ru_d += sum_(e,i) G_e[i][u] s_de[i]
+        for (int t = lane; t < ng; t += 64) {
+          const int d = PHYS == kDarcy ? 0 : t / (D * np), k = t - d * D * np;
+          const int e = k / np, i = k - e * np;
           double acc = 0.0;
-          for (int a = 0; a < D; ++a) acc = fma(-alpha[1 + e * D + a], qv[a * np + i], acc);
+          for (int a = 0; a < D; ++a)
+            acc = fma(cof(e, a), qv[(PHYS == kDarcy ? a : stress(d, a)) * np + i], acc);
           tv[t] = acc;
         }
         wave_sync_lds();
-        if (lane < nu) {
+#pragma unroll
+        for (int t = 0; t < KU; ++t) {
+          const int r = lane + 64 * t;
+          if (r < nu) {
+            const int d = PHYS == kDarcy ? 0 : r / nq, u = r - d * nq;
+            const double* sd = tv + d * D * np;
 #pragma unroll 4
-          for (int t = 0; t < D * np; ++t) ru = fma(gsrc[(int64_t)t * gld + lane], tv[t], ru);
-          uv[lane] = ru;
+            for (int k = 0; k < D * np; ++k) ru[t] = fma(gsrc[(int64_t)k * gld + u], sd[k], ru[t]);
+            uv[r] = ru[t];
+          }
         }
-      } else if (lane < nu) {
+      } else {
+#pragma unroll
+        for (int t = 0; t < KU; ++t) {
+          const int r = lane + 64 * t;
+          if (r < nu) {
 #pragma unroll 4
-        for (int j = 0; j < na; ++j) ru = fma(-Auq[(int64_t)j * nu + lane], qv[j], ru);
-        uv[lane] = ru;
+            for (int j = 0; j < na; ++j) ru[t] = fma(-Auq[(int64_t)j * nu + r], qv[j], ru[t]);
+            uv[r] = ru[t];
+          }
+        }
       }
       wave_sync_lds();
-      double du = 0.0;
-      if (lane < nu)
+      double du[KU];
+#pragma unroll
+      for (int t = 0; t < KU; ++t) {
+        const int r = lane + 64 * t;
+        du[t] = 0.0;
+        if (r < nu)
 #pragma unroll 4
-        for (int j = 0; j < nu; ++j) du = fma(Ri[(int64_t)j * nu + lane], uv[j], du);
+          for (int j = 0; j < nu; ++j) du[t] = fma(Ri[(int64_t)j * nu + r], uv[j], du[t]);
+      }
       wave_sync_lds();
-      if (lane < nu) uv[lane] = du;
+#pragma unroll
+      for (int t = 0; t < KU; ++t)
+        if (lane + 64 * t < nu) uv[lane + 64 * t] = du[t];
       wave_sync_lds();
       // d_q = z - A_qq^-1 (A_qu d_u);  A_qu x_u advances by A_qu d_u
       aqu_apply(Aqu, uv);
@@ -4596,7 +4040,7 @@ __global__ void __launch_bounds__(256)
       }
       wave_sync_lds();
       flux_apply(qv, Minv, c6 + 36);
-      double dmax = lane < nu ? fabs(du) : 0.0, xmax = 0.0;
+      double dmax = 0.0, xmax = 0.0;
 #pragma unroll
       for (int t = 0; t < KQ; ++t) {
         const int r = lane + 64 * t;
@@ -4608,72 +4052,79 @@ __global__ void __launch_bounds__(256)
           xmax = fmax(xmax, fabs(x));
         }
       }
-      if (lane < nu) {
-        const double x = xuv[lane] + du;
-        xuv[lane] = x;
-        xmax = fmax(xmax, fabs(x));
+#pragma unroll
+      for (int t = 0; t < KU; ++t) {
+        const int r = lane + 64 * t;
+        if (r < nu) {
+          const double x = xuv[r] + du[t];
+          xuv[r] = x;
+          dmax = fmax(dmax, fabs(du[t]));
+          xmax = fmax(xmax, fabs(x));
+        }
       }
       wave_sync_lds();
       dmax = __builtin_bit_cast(double, wave_max_i64(__builtin_bit_cast(int64_t, dmax)));
       xmax = __builtin_bit_cast(double, wave_max_i64(__builtin_bit_cast(int64_t, xmax)));
-      if (dmax <= 0x1p-48 * xmax) break;  // wave-uniform
+      if (it > 0 && dmax <= 0x1p-48 * xmax) break;  // wave-uniform
     }
 #pragma unroll
     for (int t = 0; t < KQ; ++t) {
       const int r = lane + 64 * t;
       if (r < na) out[cell * na + r] = xq[r];
     }
-    if (lane < nu) out[ncells * na + cell * nu + lane] = xuv[lane];
+    for (int r = lane; r < nu; r += 64) out[ncells * na + cell * nu + r] = xuv[r];
     wave_sync_lds();
   }
 }
 
-hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U,
-                               const double* Y, int64_t usz, int64_t ysz, bool ref,
-                               const int32_t* cell_dofs, const double* lam_free,
+hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, int64_t usz,
+                               bool ref, const int32_t* cell_dofs, const double* lam_free,
                                const double* lam_dir, double* out, int64_t nfree,
                                hipStream_t st) {
   const int na = T.na, nu = T.ni - na, nb = T.nb;
-  if (na > (ref ? kRecMaxNa : kMixedMaxNi) || nu > 64 || nb > kFusedMaxNb || T.np > kFluxMaxNp)
+  const SysShape sh = sys_shape(T);
+  ref = ref || T.phys != kDarcy;
+  if (na > (ref ? kRecMaxNa : 128) || nu > (ref ? 128 : 64) || nb > kFusedMaxNb ||
+      T.np > kFluxMaxNp)
     return hipErrorInvalidValue;
-  if (ref && (T.phys != kDarcy || !T.fr_G)) return hipErrorInvalidValue;
   RecSlot rs;
   rs.slot = U;
   rs.usz = usz;
-  const FluxSlot fs = flux_slot(na, nu);
-  if (usz < fs.size || ysz < (int64_t)(nb + 1) * nu) return hipErrorInvalidValue;
+  const FluxSlot fs = flux_slot(sh.flux_keep, nu);
+  if (usz < fs.size) return hipErrorInvalidValue;
   rs.ri = fs.ri;
   rs.auu = fs.auu;
   rs.aqu = fs.aqu;
   rs.auq = fs.auq;
-  rs.uinv = fs.uinv;
-  rs.w = Y;
-  rs.wsz = ysz;
-  rs.wld = nu;
   if (M.ncells > 0) {
     const int64_t blocks = (M.ncells + kRecWaves - 1) / kRecWaves;
     const int grid = (int)(blocks < 65536 ? blocks : 65536);
-    const size_t base = (2 * (size_t)T.np * T.np + kRecWaves * (size_t)rec_wave_lds(na, nu, nb)) *
-                        sizeof(double);
-    const size_t gbytes = (size_t)T.D * T.np * nu * sizeof(double);
+    const int ng = ref ? (T.phys == kDarcy ? 1 : T.D) * T.D * T.np : 0;
+    const size_t base =
+        (2 * (size_t)T.np * T.np + kRecWaves * (size_t)rec_wave_lds(na, nu, nb, ng)) *
+        sizeof(double);
+    const size_t gbytes = (size_t)T.D * T.np * T.nq * sizeof(double);
     // G_e in LDS while two workgroups still fit a CU
     const bool g_lds = ref && base + gbytes <= 64 * 1024;
     const size_t lds = base + (g_lds ? gbytes : 0);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     ClockScope clk_(st, "recover_flux");
-#define HDG_RF(P_, K_, R_)                                                                     \
-  hipLaunchKernelGGL((recover_flux_kernel<P_, K_, R_>), dim3(grid), dim3(64 * kRecWaves), lds, \
-                     st, FusedGen<P_>{T, M}, rs, cell_dofs, lam_free, lam_dir, out, g_lds)
+#define HDG_RF(P_, K_, U_, R_)                                                                  \
+  hipLaunchKernelGGL((recover_flux_kernel<P_, K_, U_, R_>), dim3(grid), dim3(64 * kRecWaves),   \
+                     lds, st, FusedGen<P_>{T, M}, rs, cell_dofs, lam_free, lam_dir, out, g_lds)
     if (T.phys == kDarcy) {
       if (ref) {
-        if (na <= 64) HDG_RF(kDarcy, 1, true);
-        else if (na <= 128) HDG_RF(kDarcy, 2, true);
-        else HDG_RF(kDarcy, 3, true);
+        if (nu > 64) HDG_RF(kDarcy, 3, 2, true);
+        else if (na <= 64) HDG_RF(kDarcy, 1, 1, true);
+        else if (na <= 128) HDG_RF(kDarcy, 2, 1, true);
+        else HDG_RF(kDarcy, 3, 1, true);
       } else {
-        if (na <= 64) HDG_RF(kDarcy, 1, false); else HDG_RF(kDarcy, 2, false);
+        if (na <= 64) HDG_RF(kDarcy, 1, 1, false); else HDG_RF(kDarcy, 2, 1, false);
       }
     } else {
-      if (na <= 64) HDG_RF(kElasticity, 1, false); else HDG_RF(kElasticity, 2, false);
+      if (nu > 64 || na > 128) HDG_RF(kElasticity, 3, 2, true);
+      else if (na <= 64) HDG_RF(kElasticity, 1, 1, true);
+      else HDG_RF(kElasticity, 2, 1, true);
     }
 #undef HDG_RF
   }

@@ -345,8 +345,8 @@ int hdg_cell_blocks(hdg_mesh* mesh, const double** S, const double** g,
  * in natural interior order.  After a flux-block condensation (family 8) U
  * and Y are the factors of the reduced system of the m = ni - n_flux
  * non-flux interior unknowns, at the start of each cell's slot (the rest of
- * the slot holds the recovery's kept blocks and the inverses of the reduced
- * factors; not part of this interface).  Cell c's slots start at c * u_stride and c * y_stride
+ * the slot holds the recovery's kept blocks and the inverse of the reduced
+ * interior block; not part of this interface).  Cell c's slots start at c * u_stride and c * y_stride
  * (hdg_mesh_factor_layout). */
 int hdg_local_factors(hdg_mesh* mesh, const double** U, const double** Y);
 /* Layout of the resident factors: rows m of the factored system (ni, or
@@ -411,11 +411,13 @@ typedef struct {
  * updates, 7 16x16 grid (2, 6 and 9 are reserved), 8 flux-block Schur
  * complement: where the flux block of A_ii is C (x) M (per-cell coefficient
  * matrix C, fixed scalar mass matrix M; both weak forms here), the flux
- * unknowns are eliminated with C^-1 (x) M^-1 in two FP64 MFMA products and
- * the reduced system is condensed by one of the families above, 10 the same
- * elimination with the Darcy flux products formed from reference-cell
- * products and each cell's Jacobian cofactors (Darcy with det J > 0; the
- * default there).  With the environment variable HDG_AUTOTUNE_LOG set, the
+ * unknowns are eliminated with C^-1 (x) M^-1 and the reduced system is
+ * condensed by family 11 -- in two FP64 MFMA products per cell (Darcy) or from
+ * reference-cell products and each cell's Jacobian cofactors (elasticity, the
+ * default there) -- 10 the latter for Darcy with det J > 0 (the default for its
+ * larger classes), 11 blocked elimination with the interior block in LDS and
+ * FP64 MFMA products (map level and reduced systems; interiors of at most 128
+ * unknowns).  With the environment variable HDG_AUTOTUNE_LOG set, the
  * autotuner prints every candidate's time to stderr. */
 
 /* flags: HDG_BATCH_AUTOTUNE times every kernel family and grid size able to
