@@ -864,11 +864,12 @@ void detect_flux_sym(TablesHost& t) {
 //   fr_ub  H_(e, fix(F)) on potential x trace columns [e][i][(F, m)];
 //   fr_bb  H_(fix(F), fix(F')) on the trace columns;
 //   fr_qm  Fqm as [i][(F, m)];
+//   fr_mm  Fmm as [(F, m)][(F', m')], zero between facets;
 //   fr_hm  (Darcy) H_e = M^-1 G_e [e][i][column], for a flux right-hand side;
 //   fr_G   G_e.
 void build_flux_ref(TablesHost& t) {
   t.fr_npair = 0;
-  for (auto* v : {&t.fr_uu, &t.fr_ub, &t.fr_bb, &t.fr_qm, &t.fr_hm, &t.fr_G}) v->clear();
+  for (auto* v : {&t.fr_uu, &t.fr_ub, &t.fr_bb, &t.fr_qm, &t.fr_mm, &t.fr_hm, &t.fr_G}) v->clear();
   const int D = t.D, np = t.np, nq = t.nq, nm = t.nm, nF = t.nF, nbs = nF * nm;
   const bool darcy = t.phys == kDarcy;
   if ((t.fb_sym & 1) == 0 || t.fb_minv.empty()) return;
@@ -940,6 +941,10 @@ void build_flux_ref(TablesHost& t) {
   for (int r = 0; r < nq; ++r)
     for (int b = 0; b < nbs; ++b)
       t.fr_qm[(size_t)r * nbs + b] = t.Fqm[((size_t)(b / nm) * nq + r) * nm + b % nm];
+  t.fr_mm.assign((size_t)nbs * nbs, 0.0);
+  for (int b = 0; b < nbs; ++b)
+    for (int m = 0; m < nm; ++m)
+      t.fr_mm[(size_t)b * nbs + b / nm * nm + m] = t.Fmm[(size_t)(b % nm) * nm + m];
   t.fr_G.assign(G.size(), 0.0);
   for (size_t k = 0; k < G.size(); ++k) t.fr_G[k] = (double)G[k];
   if (darcy) t.fr_hm.assign(H.begin(), H.end());

@@ -78,6 +78,7 @@ struct TablesHost {
   std::vector<double> fr_ub;  // [D][nq][nbs]
   std::vector<double> fr_bb;  // [nbs][nbs]
   std::vector<double> fr_qm;  // [nq][nbs]
+  std::vector<double> fr_mm;  // [nbs][nbs]
   std::vector<double> fr_hm;  // [D][np][nq + nbs] (Darcy)
   std::vector<double> fr_G;   // [D][np][nq + nbs]
 };
@@ -123,6 +124,7 @@ struct Tables {
   const double* fr_ub;
   const double* fr_bb;
   const double* fr_qm;
+  const double* fr_mm;
   const double* fr_hm;
   const double* fr_G;
 };

@@ -414,6 +414,7 @@ struct DenseShared {
   int dummy;
 };
 struct DenseGen {
+  static constexpr bool kHeavy = false, kStoresY = false;
   DenseIn in;
   using Shared = DenseShared;
   __device__ void begin(int64_t, Shared&) const {}
@@ -427,6 +428,7 @@ struct DenseGen {
 
 // Dense backward map: rows/cols = interior only; rhs = b_i - A_ib x.
 struct BackwardGen {
+  static constexpr bool kHeavy = false, kStoresY = false;
   DenseIn in;
   const double* x;  // [ncells][nb]
   using Shared = DenseShared;
@@ -2481,9 +2483,13 @@ int condense_grid_options(int fam, int* gm, int max) {
 static size_t flux_workspace_bytes(int nr, int64_t ncells);
 
 int condense_default_family(const SysShape& sh) {
-  // small systems stay with the register-resident kernels (one wavefront or
-  // an 8x8 grid per cell), which no two-stage scheme beats
-  if ((sh.flux || sh.ref) && !wave_class(sh.ni, sh.nb) && sh.ni + sh.nb > 96)
+  // Where the flux block goes through reference products the reduced system wins
+  // from the 48 + 16 and 32 + 24 rows of Darcy 2D k=3 and 3D k=1 on (a step of
+  // 16,247 cells 1,113 -> 470 us, of 13,547 cells 696 -> 400 us, against the
+  // wavefront kernel with a row per lane); at 12 + 8 it loses (512^2 cells
+  // 2.27 -> 2.88 ms).  27 + 12 belong to the wavefront kernel by contract: its
+  // factor is that of all 27 rows.  Elasticity's products win from 54 + 54.
+  if ((sh.flux || sh.ref) && sh.ni + sh.nb > (sh.ref ? 44 : 96))
     return sh.ref ? kFamRef : kFamFlux;
   return default_family(sh.ni, sh.nb, true);
 }
@@ -3490,6 +3496,7 @@ __global__ void __launch_bounds__(64 * kFluxWaves, 3)  // two workgroups per CU
 // for the regular elimination kernels (rows and columns in reduced order, the
 // last column is the right-hand side).
 struct ReducedGen {
+  static constexpr bool kHeavy = false, kStoresY = true;
   const double* R;  // [count][nc][nr]
   int nr;
   using Shared = DenseShared;
