@@ -742,7 +742,7 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
                                                    &th.Fpm, &th.Fqm, &th.Fmm, &th.Bp, &th.Bq,
                                                    &th.xq, &th.fb_minv, &th.fr_uu, &th.fr_ub,
                                                    &th.fr_bb, &th.fr_qm, &th.fr_mm, &th.fr_hm,
-                                                   &th.fr_G};
+                                                   &th.fr_G, &th.fr_Gt};
     size_t nd = 0;
     for (auto* v : dv) nd += v->size();
     size_t bytes = nd * sizeof(double) + th.prog_val.size() * sizeof(double) +
@@ -826,7 +826,7 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
     T.nqc = th.nqc;
     const double** ptrs[] = {&T.Mpp, &T.Gpq, &T.Gqp, &T.Fqp, &T.Fqq, &T.Fpm, &T.Fqm,
                              &T.Fmm, &T.Bp,  &T.Bq,  &T.xq,  &T.fb_minv, &T.fr_uu, &T.fr_ub,
-                             &T.fr_bb, &T.fr_qm, &T.fr_mm, &T.fr_hm, &T.fr_G};
+                             &T.fr_bb, &T.fr_qm, &T.fr_mm, &T.fr_hm, &T.fr_G, &T.fr_Gt};
     for (size_t i = 0; i < dv.size(); ++i) *ptrs[i] = reinterpret_cast<const double*>(base + offs[i]);
     T.pmask = reinterpret_cast<const uint8_t*>(base + off_pm);
     T.qmask = reinterpret_cast<const uint8_t*>(base + off_qm);

@@ -866,10 +866,12 @@ void detect_flux_sym(TablesHost& t) {
 //   fr_qm  Fqm as [i][(F, m)];
 //   fr_mm  Fmm as [(F, m)][(F', m')], zero between facets;
 //   fr_hm  (Darcy) H_e = M^-1 G_e [e][i][column], for a flux right-hand side;
-//   fr_G   G_e.
+//   fr_G   G_e, [e][i][column]; fr_Gt  the same as [e][column][i].
 void build_flux_ref(TablesHost& t) {
   t.fr_npair = 0;
-  for (auto* v : {&t.fr_uu, &t.fr_ub, &t.fr_bb, &t.fr_qm, &t.fr_mm, &t.fr_hm, &t.fr_G}) v->clear();
+  for (auto* v : {&t.fr_uu, &t.fr_ub, &t.fr_bb, &t.fr_qm, &t.fr_mm, &t.fr_hm, &t.fr_G,
+                  &t.fr_Gt})
+    v->clear();
   const int D = t.D, np = t.np, nq = t.nq, nm = t.nm, nF = t.nF, nbs = nF * nm;
   const bool darcy = t.phys == kDarcy;
   if ((t.fb_sym & 1) == 0 || t.fb_minv.empty()) return;
@@ -947,6 +949,11 @@ void build_flux_ref(TablesHost& t) {
       t.fr_mm[(size_t)b * nbs + b / nm * nm + m] = t.Fmm[(size_t)(b % nm) * nm + m];
   t.fr_G.assign(G.size(), 0.0);
   for (size_t k = 0; k < G.size(); ++k) t.fr_G[k] = (double)G[k];
+  t.fr_Gt.assign(G.size(), 0.0);
+  for (int e = 0; e < D; ++e)
+    for (int i = 0; i < np; ++i)
+      for (int c = 0; c < nr; ++c)
+        t.fr_Gt[((size_t)e * nr + c) * np + i] = t.fr_G[((size_t)e * np + i) * nr + c];
   if (darcy) t.fr_hm.assign(H.begin(), H.end());
 }
 

@@ -81,6 +81,7 @@ struct TablesHost {
   std::vector<double> fr_mm;  // [nbs][nbs]
   std::vector<double> fr_hm;  // [D][np][nq + nbs] (Darcy)
   std::vector<double> fr_G;   // [D][np][nq + nbs]
+  std::vector<double> fr_Gt;  // [D][nq + nbs][np]
 };
 
 // Device view of the tables (pointers into one device allocation).
@@ -127,6 +128,7 @@ struct Tables {
   const double* fr_mm;
   const double* fr_hm;
   const double* fr_G;
+  const double* fr_Gt;
 };
 
 // Device view of a mesh for the fused element generator.
@@ -158,7 +160,8 @@ struct CondenseOut {
   // per-cell slots of the full interior so every family shares one layout
   int64_t u_stride = 0, y_stride = 0;
   // (tile elimination, per cell at cell * u_stride) A_ii^-1 and, from the
-  // reference products, the kept block A_uu, both [col][row]
+  // reference products where the recovery reads it, the block A_uu, both
+  // [col][row]
   double* Rinv = nullptr;
   double* Auu = nullptr;
 };

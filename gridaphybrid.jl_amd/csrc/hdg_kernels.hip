@@ -3647,6 +3647,8 @@ static hipError_t launch_flux_schur(const Tables& T, const MeshDev& M, const Con
   return hipSuccess;
 }
 
+#include "recover_ref.h"
+
 hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                 hipStream_t st, Workspace& ws, int gridmul, bool ref) {
   const SysShape sh = sys_shape(T);
@@ -3660,7 +3662,7 @@ hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const Condens
   const FluxSlot fs = flux_slot(sh.flux_keep, nu);
   if (T.phys == kDarcy && !ref) return launch_flux_schur(T, M, out, fs, st, ws, gridmul);
   CondenseOut o = out;
-  o.Auu = out.U + fs.auu;
+  if (!rec_by_group(T, M.ncells)) o.Auu = out.U + fs.auu;
   o.Rinv = out.U + fs.ri;
   if (T.phys == kDarcy)
     return T.D == 2 ? launch_tile_ref<kDarcy, 2>(T, M, o, st, gridmul)
@@ -3676,7 +3678,7 @@ size_t factor_slot(const SysShape& sh) {
 }
 
 // The reference decomposition has kernels for the sizes: the tile elimination
-// and the recovery (one wavefront per cell, at most kRecMaxNa flux rows).
+// and the recovery (at most kRecMaxNa flux rows).
 static bool ref_fits(int npair, int na, int np, int ni, int nb) {
   if (npair <= 0 || na <= 0 || na >= ni || na > kRecMaxNa || nb > kFusedMaxNb) return false;
   return ref_tile_ok(ni - na, nb, np);
@@ -3703,7 +3705,8 @@ SysShape sys_shape(const Tables& T) { return shape_of(T, T.fb_minv != nullptr); 
 
 SysShape sys_shape(const TablesHost& t) { return shape_of(t, !t.fb_minv.empty()); }
 
-// Flux recovery, one wavefront per cell, for both flux families.  The cell's
+// Flux recovery, one wavefront per cell (family 8, elasticity, and small meshes
+// of small Darcy classes; others recover_ref_kernel).  The cell's
 // slot holds R_uu^-1 of the reduced system and the interior blocks A_uu, A_qu,
 // A_uq (RecSlot gives where).  With c = b_i - A_ib lambda (boundary columns of
 // the program), the structured solve of a right-hand side r is
@@ -4103,7 +4106,11 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
   rs.auu = fs.auu;
   rs.aqu = fs.aqu;
   rs.auq = fs.auq;
-  if (M.ncells > 0) {
+  if (M.ncells > 0 && ref && rec_by_group(T, M.ncells)) {
+    const auto go = T.D == 2 ? launch_recover_ref<2> : launch_recover_ref<3>;
+    const hipError_t e = go(T, M, U + fs.ri, usz, cell_dofs, lam_free, lam_dir, out, st);
+    if (e != hipSuccess) return e;
+  } else if (M.ncells > 0) {
     const int64_t blocks = (M.ncells + kRecWaves - 1) / kRecWaves;
     const int grid = (int)(blocks < 65536 ? blocks : 65536);
     const int ng = ref ? (T.phys == kDarcy ? 1 : T.D) * T.D * T.np : 0;
