@@ -572,7 +572,10 @@ __global__ void __launch_bounds__(PR * PC)
         for (int r = 0; r < R; ++r) {
           const int row = tr + PR * r;
           const bool cand = row < ni && ((act >> r) & 1u);
-          const double av = cand ? fabs(colv[r]) : -1.0;
+          // (NaN ranks highest: a column of nothing else must still name a row, the
+          // positions index the outputs)
+          const double mag = fabs(colv[r]);
+          const double av = !cand ? -1.0 : (mag == mag ? mag : HUGE_VAL);
           const int pr = s_pos[row];
           const bool better = av > bav || (av == bav && cand && pr < bpos);
           bav = better ? av : bav;
