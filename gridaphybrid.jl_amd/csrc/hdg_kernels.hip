@@ -1607,7 +1607,12 @@ __global__ void assemble_kernel(PairTable P, const double* __restrict__ S,
 // rhs: for free dof (G, m), sum over cells around G (ascending) of
 // g_c[i] - sum_{j Dirichlet} S_c[i, j] lam_dir (Gridap _attach_dirichlet).
 // Only cells flagged in glpos have Dirichlet dofs; the others skip the scan
-// of their dof row, which otherwise is most of the kernel's traffic.
+// of their dof row, which otherwise is most of the kernel's traffic.  Bounded by
+// the latency of that scan: the dofs and values of kRhsChunk columns are loaded
+// together, then S where a value is not zero (a column after the other: 175 us
+// for 8 cells with 180 columns, 242 us for 1,728; so 43 and 61 us).
+constexpr int kRhsChunk = 16;
+
 __global__ void rhs_kernel(PairTable P, const double* __restrict__ S, const double* __restrict__ g,
                            const int32_t* __restrict__ cell_dofs, const double* __restrict__ lam_dir,
                            double* __restrict__ rhs) {
@@ -1627,12 +1632,30 @@ __global__ void rhs_kernel(PairTable P, const double* __restrict__ S, const doub
       double v = g[(int64_t)c * nb + i];
       if (gl & kGlposDirichlet) {
         const int32_t* d = cell_dofs + (int64_t)c * nb;
-        for (int j = 0; j < nb; ++j) {
-          const int32_t dj = d[j];
-          if (dj < 0) {
-            const double ld = lam_dir[-(int64_t)dj - 1];
-            if (ld != 0.0) v -= S[((int64_t)c * nb + j) * nb + i] * ld;
+        for (int j0 = 0; j0 < nb; j0 += kRhsChunk) {
+          int32_t dj[kRhsChunk];
+          double ld[kRhsChunk];
+#pragma unroll
+          for (int u = 0; u < kRhsChunk; ++u) dj[u] = d[min(j0 + u, nb - 1)];
+          int32_t lo = 0;
+#pragma unroll
+          for (int u = 0; u < kRhsChunk; ++u) lo = min(lo, dj[u]);
+          if (lo >= 0) continue;
+          bool any = false;
+#pragma unroll
+          for (int u = 0; u < kRhsChunk; ++u) {
+            ld[u] = lam_dir[dj[u] < 0 ? -(int64_t)dj[u] - 1 : 0];
+            if (j0 + u >= nb || dj[u] >= 0) ld[u] = 0.0;
+            any |= ld[u] != 0.0;
           }
+          if (!any) continue;
+          const double* const Sr = S + (int64_t)c * nb * nb + i;
+          double sv[kRhsChunk];
+#pragma unroll
+          for (int u = 0; u < kRhsChunk; ++u)
+            sv[u] = Sr[ld[u] != 0.0 ? (int64_t)(j0 + u) * nb : 0];
+#pragma unroll
+          for (int u = 0; u < kRhsChunk; ++u) v = ld[u] != 0.0 ? v - sv[u] * ld[u] : v;
         }
       }
       acc += v;
