@@ -130,12 +130,13 @@ __device__ inline double sel3(const double* x, int i) {
   return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]);
 }
 
-__device__ inline double elas_h(int D, const double* x, int i, int j, int k) {
+// sn[i] = sin(pi (x_i + x_{i+1}/2)): the D distinct sines, once per point
+__device__ inline double elas_h(int D, const double* sn, int i, int j, int k) {
   // d2 u_i / dx_j dx_k of u_i = sin(pi (x_i + x_{i+1}/2))
   const int i1 = (i + 1) % D;
   const double dj = (j == i ? 1.0 : 0.0) + (j == i1 ? 0.5 : 0.0);
   const double dk = (k == i ? 1.0 : 0.0) + (k == i1 ? 0.5 : 0.0);
-  return -M_PI * M_PI * sin(M_PI * (sel3(x, i) + 0.5 * sel3(x, i1))) * dj * dk;
+  return -M_PI * M_PI * sel3(sn, i) * dj * dk;
 }
 
 __device__ inline void elas_source(int src, int D, const double* x, double E, double nu,
@@ -144,15 +145,18 @@ __device__ inline void elas_source(int src, int D, const double* x, double E, do
   if (src != 12) return;  // the linear displacement has zero body load
   const double lam = E * nu / ((1.0 + nu) * (1.0 - (D - 1) * nu));
   const double mu2 = E / (1.0 + nu);
+  double sn[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) sn[i] = sin(M_PI * (x[i] + 0.5 * (i + 1 < D ? sel3(x, i + 1) : x[0])));
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     if (j >= D) break;
     double s = 0.0;
     for (int i = 0; i < D; ++i) {
-      const double deps = 0.5 * (elas_h(D, x, i, j, i) + elas_h(D, x, j, i, i));
+      const double deps = 0.5 * (elas_h(D, sn, i, j, i) + elas_h(D, sn, j, i, i));
       double dtr = 0.0;
       if (i == j)
-        for (int q = 0; q < D; ++q) dtr += elas_h(D, x, q, q, i);
+        for (int q = 0; q < D; ++q) dtr += elas_h(D, sn, q, q, i);
       s += mu2 * deps + lam * dtr;
     }
     f[j] = s;
@@ -166,7 +170,6 @@ __device__ inline void elas_source(int src, int D, const double* x, double E, do
 //                        a barrier in the caller)
 //   entry(sh, row, col)  entry (row, col) of [A | b] in condensed order
 // --------------------------------------------------------------------------
-constexpr int kMaxQP = 128;
 
 __device__ inline void sym_pair(int D, int a, int& i, int& j) {
   // upper triangle, row-major: 2D (11,12,22), 3D (11,12,13,22,23,33);
@@ -381,31 +384,6 @@ struct FusedGen {
       if (ok[u] && col[u] >= n) acc = row[u] < T.ni ? sh.b[row[u]] : 0.0;
       out[u] = ok[u] ? acc : 0.0;
     }
-  }
-
-  // right-hand side: per-cell quadrature of the source (|det J| * values at
-  // the cell quadrature points, src[q][component]) against the test basis
-  __device__ double rhs(const double (*src)[4], int row) const {
-    const int D = T.D, np = T.np, nq = T.nq, na = T.na, ni = T.ni;
-    if (row >= ni) return 0.0;
-    double s = 0.0;
-    if (PHYS == kDarcy) {
-      if (row < na) {  // v . f
-        const int a = row / np, i = row - a * np;
-#pragma unroll 4
-        for (int q = 0; q < T.nqc; ++q) s += T.Bp[q * np + i] * src[q][a];
-      } else {  // w g
-        const int i = row - na;
-#pragma unroll 4
-        for (int q = 0; q < T.nqc; ++q) s += T.Bq[q * nq + i] * src[q][D];
-      }
-      return s;
-    }
-    if (row < na) return 0.0;
-    const int c = (row - na) / nq, j = row - na - c * nq;  // -omega . f
-#pragma unroll 4
-    for (int q = 0; q < T.nqc; ++q) s += T.Bq[q * nq + j] * src[q][c];
-    return -s;
   }
 };
 
@@ -2537,29 +2515,87 @@ bool condense_supported(int n) {
   return pick_bucket(n, b) || (n > 64 && n <= kLargeMaxN);
 }
 
-// Interior right-hand side b_i of every cell, one wavefront per cell: a lane
-// per cell quadrature point evaluates |det J| times the source there, then a
-// lane per row runs FusedGen::rhs (the quadrature of the source against the
-// test basis); b_i is kept in the per-cell scratch, so the generators read one
-// value per right-hand-side entry.
-template <int PHYS>
-__global__ void __launch_bounds__(256) cell_rhs_kernel(FusedGen<PHYS> gen) {
-  constexpr int WPB = 4;
-  __shared__ double s_src[WPB][kMaxQP][4];
-  const Tables& T = gen.T;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int64_t cell = (int64_t)blockIdx.x * WPB + w; cell < gen.M.ncells;
-       cell += (int64_t)gridDim.x * WPB) {
-    double* sq = gen.M.srcq + cell * srcq_stride(T);
-    for (int q = lane; q < T.nqc; q += 64) {
-      double v[4];
-      cell_source<PHYS>(T, gen.M, cell, q, v);
+// Interior right-hand side b_i of every cell: the products of the bases at the
+// cell quadrature points (reference tables) with |det J| times the source
+// there, a workgroup per 16 cells.  Its threads evaluate the sources, a (cell,
+// point) each, kRhsPoints points at a time into LDS; its wavefronts then share
+// the 16-row tiles of the outputs (component, rows) as FP64 MFMA products whose
+// columns are the cells.  b_i is kept in the per-cell scratch, so the
+// generators read one value per right-hand-side entry.
+// (Bounded by the sources' sines and the store of b_i, 0.6 TB/s at 64^3 k=2.
+// Against a wavefront per cell with a lane per point, 27 of 64 in 3D k=2, then a
+// lane per row: 64^3 k=2 1,550 -> 384 us, 512^2 k=2 354 -> 105, 24^3 k=3 229 ->
+// 74, elasticity of 5,814 cells k=2 54 -> 28; 1,728 cells k=3 57 -> 74.)
+constexpr int kRhsPoints = 32;
+constexpr int kRhsTiles = 4;  // output tiles of a wavefront in one pass over the points
+
+template <int PHYS, int D>
+__global__ void __launch_bounds__(256) cell_rhs_kernel(Tables T, MeshDev M) {
+  constexpr int NV = PHYS == kDarcy ? D + 1 : D, LD = 17;
+  __shared__ double s_v[NV][kRhsPoints * LD];  // [component][point][cell]
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int i16 = lane & 15, q4 = lane >> 4;
+  const int np = T.np, nq = T.nq, na = T.na, nqc = T.nqc;
+  // output tiles: the potential components, then the flux components (elasticity: 0)
+  const int tq = (nq + 15) >> 4, tp = (np + 15) >> 4;
+  constexpr int NC = PHYS == kDarcy ? D : D * (D + 1) / 2;
+  const int nu = (PHYS == kDarcy ? 1 : D) * tq, nt = nu + NC * tp;
+  const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
+  for (int64_t c0 = (int64_t)blockIdx.x * 16; c0 < M.ncells; c0 += (int64_t)gridDim.x * 16) {
+    const int64_t cell = min(c0 + (tid & 15), M.ncells - 1);
+    double* const sq = M.srcq + cell * srcq_stride(T);
+    for (int t0 = 0; t0 < nt; t0 += 4 * kRhsTiles) {
+      dbl4 acc[kRhsTiles];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) s_src[w][q][c] = v[c];
+      for (int j = 0; j < kRhsTiles; ++j) acc[j] = zero;
+      for (int p0 = 0; p0 < nqc; p0 += kRhsPoints) {
+        const int pn = min(kRhsPoints, nqc - p0), pn4 = (pn + 3) & ~3;
+        bool flux = false;
+        for (int p = tid >> 4; p < pn4; p += 16) {
+          double v[4];
+          cell_source<PHYS>(T, M, cell, min(p0 + p, nqc - 1), v);
+#pragma unroll
+          for (int c = 0; c < NV; ++c) {
+            const double x = p < pn ? v[c] : 0.0;
+            s_v[c][p * LD + (tid & 15)] = x;
+            if (PHYS == kDarcy && c < D) flux |= x != 0.0;
+          }
+        }
+        flux = __syncthreads_or(flux);
+#pragma unroll
+        for (int j = 0; j < kRhsTiles; ++j) {
+          const int t = t0 + w + 4 * j;  // wave-uniform
+          if (t >= (PHYS == kDarcy && flux ? nt : nu)) continue;
+          const bool u = t < nu;
+          const int c = u ? (PHYS == kDarcy ? D : t / tq) : (t - nu) / tp;
+          const int n = u ? nq : np, r = 16 * (u ? t % tq : (t - nu) % tp) + i16;
+          const double* const B = (u ? T.Bq : T.Bp) + min(r, n - 1);
+          double b[kRhsPoints / 4];  // a chunk's in flight together
+#pragma unroll
+          for (int s = 0; s < kRhsPoints / 4; ++s)
+            b[s] = B[(int64_t)min(p0 + 4 * s + q4, nqc - 1) * n];
+#pragma unroll
+          for (int s = 0; s < kRhsPoints / 4; ++s)
+            if (4 * s < pn4)
+              acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[s], s_v[c][(4 * s + q4) * LD + i16],
+                                                            acc[j], 0, 0, 0);
+        }
+        __syncthreads();
+      }
+      if (c0 + i16 >= M.ncells) continue;  // (no barrier before the next pass's first)
+#pragma unroll
+      for (int j = 0; j < kRhsTiles; ++j) {
+        const int t = t0 + w + 4 * j;
+        if (t >= nt) continue;
+        const bool u = t < nu;
+        const int c = u ? (PHYS == kDarcy ? 0 : t / tq) : (t - nu) / tp;
+        const int n = u ? nq : np, r0 = 16 * (u ? t % tq : (t - nu) % tp) + q4;
+        double* const dst = sq + (u ? na + c * nq : c * np);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (r0 + 4 * v < n) dst[r0 + 4 * v] = PHYS == kDarcy ? acc[j][v] : -acc[j][v];
+      }
     }
-    wave_sync_lds();
-    for (int r = lane; r < T.ni; r += 64) sq[r] = gen.rhs(s_src[w], r);
-    wave_sync_lds();
   }
 }
 
@@ -2577,15 +2613,13 @@ static hipError_t launch_prep(const Tables& T, const MeshDev& M, hipStream_t st)
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int64_t wblocks = (M.ncells + 3) / 4;
-  const int wgrid = (int)(wblocks < 65536 ? wblocks : 65536);
+  const int wgrid = (int)std::min<int64_t>((M.ncells + 15) / 16, 1 << 16);
   ClockScope clk_(st, "prep_rhs");
-  if (T.phys == kDarcy)
-    hipLaunchKernelGGL(cell_rhs_kernel<kDarcy>, dim3(wgrid), dim3(256), 0, st,
-                       FusedGen<kDarcy>{T, M});
-  else
-    hipLaunchKernelGGL(cell_rhs_kernel<kElasticity>, dim3(wgrid), dim3(256), 0, st,
-                       FusedGen<kElasticity>{T, M});
+  const auto kernel = T.phys == kDarcy
+                          ? (T.D == 2 ? cell_rhs_kernel<kDarcy, 2> : cell_rhs_kernel<kDarcy, 3>)
+                          : (T.D == 2 ? cell_rhs_kernel<kElasticity, 2>
+                                      : cell_rhs_kernel<kElasticity, 3>);
+  hipLaunchKernelGGL(kernel, dim3(wgrid), dim3(256), 0, st, T, M);
   return hipGetLastError();
 }
 
