@@ -1464,7 +1464,7 @@ int hdg_skeleton_solve(hdg_mesh* m, double rtol, int maxit, double* lam_free, in
   auto true_residual = [&](double bnorm) -> hipError_t {
     hipError_t e = launch_spmv_sym(colptr, rowval, nzval, x, t, n, 1.0, st);
     if (e == hipSuccess)
-      e = launch_krylov_update(3, n, 0, 0, 0, 0, t, nullptr, rhs, t, nullptr, st);
+      e = launch_subtract(n, t, rhs, t, st);
     if (e == hipSuccess) e = dots(1, t, t, nullptr, nullptr);
     res = std::sqrt(h[0]) / bnorm;
     return e;
@@ -1493,26 +1493,18 @@ int hdg_skeleton_solve(hdg_mesh* m, double rtol, int maxit, double* lam_free, in
   bool conv = false;
   while (it < maxit && !conv) {
     ++it;
-    HIP_TRY(ctx, launch_krylov_update_dev(2, n, sc, MS::kInvBeta, -1, -1, -1, v, nullptr, y,
-                                          nullptr, nullptr, st), "v");
-    HIP_TRY(ctx, launch_spmv_sym(colptr, rowval, nzval, v, y, n, 1.0, st), "spmv");
-    if (it >= 2)
-      HIP_TRY(ctx, launch_krylov_update_dev(0, n, sc, MS::kBetaOldb, -1, -1, -1, r1, y, nullptr,
-                                            nullptr, nullptr, st), "y");
-    HIP_TRY(ctx, launch_multidot(1, n, v, y, nullptr, nullptr, nullptr, nullptr, scr, st), "dot");
-    HIP_TRY(ctx, launch_minres_scalar(1, dres, sc, st), "alfa");
-    HIP_TRY(ctx, launch_krylov_update_dev(0, n, sc, MS::kAlfaBeta, -1, -1, -1, r2, y, nullptr,
-                                          nullptr, nullptr, st), "y");
-    std::swap(r1, r2);  // r1 <- r2, r2 <- y, y <- the old r1
-    std::swap(r2, y);
-    HIP_TRY(ctx, launch_block_apply(binv, r2, y, n, bs, st), "precond");
-    HIP_TRY(ctx, launch_multidot(1, n, r2, y, nullptr, nullptr, nullptr, nullptr, scr, st), "dot");
-    HIP_TRY(ctx, launch_minres_scalar(2, dres, sc, st), "rotation");
+    // t = K v - (beta / oldb) r1, v = y / beta; alfa = (v, t)
+    HIP_TRY(ctx, launch_lanczos_spmv(colptr, rowval, nzval, y, it >= 2 ? r1 : nullptr, sc, v, t, n,
+                                     st), "spmv");
+    HIP_TRY(ctx, launch_multidot(1, n, v, t, nullptr, nullptr, nullptr, nullptr, scr, st, 1, sc),
+            "alfa");
+    // r1 <- r2, r2 <- t - (alfa / beta) r2, y <- preconditioned r2; rotation
+    HIP_TRY(ctx, launch_lanczos_apply(binv, t, r2, sc, r1, y, n, bs, scr, st), "precond");
+    std::swap(r1, r2);
     // w1 <- w2, w2 <- w, w <- (v - oldeps w1 - delta w2) / gamma; x += phi w
     std::swap(w1, w2);  // w1 = old w2, w2 = old w1 (dead)
     std::swap(w2, w);   // w2 = old w, w = dead buffer
-    HIP_TRY(ctx, launch_krylov_update_dev(1, n, sc, MS::kOldEps, MS::kDelta, MS::kInvGamma,
-                                          MS::kPhi, w, x, v, w1, w2, st), "w, x");
+    HIP_TRY(ctx, launch_minres_update(n, w, x, v, w1, w2, sc, st), "w, x");
     if (it % kCheck == 0 || it == maxit) {
       HIP_TRY(ctx, hipMemcpyAsync(hs, sc, sizeof hs, hipMemcpyDeviceToHost, st), "d2h");
       HIP_TRY(ctx, hipStreamSynchronize(st), "sync");

@@ -331,9 +331,8 @@ hipError_t launch_block_inv(const int64_t* colptr, const int32_t* rowval, const 
                             double* binv, int64_t nblk, int bs, hipStream_t st);
 hipError_t launch_block_apply(const double* binv, const double* r, double* z, int64_t n, int bs,
                               hipStream_t st);
-hipError_t launch_krylov_update(int op, int64_t n, double a, double b, double c, double d,
-                                double* u0, double* u1, const double* w0, const double* w1,
-                                const double* w2, hipStream_t st);
+hipError_t launch_subtract(int64_t n, double* u, const double* a, const double* b,
+                           hipStream_t st);
 int block_jacobi_max();
 // MINRES scalar state kept on the device (indices into a double array)
 struct MinresScalar {
@@ -342,16 +341,25 @@ struct MinresScalar {
     kAlfaBeta, kOldEps, kDelta, kInvGamma, kPhi, kFrozen, kIndefinite, kCount
   };
 };
-hipError_t launch_krylov_update_dev(int op, int64_t n, const double* sc, int ia, int ib, int ic,
-                                    int id, double* u0, double* u1, const double* w0,
-                                    const double* w1, const double* w2, hipStream_t st);
+// one Lanczos step: v = z / beta, y = K v - (beta / oldb) r1 (r1 may be null);
+// r2n = y - (alfa / beta) r2, z = M^-1 r2n, and the rotation from (r2n, z)
+hipError_t launch_lanczos_spmv(const int64_t* colptr, const int32_t* rowval, const double* nzval,
+                               const double* z, const double* r1, const double* sc, double* v,
+                               double* y, int64_t n, hipStream_t st);
+hipError_t launch_lanczos_apply(const double* binv, const double* y, const double* r2, double* sc,
+                                double* r2n, double* z, int64_t n, int bs, double* scratch,
+                                hipStream_t st);
+hipError_t launch_minres_update(int64_t n, double* w, double* x, const double* v, const double* w1,
+                                const double* w2, const double* sc, hipStream_t st);
 // step 0: init from dot[0] = (r1, M^-1 r1); 1: alfa = dot[0]; 2: beta^2 = dot[0]
 hipError_t launch_minres_scalar(int step, const double* dot, double* sc, hipStream_t st);
 size_t multidot_scratch_doubles();
-// nd (1..3) dot products (a_k, b_k); the sums land in scratch[3 * 1024 + k]
+// nd (1..3) dot products (a_k, b_k); the sums land in scratch[3 * 1024 + k] (sc:
+// and the first of them takes the recurrences' step)
 hipError_t launch_multidot(int nd, int64_t n, const double* a0, const double* b0,
                            const double* a1, const double* b1, const double* a2,
-                           const double* b2, double* scratch, hipStream_t st);
+                           const double* b2, double* scratch, hipStream_t st,
+                           int step = 0, double* sc = nullptr);
 hipError_t launch_gather(const double* src, const int64_t* idx, double* dst, int64_t n,
                          hipStream_t st);
 hipError_t launch_copy(const double* src, double* dst, int64_t n, hipStream_t st);

@@ -2682,6 +2682,34 @@ __global__ void __launch_bounds__(256) spmv_sym_kernel(const int64_t* __restrict
   }
 }
 
+// The Lanczos step's product: v = z / beta (written as it is gathered) and
+// y = K v - (beta / oldb) r1 (r1 null in the first step).  Iterations of small
+// systems are bound by their launches, which this and lanczos_apply_kernel cut
+// from 12 to 6 (a request of 6 x 5 x 5 cells of k=2, 100 iterations: 5.61 -> 3.92 ms).
+__global__ void __launch_bounds__(256) lanczos_spmv_kernel(const int64_t* __restrict__ colptr,
+                                                           const int32_t* __restrict__ rowval,
+                                                           const double* __restrict__ nzval,
+                                                           const double* __restrict__ z,
+                                                           const double* __restrict__ r1,
+                                                           const double* __restrict__ sc,
+                                                           double* __restrict__ v,
+                                                           double* __restrict__ y, int64_t n) {
+  const int lane = threadIdx.x & 63;
+  const double a = sc[MinresScalar::kInvBeta], b = sc[MinresScalar::kBetaOldb];
+  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < n;
+       i += ((int64_t)gridDim.x * blockDim.x) >> 6) {
+    const int64_t k0 = colptr[i], k1 = colptr[i + 1];
+    double acc = 0.0;
+    for (int64_t k = k0 + lane; k < k1; k += 64) acc = fma(nzval[k], a * z[rowval[k]], acc);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) {
+      v[i] = a * z[i];
+      y[i] = r1 ? fma(-b, r1[i], acc) : acc;
+    }
+  }
+}
+
 constexpr int kBlkMax = 32;  // largest diagonal block of the block-Jacobi preconditioner
 
 // SPD preconditioner blocks: for each bs x bs diagonal block B of K (rows
@@ -2771,52 +2799,39 @@ __global__ void block_apply_kernel(const double* __restrict__ binv,
   }
 }
 
-// MINRES vector updates; with sc non-null the coefficients are read from the
-// device scalar state (MinresScalar indices in ia, ib, ic, id; < 0: 0):
-// op 0: y = y - a u0                        (u0 = r1 or r2)
-// op 1: w = (v - a w1 - b w2) c, x += d w   (u0 = w, u1 = x, w0 = v, w1 = w1, w2 = w2)
-// op 2: u0 = a w0
-// op 3: u0 = w0 - w1                        (the residual b - K x)
-__global__ void krylov_update_kernel(int op, int64_t n, double a, double b, double c, double d,
-                                     double* u0, double* u1, const double* w0,
-                                     const double* w1, const double* w2, const double* sc,
-                                     int ia, int ib, int ic, int id) {
-  if (sc) {
-    a = ia >= 0 ? sc[ia] : 0.0;
-    b = ib >= 0 ? sc[ib] : 0.0;
-    c = ic >= 0 ? sc[ic] : 0.0;
-    d = id >= 0 ? sc[id] : 0.0;
-  }
+// MINRES solution update with the device scalar state:
+// w = (v - oldeps w1 - delta w2) / gamma, x += phi w
+__global__ void minres_update_kernel(int64_t n, double* w, double* x, const double* v,
+                                     const double* w1, const double* w2, const double* sc) {
+  const double a = sc[MinresScalar::kOldEps], b = sc[MinresScalar::kDelta],
+               c = sc[MinresScalar::kInvGamma], d = sc[MinresScalar::kPhi];
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    if (op == 0) {
-      u1[i] = fma(-a, u0[i], u1[i]);
-    } else if (op == 1) {
-      const double wv = (w0[i] - a * w1[i] - b * w2[i]) * c;
-      u0[i] = wv;
-      u1[i] = fma(d, wv, u1[i]);
-    } else if (op == 2) {
-      u0[i] = a * w0[i];
-    } else {
-      u0[i] = w0[i] - w1[i];
-    }
+    const double wv = (v[i] - a * w1[i] - b * w2[i]) * c;
+    w[i] = wv;
+    x[i] = fma(d, wv, x[i]);
   }
+}
+
+// u = a - b (the residual b - K x; u may be b)
+__global__ void subtract_kernel(int64_t n, double* u, const double* a, const double* b) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    u[i] = a[i] - b[i];
 }
 
 constexpr int kDotBlocks = 1024;
 
-// MINRES recurrences on the device (one thread): step 0 initialises from
+// MINRES recurrences on the device (by one thread): step 0 initialises from
 // (r1, y) = beta1^2; step 1 takes alfa = (v, y); step 2 takes beta^2 = (r2, y)
 // and advances the Givens rotation.  A zero beta (the Krylov space is
 // exhausted) or a negative beta^2 (an indefinite preconditioner) freezes the
 // state: every later update is then a no-op, and the host reads the flags.
-__global__ void minres_scalar_kernel(int step, const double* __restrict__ dot,
-                                     double* __restrict__ sc) {
+__device__ inline void minres_scalar(int step, double dot0, double* sc) {
   using M = MinresScalar;
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
   const bool frozen = sc[M::kFrozen] != 0.0;
   if (step == 0) {
-    const double b1 = dot[0] > 0.0 ? sqrt(dot[0]) : 0.0;
+    const double b1 = dot0 > 0.0 ? sqrt(dot0) : 0.0;
     sc[M::kBeta1] = b1;
     sc[M::kBeta] = b1;
     sc[M::kPhibar] = b1;
@@ -2827,9 +2842,9 @@ __global__ void minres_scalar_kernel(int step, const double* __restrict__ dot,
     sc[M::kSn] = 0.0;
     sc[M::kInvBeta] = b1 > 0.0 ? 1.0 / b1 : 0.0;
     sc[M::kFrozen] = b1 > 0.0 ? 0.0 : 1.0;
-    sc[M::kIndefinite] = dot[0] < 0.0 ? 1.0 : 0.0;
+    sc[M::kIndefinite] = dot0 < 0.0 ? 1.0 : 0.0;
   } else if (step == 1) {
-    const double alfa = frozen ? 0.0 : dot[0];
+    const double alfa = frozen ? 0.0 : dot0;
     sc[M::kAlfa] = alfa;
     sc[M::kAlfaBeta] = frozen ? 0.0 : alfa / sc[M::kBeta];
   } else {
@@ -2841,10 +2856,10 @@ __global__ void minres_scalar_kernel(int step, const double* __restrict__ dot,
       sc[M::kAlfaBeta] = 0.0;
       return;
     }
-    if (dot[0] < 0.0) sc[M::kIndefinite] = 1.0;
+    if (dot0 < 0.0) sc[M::kIndefinite] = 1.0;
     const double alfa = sc[M::kAlfa], cs = sc[M::kCs], sn = sc[M::kSn], dbar = sc[M::kDbar];
     const double oldb = sc[M::kBeta];
-    const double beta = dot[0] > 0.0 ? sqrt(dot[0]) : 0.0;
+    const double beta = dot0 > 0.0 ? sqrt(dot0) : 0.0;
     const double oldeps = sc[M::kEpsln];
     const double delta = cs * dbar + sn * alfa;
     const double gbar = sn * dbar - cs * alfa;
@@ -2866,6 +2881,11 @@ __global__ void minres_scalar_kernel(int step, const double* __restrict__ dot,
     sc[M::kBetaOldb] = beta / oldb;
     if (!(beta > 0.0)) sc[M::kFrozen] = 1.0;
   }
+}
+
+__global__ void minres_scalar_kernel(int step, const double* __restrict__ dot,
+                                     double* __restrict__ sc) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) minres_scalar(step, dot[0], sc);
 }
 
 // up to three dot products at once: per-block partial sums in a fixed order,
@@ -2894,7 +2914,9 @@ __global__ void __launch_bounds__(256) multidot_kernel(int nd, int64_t n, const 
   if (threadIdx.x < 3) partial[threadIdx.x * kDotBlocks + blockIdx.x] = s_red[threadIdx.x][0];
 }
 
-__global__ void __launch_bounds__(256) dot_finish_kernel(const double* partial, double* out) {
+// (sc: and with the first sum the MINRES recurrences' step)
+__global__ void __launch_bounds__(256) dot_finish_kernel(const double* partial, double* out,
+                                                         int step, double* sc) {
   __shared__ double s_red[3][256];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -2910,6 +2932,37 @@ __global__ void __launch_bounds__(256) dot_finish_kernel(const double* partial, 
     __syncthreads();
   }
   if (threadIdx.x < 3) out[threadIdx.x] = s_red[threadIdx.x][0];
+  if (sc && threadIdx.x == 0) minres_scalar(step, s_red[0][0], sc);
+}
+
+// The Lanczos step's second half: r2' = y - (alfa / beta) r2, z = blockdiag(binv)
+// r2', and the partial sums of (r2', z) in multidot_kernel's order.  A thread per
+// row forms its block's r2' for itself.
+__global__ void __launch_bounds__(256) lanczos_apply_kernel(
+    const double* __restrict__ binv, const double* __restrict__ y, const double* __restrict__ r2,
+    const double* __restrict__ sc, double* __restrict__ r2n, double* __restrict__ z, int64_t n,
+    int bs, double* __restrict__ partial) {
+  __shared__ double s_red[256];
+  const double a = sc[MinresScalar::kAlfaBeta];
+  double dot = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r0 = i - i % bs;
+    const double* b = binv + i * bs;
+    double acc = 0.0;
+    for (int j = 0; j < bs; ++j) acc = fma(b[j], fma(-a, r2[r0 + j], y[r0 + j]), acc);
+    const double r = fma(-a, r2[i], y[i]);
+    r2n[i] = r;
+    z[i] = acc;
+    dot = fma(r, acc, dot);
+  }
+  s_red[threadIdx.x] = dot;
+  __syncthreads();
+  for (int h = 128; h >= 1; h >>= 1) {
+    if ((int)threadIdx.x < h) s_red[threadIdx.x] += s_red[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) partial[blockIdx.x] = s_red[0];
 }
 
 static int vec_grid(int64_t n) {
@@ -2944,21 +2997,39 @@ hipError_t launch_block_apply(const double* binv, const double* r, double* z, in
   return hipGetLastError();
 }
 
-hipError_t launch_krylov_update(int op, int64_t n, double a, double b, double c, double d,
-                                double* u0, double* u1, const double* w0, const double* w1,
-                                const double* w2, hipStream_t st) {
+hipError_t launch_lanczos_spmv(const int64_t* colptr, const int32_t* rowval, const double* nzval,
+                               const double* z, const double* r1, const double* sc, double* v,
+                               double* y, int64_t n, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(krylov_update_kernel, dim3(vec_grid(n)), dim3(256), 0, st, op, n, a, b, c,
-                     d, u0, u1, w0, w1, w2, (const double*)nullptr, -1, -1, -1, -1);
+  const int64_t blocks = (n + 3) / 4;  // four rows (wavefronts) per workgroup
+  ClockScope clk_(st, "skeleton_spmv");
+  hipLaunchKernelGGL(lanczos_spmv_kernel, dim3((unsigned)(blocks < 65536 ? blocks : 65536)),
+                     dim3(256), 0, st, colptr, rowval, nzval, z, r1, sc, v, y, n);
   return hipGetLastError();
 }
 
-hipError_t launch_krylov_update_dev(int op, int64_t n, const double* sc, int ia, int ib, int ic,
-                                    int id, double* u0, double* u1, const double* w0,
-                                    const double* w1, const double* w2, hipStream_t st) {
+hipError_t launch_lanczos_apply(const double* binv, const double* y, const double* r2, double* sc,
+                                double* r2n, double* z, int64_t n, int bs, double* scratch,
+                                hipStream_t st) {
+  hipLaunchKernelGGL(lanczos_apply_kernel, dim3(kDotBlocks), dim3(256), 0, st, binv, y, r2, sc,
+                     r2n, z, n, bs, scratch);
+  hipLaunchKernelGGL(dot_finish_kernel, dim3(1), dim3(256), 0, st, scratch,
+                     scratch + 3 * kDotBlocks, 2, sc);
+  return hipGetLastError();
+}
+
+hipError_t launch_minres_update(int64_t n, double* w, double* x, const double* v, const double* w1,
+                                const double* w2, const double* sc, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(krylov_update_kernel, dim3(vec_grid(n)), dim3(256), 0, st, op, n, 0.0, 0.0,
-                     0.0, 0.0, u0, u1, w0, w1, w2, sc, ia, ib, ic, id);
+  hipLaunchKernelGGL(minres_update_kernel, dim3(vec_grid(n)), dim3(256), 0, st, n, w, x, v, w1, w2,
+                     sc);
+  return hipGetLastError();
+}
+
+hipError_t launch_subtract(int64_t n, double* u, const double* a, const double* b,
+                           hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(subtract_kernel, dim3(vec_grid(n)), dim3(256), 0, st, n, u, a, b);
   return hipGetLastError();
 }
 
@@ -2973,13 +3044,14 @@ size_t multidot_scratch_doubles() { return 3 * (size_t)kDotBlocks + 3; }
 
 hipError_t launch_multidot(int nd, int64_t n, const double* a0, const double* b0,
                            const double* a1, const double* b1, const double* a2,
-                           const double* b2, double* scratch, hipStream_t st) {
+                           const double* b2, double* scratch, hipStream_t st, int step,
+                           double* sc) {
   hipLaunchKernelGGL(multidot_kernel, dim3(kDotBlocks), dim3(256), 0, st, nd, n, a0, b0,
                      a1 ? a1 : a0, b1 ? b1 : b0, a2 ? a2 : a0, b2 ? b2 : b0, scratch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(dot_finish_kernel, dim3(1), dim3(256), 0, st, scratch,
-                     scratch + 3 * kDotBlocks);
+                     scratch + 3 * kDotBlocks, step, sc);
   return hipGetLastError();
 }
 
