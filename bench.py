@@ -68,17 +68,17 @@ def kernel_model(kname, info, D, sweeps, family=None, nqc=0):
         return "hbm", 8 * (D + D * D + 1 + ni), "byte"
     if kname == "condense_tile":
         # the tile elimination of the flux families' reduced systems: reads the
-        # cell coefficients (72) and b_i; writes S, g, U (packed), the kept block
-        # A_uu of one potential component, R_uu^-1 and Y
-        nq = nu // (1 if nu * D == na else D)
+        # cell coefficients (72) and b_i; writes S, g, U (packed), R_uu^-1, Y and
+        # (but for Darcy's reference products) A_uu of one potential component
+        nq = 0 if family == 10 else nu // (1 if nu * D == na else D)
         return "hbm", 8 * (72 + ni + nb * nb + nb + nu * (nu + 1) // 2 + nq * nq + nu * nu
                            + (nb + 1) * nu), "byte"
     if kname == "recover_flux":
-        # reads A_uu, R_uu^-1 (and, for the MFMA-product family, the kept A_qu
+        # reads R_uu^-1 (and, for the MFMA-product family, the kept A_uu, A_qu
         # and A_uq), the cell coefficients and b_i, the cell's trace values and
         # ids; writes (q, u)
-        kept = 0 if family == 10 else 2 * na * nu
-        return "hbm", 8 * (2 * nu * nu + kept + 72 + ni + nb + ni) + 4 * nb, "byte"
+        kept = 0 if family == 10 else nu * nu + 2 * na * nu
+        return "hbm", 8 * (nu * nu + kept + 72 + ni + nb + ni) + 4 * nb, "byte"
     if kname == "assemble":
         # reads every S block once; writes the CSC values
         return "hbm", 8 * nb * nb + 8 * int(info.nnz) / nc, "byte"
