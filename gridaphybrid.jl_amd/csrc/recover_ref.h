@@ -15,9 +15,9 @@
 // LDS as [row][cell].  R_uu^-1, the one block of a cell's own, is applied with a
 // thread per (cell, row), the only large read of a step.
 //
-// What bounds it: the latency of R_uu^-1's columns (8 in flight a thread; all
-// in all 1.6 TB/s at 64^3 k=2) and of the chained products; MFMA issue is a
-// fifth.  Measured against a wavefront per cell (recover_flux_kernel):
+// What bounds it: the latency of R_uu^-1's columns (8 in flight a thread; 3.0
+// TB/s at 64^3 k=2, read once a step) and of the chained products; MFMA issue is
+// a fifth.  Measured against a wavefront per cell (recover_flux_kernel):
 //   64^3 k=2 7.61 -> 1.74 ms, 24^3 k=3 3.08 -> 0.62 ms, 2D k=3, 16,247 cells,
 //   136 -> 56 us, 3D k=1, 13,547 cells, 92 -> 46 us.
 // Elasticity's six components and 12 to 21 coefficients a cell fill the
