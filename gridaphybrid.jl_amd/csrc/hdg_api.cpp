@@ -119,6 +119,7 @@ struct hdg_mesh {
   // its grid; the family of the last condensation decides the recovery
   int family = -1, gridmul = 0;
   int used_family = -1;
+  bool rec_group = false;  // (family 10) the recovery's kernel, by which the condensation kept A_uu
   DevBuf d_fptr, d_pptr, d_pfacet, d_pcell, d_plpos, d_gcell, d_glpos;
   DevBuf d_pperm, d_gperm, d_iperm;  // allocated for oriented meshes only
   // trace split into trace_fields scalar fields (hdg_mesh_set_trace_fields):
@@ -181,6 +182,11 @@ struct CellLayout {
         alpha(72),
         srcq((size_t)t.ni) {}  // interior right-hand side b_i
 };
+
+// After a condensation by `family`, the mesh recovers 16 cells a workgroup.
+bool recovers_by_group(const hdg_mesh* m, int family) {
+  return family == kFamilyFluxRef && recover_by_group(m->tdev, m->ncells);
+}
 
 // Allocates the mesh's own per-cell state (S, g, U, Y, alpha, srcq, info) and
 // binds the kernel pointers to it.
@@ -1267,6 +1273,8 @@ int hdg_condense(hdg_mesh* m, int precision) {
   } else {
     out.U = m->pU;
     const int fam = m->family >= 0 ? m->family : condense_default_family(sys_shape(m->tdev));
+    m->rec_group = recovers_by_group(m, fam);
+    out.keep_uu = !m->rec_group;
     HIP_TRY(ctx, launch_condense_fused(m->tdev, m->meshdev(), out, ctx->stream, ctx->ws, true,
                                        fam, m->gridmul),
             "condense kernel");
@@ -1572,7 +1580,7 @@ int recover_facet_major(hdg_mesh* m, const double* lam_free, double* free_values
   if (m->used_family == kFamilyFluxSchur || m->used_family == kFamilyFluxRef) {
     const CellLayout L(m->th);
     HIP_TRY(ctx, launch_recover_flux(m->tdev, m->meshdev(), m->pU, (int64_t)L.U,
-                                     m->used_family == kFamilyFluxRef,
+                                     m->used_family == kFamilyFluxRef, m->rec_group,
                                      m->d_cell_dofs.as<int32_t>(), lam_free,
                                      m->d_lam_dir.as<double>(), free_values, m->nfree,
                                      ctx->stream),
@@ -1618,6 +1626,7 @@ struct hdg_batch {
     const hdg_mesh* lead = nullptr;  // reference tables shared by the members
     DevBuf S, g, U, Y, alpha, srcq, infos, iters, xinv;
     bool mixed = false;  // condensed in mixed precision at the last launch
+    bool keep_uu = false;  // some member's recovery reads A_uu
     // the class's branch of the batch graph: its own stream (captured after a
     // fork from the context stream), workspace and join event, so that the
     // classes' preparation, condensation and assembly run concurrently
@@ -1647,6 +1656,7 @@ struct hdg_batch {
       const CellLayout L(lead->th);
       o.u_stride = (int64_t)L.U;
       o.y_stride = (int64_t)L.Y;
+      o.keep_uu = keep_uu;
       return o;
     }
   };
@@ -1896,6 +1906,7 @@ int hdg_batch_create(hdg_ctx* ctx, int nmesh, hdg_mesh* const* meshes, int flags
     c->members.push_back(i);
     c->info.nmesh++;
     c->info.ncells += m->ncells;
+    c->keep_uu |= !recover_by_group(m->tdev, m->ncells);
   }
   HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream), "sync");
@@ -2008,6 +2019,7 @@ int hdg_batch_launch(hdg_batch* b, int precision) {
       m->condensed = true;
       m->mixed = c->mixed;
       m->used_family = c->mixed ? -1 : c->info.family;
+      m->rec_group = recovers_by_group(m, m->used_family);
       m->fp64_fallback = false;
     }
   }

@@ -164,6 +164,10 @@ struct CondenseOut {
   // [col][row]
   double* Rinv = nullptr;
   double* Auu = nullptr;
+  // a recovery of these cells reads A_uu (some of them by recover_flux_kernel:
+  // a batch's class is condensed in one launch, its members recover by
+  // themselves)
+  bool keep_uu = true;
 };
 
 // Dense cell systems in HBM for the map-level API.
@@ -296,9 +300,14 @@ hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const Condens
 // Recovery after a flux-block condensation (families 8 and 10): the structured
 // solve through R_uu^-1 and C^-1 (x) M^-1, refined in FP64 against the residual
 // of the full interior system (the reduced system is worse conditioned than
-// A_ii).
+// A_ii).  group: 16 cells a workgroup (after family 10 only) instead of a
+// wavefront per cell, which reads the condensation's A_uu; whoever condenses
+// decides with recover_by_group on the cells of one recovery and keeps the
+// answer for it.
+bool recover_by_group(const Tables& T, int64_t ncells);
 hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, int64_t usz,
-                               bool ref, const int32_t* cell_dofs, const double* lam_free,
+                               bool ref, bool group, const int32_t* cell_dofs,
+                               const double* lam_free,
                                const double* lam_dir, double* out, int64_t nfree,
                                hipStream_t st);
 constexpr int kFluxRefineSteps = 2;  // FP64 refinement steps of the flux recovery (at most)

@@ -3794,7 +3794,7 @@ hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const Condens
   const FluxSlot fs = flux_slot(sh.flux_keep, nu);
   if (T.phys == kDarcy && !ref) return launch_flux_schur(T, M, out, fs, st, ws, gridmul);
   CondenseOut o = out;
-  if (!rec_by_group(T, M.ncells)) o.Auu = out.U + fs.auu;
+  if (out.keep_uu) o.Auu = out.U + fs.auu;
   o.Rinv = out.U + fs.ri;
   if (T.phys == kDarcy)
     return T.D == 2 ? launch_tile_ref<kDarcy, 2>(T, M, o, st, gridmul)
@@ -4220,9 +4220,9 @@ __global__ void __launch_bounds__(256)
 }
 
 hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, int64_t usz,
-                               bool ref, const int32_t* cell_dofs, const double* lam_free,
-                               const double* lam_dir, double* out, int64_t nfree,
-                               hipStream_t st) {
+                               bool ref, bool group, const int32_t* cell_dofs,
+                               const double* lam_free, const double* lam_dir, double* out,
+                               int64_t nfree, hipStream_t st) {
   const int na = T.na, nu = T.ni - na, nb = T.nb;
   const SysShape sh = sys_shape(T);
   ref = ref || T.phys != kDarcy;
@@ -4238,7 +4238,7 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
   rs.auu = fs.auu;
   rs.aqu = fs.aqu;
   rs.auq = fs.auq;
-  if (M.ncells > 0 && ref && rec_by_group(T, M.ncells)) {
+  if (M.ncells > 0 && group) {
     const auto go = T.D == 2 ? launch_recover_ref<2> : launch_recover_ref<3>;
     const hipError_t e = go(T, M, U + fs.ri, usz, cell_dofs, lam_free, lam_dir, out, st);
     if (e != hipSuccess) return e;

@@ -374,8 +374,10 @@ __global__ void __launch_bounds__(512, 2)
 // Which cells come here: with one row tile (np, nq <= 16) a wavefront per cell
 // is faster below about 2,000 cells (77 cells of 2D k=3 23 against 33 us, 2,400
 // cells 36 against 33, 125 cells of 3D k=1 18 against 31); with more, never
-// (8 cells of 3D k=2 59 and 59 us, of k=3 168 and 127).
-static bool rec_by_group(const Tables& T, int64_t ncells) {
+// (8 cells of 3D k=2 59 and 59 us, of k=3 168 and 127).  Asked by whoever
+// condenses, once, with the cells of one recovery: it decides whether A_uu is
+// kept (a batch's class has more cells than each of its meshes).
+bool recover_by_group(const Tables& T, int64_t ncells) {
   const int rows = std::max(T.np, T.nq);
   return T.phys == kDarcy && rows <= 128 &&
          rec_ref_lds(T.D, T.np, T.nq, T.nb) * sizeof(double) <= 160 * 1024 &&
