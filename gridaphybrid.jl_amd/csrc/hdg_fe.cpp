@@ -882,8 +882,10 @@ void build_flux_ref(TablesHost& t) {
       for (int b = 0; b < D; ++b)
         if (t.fb_cid[6 * a + b] != (a == b ? 0 : -1)) return;
   } else {
-    // s_u = s_b = -1, C the compliance in the first 36 coefficients
-    if (t.fb_nc != D * (D + 1) / 2 || (t.fb_sym & 6) != 6) return;
+    // s_u = s_b = -1, C the compliance in the first 36 coefficients (piecewise
+    // constant stresses: no coupling to the potential, which has no sign then)
+    const bool qu = std::any_of(t.Gpq.begin(), t.Gpq.end(), [](double v) { return v != 0.0; });
+    if (t.fb_nc != D * (D + 1) / 2 || (t.fb_sym & 6) != (qu ? 6 : 4)) return;
     for (int a = 0; a < t.fb_nc; ++a)
       for (int b = 0; b < t.fb_nc; ++b)
         if (t.fb_cid[6 * a + b] != 6 * a + b) return;
