@@ -831,13 +831,13 @@ __device__ inline void tile_inverse(const Tile<NT>& tl, const int* perm, dbl4 (&
 // --------------------------------------------------------------------------
 template <int NT, class Gen>
 struct TileGroup {
-  static constexpr int kWaves = NT <= 4 ? 4 : 8;
+  static constexpr int kWaves = NT <= 5 ? 4 : 8;
   // strips per wavefront.  (A generator whose Y is stored anyway rereads it; one
   // that keeps its strips of Y in registers beside Z's has room for two of four
-  // tiles each, or one of seven.)
-  static constexpr int kStrips = NT <= 4 || Gen::kStoresY ? 2 : 1;
-  static constexpr int kHold = NT <= 4 || !Gen::kStoresY ? kStrips : 1;  // strips of Z at a time
-  static constexpr int kMinBlocks = NT <= 4 ? 2 : 1;  // workgroups per CU: two wavefronts a SIMD
+  // tiles each, two of five with one of Z's at a time, or one of seven.)
+  static constexpr int kStrips = NT <= 5 || Gen::kStoresY ? 2 : 1;
+  static constexpr int kHold = NT <= 4 || (NT > 5 && !Gen::kStoresY) ? kStrips : 1;  // strips of Z at a time
+  static constexpr int kMinBlocks = NT <= 5 ? 2 : 1;  // workgroups per CU: two wavefronts a SIMD
 };
 
 template <int NT, class Gen, bool BACKSUB>
@@ -1167,7 +1167,13 @@ __global__ void __launch_bounds__(64, 3)
 // boundary columns per wavefront (a wavefront per cell: four strips).
 static bool tile_one_wave(int ni, int nb) { return ni <= 32 && nb < 64; }
 
-static int tile_nt(int ni) { return ni <= 64 ? 4 : (ni <= 112 ? 7 : 8); }
+// Row tiles of a workgroup's kernel.  With seven, 65 to 80 rows took a workgroup a
+// CU and up to 1.16 times the time of the panel kernel they had before on few
+// boundary columns and many cells; with five, two workgroups share a CU
+// (forward map with the caller's transposes, panel kernel, seven and five tiles:
+// 3,000 cells of 72 + 16 1,325, 1,474 and 817 us, 6,000 of 80 + 40 3,868, 3,501
+// and 2,055 us).
+static int tile_nt(int ni) { return ni <= 64 ? 4 : ni <= 80 ? 5 : ni <= 112 ? 7 : 8; }
 
 // (stored: the generators that store Y, with two strips a wavefront throughout)
 static bool tile_ok(int ni, int nb, bool stored = false) {
@@ -1228,6 +1234,7 @@ static hipError_t launch_tile(const Gen& gen, const CondenseOut& out, int64_t nc
     return launch_tile_small<Gen, BACKSUB>(gen, out, ncells, ni, nb, st, gridmul);
   switch (tile_nt(ni)) {
     case 4: return launch_tile_nt<4, Gen, BACKSUB>(gen, out, ncells, ni, nb, st, gridmul);
+    case 5: return launch_tile_nt<5, Gen, BACKSUB>(gen, out, ncells, ni, nb, st, gridmul);
     case 7: return launch_tile_nt<7, Gen, BACKSUB>(gen, out, ncells, ni, nb, st, gridmul);
     default: return launch_tile_nt<8, Gen, BACKSUB>(gen, out, ncells, ni, nb, st, gridmul);
   }
