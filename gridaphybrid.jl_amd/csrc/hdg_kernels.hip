@@ -3837,8 +3837,8 @@ SysShape sys_shape(const Tables& T) { return shape_of(T, T.fb_minv != nullptr); 
 
 SysShape sys_shape(const TablesHost& t) { return shape_of(t, !t.fb_minv.empty()); }
 
-// Flux recovery, one wavefront per cell (family 8, elasticity, and small meshes
-// of small Darcy classes; others recover_ref_kernel).  The cell's
+// Flux recovery, one wavefront per cell (family 8, elasticity, and Darcy's
+// meshes that recover_by_group leaves here; others recover_ref_kernel).  The cell's
 // slot holds R_uu^-1 of the reduced system and the interior blocks A_uu, A_qu,
 // A_uq (RecSlot gives where).  With c = b_i - A_ib lambda (boundary columns of
 // the program), the structured solve of a right-hand side r is
@@ -3892,7 +3892,7 @@ __device__ inline double flux_cinv_entry(const double* alpha, int D, int a, int 
 //   elasticity: (A_qu v)[(s, i)] = sum over the components d of s = (p, q) of
 //               sum_e c_e,partner t_de[i],  t_de = G_e v_d;
 // and A_uq = -A_qu^T; A_uu is kept for one potential component.  G_e is staged
-// in LDS once per workgroup (g_lds), or, where it does not fit (3D Darcy k=3),
+// in LDS once per workgroup (g_lds), or, where it does not fit (2D Darcy k=6),
 // read from the table, which every cell shares (L2-resident).
 template <int PHYS, int KQ, int KU, bool REF>
 __global__ void __launch_bounds__(256)
@@ -4260,10 +4260,9 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
                      lds, st, FusedGen<P_>{T, M}, rs, cell_dofs, lam_free, lam_dir, out, g_lds)
     if (T.phys == kDarcy) {
       if (ref) {
-        if (nu > 64) HDG_RF(kDarcy, 3, 2, true);
-        else if (na <= 64) HDG_RF(kDarcy, 1, 1, true);
-        else if (na <= 128) HDG_RF(kDarcy, 2, 1, true);
-        else HDG_RF(kDarcy, 3, 1, true);
+        // (one row tile, or 2D: at most 98 + 64 rows)
+        if (na > 128 || nu > 64) return hipErrorInvalidValue;
+        if (na <= 64) HDG_RF(kDarcy, 1, 1, true); else HDG_RF(kDarcy, 2, 1, true);
       } else {
         if (na <= 64) HDG_RF(kDarcy, 1, 1, false); else HDG_RF(kDarcy, 2, 1, false);
       }

@@ -373,15 +373,18 @@ __global__ void __launch_bounds__(512, 2)
 
 // Which cells come here: with one row tile (np, nq <= 16) a wavefront per cell
 // is faster below about 2,000 cells (77 cells of 2D k=3 23 against 33 us, 2,400
-// cells 36 against 33, 125 cells of 3D k=1 18 against 31); with more, never
-// (8 cells of 3D k=2 59 and 59 us, of k=3 168 and 127).  Asked by whoever
-// condenses, once, with the cells of one recovery: it decides whether A_uu is
-// kept (a batch's class has more cells than each of its meshes).
+// cells 36 against 33, 125 cells of 3D k=1 18 against 31); in 2D with more
+// below about 1,000 (a recovery with its launch and copies, k=4: 256 cells 52
+// against 65 us, 1,024 53 against 65, 2,116 72 against 65; k=5: 73 against 82, 76
+// against 82, 144 against 84; k=6: 93 against 109, 111 against 110, 215 against
+// 117); in 3D with more never (8 cells of k=2 59 and 59 us, of k=3 168 and 127).
+// Asked by whoever condenses, once, with the cells of one recovery: it decides
+// whether A_uu is kept (a batch's class has more cells than each of its meshes).
 bool recover_by_group(const Tables& T, int64_t ncells) {
   const int rows = std::max(T.np, T.nq);
   return T.phys == kDarcy && rows <= 128 &&
          rec_ref_lds(T.D, T.np, T.nq, T.nb) * sizeof(double) <= 160 * 1024 &&
-         (rows > 16 || ncells >= 2048);
+         ncells >= (rows <= 16 ? 2048 : T.D == 2 ? 1024 : 0);
 }
 
 template <int D>

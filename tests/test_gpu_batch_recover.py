@@ -1,8 +1,8 @@
 """Recovery of a batch's members: a class's meshes are condensed in one launch, so
 what that launch keeps for the recovery has to serve every member, whatever
 kernel its own number of cells takes.  Darcy classes of one row tile (2D k=3, 3D
-k=1) with members on both sides of the recovery's 2,048 cells, and members below
-it whose class is above, against each mesh alone and the direct solve of the
+k=1) with members on both sides of the recovery's 2,048 cells (2D with more tiles:
+1,024), and members below it whose class is above, against each mesh alone and the direct solve of the
 cells' interior systems; the factor slots are filled with NaN before the launch
 that counts."""
 import numpy as np
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 # (D, k, members)
 CLASSES = [(2, 3, ((60, 60), (8, 8))), (2, 3, ((39, 41), (33, 31))),
-           (3, 1, ((13, 13, 13), (3, 3, 3))), (3, 1, ((3, 3, 3), (12, 12, 11), (9, 9, 9)))]
+           (3, 1, ((13, 13, 13), (3, 3, 3))), (3, 1, ((3, 3, 3), (12, 12, 11), (9, 9, 9))),
+           (2, 4, ((33, 32), (9, 7))), (2, 5, ((6, 5), (32, 33)))]
 
 
 class _Slots:
