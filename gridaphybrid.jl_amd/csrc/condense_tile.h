@@ -1229,7 +1229,7 @@ static hipError_t launch_tile_small(const Gen& gen, const CondenseOut& out, int6
 template <class Gen, bool BACKSUB>
 static hipError_t launch_tile(const Gen& gen, const CondenseOut& out, int64_t ncells, int ni,
                               int nb, hipStream_t st, int gridmul) {
-  if (!tile_ok(ni, nb, Gen::kStoresY)) return hipErrorInvalidValue;
+  if (!tile_ok(ni, nb)) return hipErrorInvalidValue;
   if (tile_one_wave(ni, nb))
     return launch_tile_small<Gen, BACKSUB>(gen, out, ncells, ni, nb, st, gridmul);
   switch (tile_nt(ni)) {

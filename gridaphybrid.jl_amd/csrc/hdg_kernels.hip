@@ -3773,7 +3773,10 @@ static hipError_t launch_flux_schur(const Tables& T, const MeshDev& M, const Con
     o.y_stride = ysz;
     o.Rinv = o.U + fs.ri;
     o.info = out.info ? out.info + first : nullptr;
-    e = launch_tile<ReducedGen, false>(ReducedGen{ws.p, nr}, o, count, nu, nb, st, gridmul);
+    const ReducedGen red{ws.p, nr};  // (flux_fits: nu <= 64)
+    e = tile_one_wave(nu, nb)
+            ? launch_tile_small<ReducedGen, false>(red, o, count, nu, nb, st, gridmul)
+            : launch_tile_nt<4, ReducedGen, false>(red, o, count, nu, nb, st, gridmul);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
