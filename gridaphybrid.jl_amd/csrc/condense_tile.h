@@ -148,7 +148,19 @@ struct RefGen {
     const double* al = M.alpha + cell * kMaxAlpha;
     const double* b = M.srcq + cell * srcq_stride(T);
     for (int t = tid; t < kMaxAlpha; t += nthreads) sh.alpha[t] = al[t];
-    for (int t = tid; t < nr; t += nthreads) sh.rhs[t] = t < nu ? b[na + t] : 0.0;
+    if (PHYS != kDarcy && T.fo_P) {  // P^T b_u, a component after the other
+      const int nq = T.nq;
+      for (int t = tid; t < nr; t += nthreads) {
+        const int c = (sh.idx[t] & 0xffff) * 8, d = sh.idx[t] >> 16;
+        double x = 0.0;
+        if (t < nu)
+#pragma unroll 8
+          for (int j = 0; j < nq; ++j) x = fma(table_at(T.fo_P + j * nq, c), b[na + d * nq + j], x);
+        sh.rhs[t] = x;
+      }
+    } else {
+      for (int t = tid; t < nr; t += nthreads) sh.rhs[t] = t < nu ? b[na + t] : 0.0;
+    }
     int load = 0;  // the flux equation's load (none: its terms are skipped)
     if (PHYS == kDarcy)
       for (int t = tid; t < na; t += nthreads) load |= b[t] != 0.0;
@@ -657,7 +669,7 @@ struct Tile {
 // A_ii into F, padded to whole tiles with the identity, by nthreads threads.
 // (Every entry by itself also where A_ii is symmetric: the mirrored triangle
 // was measured 8 times less exact in S, 5.3e-11 against 6.3e-12 of the largest
-// entry, for elasticity with k = 3.)
+// entry, for elasticity with k = 3 in the displacement's nodal basis.)
 template <int NT, class Gen>
 __device__ inline void tile_load(const Gen& gen, const typename Gen::Shared& sh, double* F,
                                  int64_t cell, int ni, int tid, int nthreads, double* keep) {

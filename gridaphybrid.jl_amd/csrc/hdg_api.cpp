@@ -119,6 +119,9 @@ struct hdg_mesh {
   // its grid; the family of the last condensation decides the recovery
   int family = -1, gridmul = 0;
   int used_family = -1;
+  // (family 8, elasticity) U and Y have been asked for: every condensation forms
+  // them, in the potential's own basis
+  bool want_factors = false;
   bool rec_group = false;  // (family 10) the recovery's kernel, by which the condensation kept A_uu
   DevBuf d_fptr, d_pptr, d_pfacet, d_pcell, d_plpos, d_gcell, d_glpos;
   DevBuf d_pperm, d_gperm, d_iperm;  // allocated for oriented meshes only
@@ -211,6 +214,23 @@ hipError_t own_cell_state(hdg_mesh* m) {
   m->pinfo = m->d_info.as<int32_t>();
   m->piters = m->d_iters.as<int32_t>();
   return hipSuccess;
+}
+
+// U and Y of the last condensation where it left them out (launch_flux_factors);
+// the other families write them themselves.
+int form_factors(hdg_mesh* m) {
+  if (m->mixed || m->used_family != kFamilyFluxSchur || !flux_orthonormal(m->tdev)) return HDG_OK;
+  hdg_ctx* ctx = m->ctx;
+  PoolScope pool_(ctx->pool);
+  HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
+  const CellLayout L(m->th);
+  CondenseOut out;
+  out.U = m->pU;
+  out.Y = m->pY;
+  out.u_stride = (int64_t)L.U;
+  out.y_stride = (int64_t)L.Y;
+  HIP_TRY(ctx, launch_flux_factors(m->tdev, m->meshdev(), out, ctx->stream), "factors kernel");
+  return HDG_OK;
 }
 
 // Frees the mesh's own per-cell state (the mesh is rebound to batch slices).
@@ -748,7 +768,9 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
                                                    &th.Fpm, &th.Fqm, &th.Fmm, &th.Bp, &th.Bq,
                                                    &th.xq, &th.fb_minv, &th.fr_uu, &th.fr_ub,
                                                    &th.fr_bb, &th.fr_qm, &th.fr_mm, &th.fr_hm,
-                                                   &th.fr_G, &th.fr_Gt};
+                                                   &th.fr_G, &th.fr_Gt, &th.fo_P, &th.fo_Pt,
+                                                   &th.fo_uu, &th.fo_ub, &th.fo_qm, &th.fo_qq,
+                                                   &th.fo_G};
     size_t nd = 0;
     for (auto* v : dv) nd += v->size();
     size_t bytes = nd * sizeof(double) + th.prog_val.size() * sizeof(double) +
@@ -832,7 +854,9 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
     T.nqc = th.nqc;
     const double** ptrs[] = {&T.Mpp, &T.Gpq, &T.Gqp, &T.Fqp, &T.Fqq, &T.Fpm, &T.Fqm,
                              &T.Fmm, &T.Bp,  &T.Bq,  &T.xq,  &T.fb_minv, &T.fr_uu, &T.fr_ub,
-                             &T.fr_bb, &T.fr_qm, &T.fr_mm, &T.fr_hm, &T.fr_G, &T.fr_Gt};
+                             &T.fr_bb, &T.fr_qm, &T.fr_mm, &T.fr_hm, &T.fr_G, &T.fr_Gt,
+                             &T.fo_P, &T.fo_Pt, &T.fo_uu, &T.fo_ub, &T.fo_qm, &T.fo_qq,
+                             &T.fo_G};
     for (size_t i = 0; i < dv.size(); ++i) *ptrs[i] = reinterpret_cast<const double*>(base + offs[i]);
     T.pmask = reinterpret_cast<const uint8_t*>(base + off_pm);
     T.qmask = reinterpret_cast<const uint8_t*>(base + off_qm);
@@ -853,6 +877,7 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
     T.fb_sym = th.fb_sym;
     std::memcpy(T.fb_cid, th.fb_cid, sizeof(T.fb_cid));
     if (th.fb_minv.empty()) T.fb_minv = nullptr;
+    if (th.fo_P.empty()) T.fo_P = nullptr;
     T.fr_npair = th.fr_npair;
   }
   m->x0.assign(desc->x0, desc->x0 + nc * D);
@@ -1282,7 +1307,7 @@ int hdg_condense(hdg_mesh* m, int precision) {
     m->used_family = fam;
   }
   m->condensed = true;
-  return HDG_OK;
+  return m->want_factors ? form_factors(m) : HDG_OK;
 }
 
 int hdg_assemble(hdg_mesh* m) {
@@ -1386,6 +1411,11 @@ int hdg_cell_blocks(hdg_mesh* m, const double** S, const double** g, const int32
 
 int hdg_local_factors(hdg_mesh* m, const double** U, const double** Y) {
   if (!m) return HDG_ERR_ARG;
+  if (!m->want_factors) {
+    m->want_factors = true;
+    if (m->condensed)
+      if (const int rc = form_factors(m)) return rc;
+  }
   if (U) *U = m->mixed ? nullptr : m->pU;
   if (Y) *Y = m->pY;
   return m->condensed ? HDG_OK : fail(m->ctx, HDG_ERR_STATE, "no factors before condensation");
@@ -2021,6 +2051,8 @@ int hdg_batch_launch(hdg_batch* b, int precision) {
       m->used_family = c->mixed ? -1 : c->info.family;
       m->rec_group = recovers_by_group(m, m->used_family);
       m->fp64_fallback = false;
+      if (m->want_factors)
+        if (const int rc = form_factors(m)) return rc;
     }
   }
   return HDG_OK;

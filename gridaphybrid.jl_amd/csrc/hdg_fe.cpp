@@ -365,6 +365,7 @@ static int build_tables_uncached(int phys, int D, int space, int kp, int kq, int
   t.Gqp.assign((size_t)D * nq * np, 0.0);
   t.Bp.assign((size_t)nqc * np, 0.0);
   t.Bq.assign((size_t)nqc * nq, 0.0);
+  t.Mqq.assign((size_t)nq * nq, 0.0);
   t.xq.assign((size_t)nqc * 3, 0.0);
   t.wq.assign((size_t)nqc, 0.0);
   std::vector<double> vp(np), gp(3 * np), vq(nq), gq(3 * nq), vm(nm);
@@ -388,6 +389,7 @@ static int build_tables_uncached(int phys, int D, int space, int kp, int kq, int
     }
     for (int i = 0; i < nq; ++i) {
       t.Bq[(size_t)q * nq + i] = vq[i] * w;
+      for (int j = 0; j < nq; ++j) t.Mqq[(size_t)i * nq + j] += vq[i] * vq[j] * w;
       for (int e = 0; e < D; ++e)
         for (int j = 0; j < np; ++j) t.Gqp[((size_t)e * nq + i) * np + j] += gq[3 * i + e] * vp[j] * w;
     }
@@ -792,6 +794,7 @@ void detect_flux_block(TablesHost& t) {
       }
     for (int i = 0; i < np * np; ++i) X[i] += D[i];
   }
+  t.fb_minv_l = X;
   t.fb_minv.resize((size_t)np * np);
   for (int i = 0; i < np * np; ++i) t.fb_minv[i] = (double)X[i];
   for (int k = 0; k < 36; ++k) t.fb_cid[k] = (int8_t)(cid[k] >= 0 ? cid[k] : -1);
@@ -867,10 +870,49 @@ void detect_flux_sym(TablesHost& t) {
 //   fr_mm  Fmm as [(F, m)][(F', m')], zero between facets;
 //   fr_hm  (Darcy) H_e = M^-1 G_e [e][i][column], for a flux right-hand side;
 //   fr_G   G_e, [e][i][column]; fr_Gt  the same as [e][column][i].
+//
+// Elasticity has them twice.  The nodal basis of P_(k+1) on the cube (nodes on a
+// simplex, extrapolated) makes R_uu worse conditioned than the problem is: 1.9e8
+// for 3D k=3, where with the potential in a basis orthonormal in the reference
+// mass it is 27.  S and g do not depend on that basis, their rounding does: S of
+// 3D k=3 was 7.0e-12 of its largest entry off with R in the nodal basis, 1.6e-12
+// after a dense elimination of all 225 rows, and is 6.5e-13 off with the
+// orthonormal one; of k=2 2.0e-13, 4.9e-14 and 2.1e-14 (against extended
+// precision; what is left is the rounding of the nodal tables).  fo_*: the tables
+// of that basis, u = fo_P u'; any fo_P is exact, the tables being formed from its
+// rounded entries.  Darcy's R_uu gains nothing (2D k=3: condition 2e5 and 2e4, S
+// 1.8e-15 and 1.6e-15).
+// P with P^T M P = I up to rounding (the transposed inverse of M's Cholesky
+// factor); false if M is not positive definite.
+static bool orthonormal_basis(int n, const std::vector<double>& M, std::vector<double>& P) {
+  std::vector<long double> C((size_t)n * n, 0.0L), X((size_t)n * n, 0.0L);
+  for (int j = 0; j < n; ++j) {
+    long double d = M[(size_t)j * n + j];
+    for (int k = 0; k < j; ++k) d -= C[(size_t)j * n + k] * C[(size_t)j * n + k];
+    // (a pivot lost to rounding: under-integrated or dependent functions)
+    if (!(d > 1e-13L * M[(size_t)j * n + j])) return false;
+    C[(size_t)j * n + j] = std::sqrt(d);
+    for (int i = j + 1; i < n; ++i) {
+      long double v = M[(size_t)i * n + j];
+      for (int k = 0; k < j; ++k) v -= C[(size_t)i * n + k] * C[(size_t)j * n + k];
+      C[(size_t)i * n + j] = v / C[(size_t)j * n + j];
+    }
+  }
+  P.assign((size_t)n * n, 0.0);
+  for (int c = 0; c < n; ++c)  // X = C^-1 by columns, P = X^T
+    for (int i = c; i < n; ++i) {
+      long double v = i == c ? 1.0L : 0.0L;
+      for (int k = c; k < i; ++k) v -= C[(size_t)i * n + k] * X[(size_t)k * n + c];
+      X[(size_t)i * n + c] = v / C[(size_t)i * n + i];
+      P[(size_t)c * n + i] = (double)X[(size_t)i * n + c];
+    }
+  return true;
+}
+
 void build_flux_ref(TablesHost& t) {
   t.fr_npair = 0;
   for (auto* v : {&t.fr_uu, &t.fr_ub, &t.fr_bb, &t.fr_qm, &t.fr_mm, &t.fr_hm, &t.fr_G,
-                  &t.fr_Gt})
+                  &t.fr_Gt, &t.fo_P, &t.fo_Pt, &t.fo_uu, &t.fo_ub, &t.fo_qm, &t.fo_qq, &t.fo_G})
     v->clear();
   const int D = t.D, np = t.np, nq = t.nq, nm = t.nm, nF = t.nF, nbs = nF * nm;
   const bool darcy = t.phys == kDarcy;
@@ -905,42 +947,48 @@ void build_flux_ref(TablesHost& t) {
               nh * (long double)t.Fpm[((size_t)F * np + i) * nm + m];
       }
     }
-  // H_e = M^-1 G_e
-  std::vector<long double> H((size_t)D * np * nr, 0.0L);
-  for (int e = 0; e < D; ++e)
-    for (int i = 0; i < np; ++i)
-      for (int k = 0; k < np; ++k) {
-        const long double m = t.fb_minv[(size_t)i * np + k];
-        for (int c = 0; c < nr; ++c)
-          H[((size_t)e * np + i) * nr + c] += m * G[((size_t)e * np + k) * nr + c];
-      }
-  auto dot = [&](int e, int r, int e2, int c) {
-    long double v = 0.0L;
-    for (int i = 0; i < np; ++i)
-      v += G[((size_t)e * np + i) * nr + r] * H[((size_t)e2 * np + i) * nr + c];
-    return v;
-  };
   auto fix = [&](int b) { return D - 1 - (b / nm) / 2; };
   t.fr_npair = darcy ? D * (D + 1) / 2 : D * D;
-  t.fr_uu.assign((size_t)t.fr_npair * nq * nq, 0.0);
-  int p = 0;
-  for (int e = 0; e < D; ++e)
-    for (int e2 = darcy ? e : 0; e2 < D; ++e2, ++p)
-      for (int r = 0; r < nq; ++r)
-        for (int c = 0; c < nq; ++c) {
-          long double v = dot(e, r, e2, c);
-          if (darcy && e2 != e) v += dot(e2, r, e, c);
-          t.fr_uu[((size_t)p * nq + r) * nq + c] = (double)v;
+  // the products of one basis, and H_e = M^-1 G_e
+  auto products = [&](const std::vector<long double>& G, std::vector<long double>& H,
+                      std::vector<double>& uu, std::vector<double>& ub) {
+    H.assign((size_t)D * np * nr, 0.0L);
+    for (int e = 0; e < D; ++e)
+      for (int i = 0; i < np; ++i)
+        for (int k = 0; k < np; ++k) {
+          const long double m = t.fb_minv_l[(size_t)i * np + k];
+          for (int c = 0; c < nr; ++c)
+            H[((size_t)e * np + i) * nr + c] += m * G[((size_t)e * np + k) * nr + c];
         }
-  t.fr_ub.assign((size_t)D * nq * nbs, 0.0);
-  for (int e = 0; e < D; ++e)
-    for (int r = 0; r < nq; ++r)
-      for (int b = 0; b < nbs; ++b)
-        t.fr_ub[((size_t)e * nq + r) * nbs + b] = (double)dot(e, r, fix(b), nq + b);
-  t.fr_bb.assign((size_t)nbs * nbs, 0.0);
-  for (int b = 0; b < nbs; ++b)
-    for (int b2 = 0; b2 < nbs; ++b2)
-      t.fr_bb[(size_t)b * nbs + b2] = (double)dot(fix(b), nq + b, fix(b2), nq + b2);
+    auto dot = [&](int e, int r, int e2, int c) {
+      long double v = 0.0L;
+      for (int i = 0; i < np; ++i)
+        v += G[((size_t)e * np + i) * nr + r] * H[((size_t)e2 * np + i) * nr + c];
+      return v;
+    };
+    uu.assign((size_t)t.fr_npair * nq * nq, 0.0);
+    int p = 0;
+    for (int e = 0; e < D; ++e)
+      for (int e2 = darcy ? e : 0; e2 < D; ++e2, ++p)
+        for (int r = 0; r < nq; ++r)
+          for (int c = 0; c < nq; ++c) {
+            long double v = dot(e, r, e2, c);
+            if (darcy && e2 != e) v += dot(e2, r, e, c);
+            uu[((size_t)p * nq + r) * nq + c] = (double)v;
+          }
+    ub.assign((size_t)D * nq * nbs, 0.0);
+    for (int e = 0; e < D; ++e)
+      for (int r = 0; r < nq; ++r)
+        for (int b = 0; b < nbs; ++b)
+          ub[((size_t)e * nq + r) * nbs + b] = (double)dot(e, r, fix(b), nq + b);
+    t.fr_bb.assign((size_t)nbs * nbs, 0.0);  // (the same in every basis)
+    for (int b = 0; b < nbs; ++b)
+      for (int b2 = 0; b2 < nbs; ++b2)
+        t.fr_bb[(size_t)b * nbs + b2] = (double)dot(fix(b), nq + b, fix(b2), nq + b2);
+  };
+  std::vector<long double> H;
+  products(G, H, t.fr_uu, t.fr_ub);
+  if (darcy) t.fr_hm.assign(H.begin(), H.end());
   t.fr_qm.assign((size_t)nq * nbs, 0.0);
   for (int r = 0; r < nq; ++r)
     for (int b = 0; b < nbs; ++b)
@@ -956,7 +1004,37 @@ void build_flux_ref(TablesHost& t) {
     for (int i = 0; i < np; ++i)
       for (int c = 0; c < nr; ++c)
         t.fr_Gt[((size_t)e * nr + c) * np + i] = t.fr_G[((size_t)e * np + i) * nr + c];
-  if (darcy) t.fr_hm.assign(H.begin(), H.end());
+  if (darcy || !orthonormal_basis(nq, t.Mqq, t.fo_P)) return;
+  t.fo_Pt.assign((size_t)nq * nq, 0.0);
+  for (int i = 0; i < nq; ++i)
+    for (int j = 0; j < nq; ++j) t.fo_Pt[(size_t)j * nq + i] = t.fo_P[(size_t)i * nq + j];
+  // B P over the columns of B, and P^T B over its rows
+  auto times_p = [&](const long double* b, int j) {
+    long double v = 0.0L;
+    for (int k = 0; k < nq; ++k) v += b[k] * t.fo_P[(size_t)k * nq + j];
+    return v;
+  };
+  std::vector<long double> Go = G;
+  for (size_t r = 0; r < (size_t)D * np; ++r)
+    for (int j = 0; j < nq; ++j) Go[r * nr + j] = times_p(&G[r * nr], j);
+  products(Go, H, t.fo_uu, t.fo_ub);
+  t.fo_G.assign(Go.begin(), Go.end());
+  t.fo_qm.assign((size_t)nq * nbs, 0.0);
+  std::vector<long double> row(nq), B((size_t)nq * nq);
+  for (int b = 0; b < nbs; ++b) {
+    for (int k = 0; k < nq; ++k) row[k] = t.fr_qm[(size_t)k * nbs + b];
+    for (int j = 0; j < nq; ++j) t.fo_qm[(size_t)j * nbs + b] = (double)times_p(row.data(), j);
+  }
+  t.fo_qq.assign((size_t)nF * nq * nq, 0.0);
+  for (int f = 0; f < nF; ++f) {
+    for (int i = 0; i < nq; ++i) {
+      for (int k = 0; k < nq; ++k) row[k] = t.Fqq[((size_t)f * nq + i) * nq + k];
+      for (int j = 0; j < nq; ++j) B[(size_t)j * nq + i] = times_p(row.data(), j);
+    }
+    for (int j = 0; j < nq; ++j)
+      for (int i = 0; i < nq; ++i)
+        t.fo_qq[((size_t)f * nq + i) * nq + j] = (double)times_p(&B[(size_t)j * nq], i);
+  }
 }
 
 }  // namespace hdg

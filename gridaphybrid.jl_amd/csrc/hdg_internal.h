@@ -66,6 +66,7 @@ struct TablesHost {
   int fb_nc = 0;
   int8_t fb_cid[36] = {};
   std::vector<double> fb_minv;
+  std::vector<long double> fb_minv_l;  // before rounding (host only, for the fr_* tables)
   // Transpose symmetry of the flux coupling (0: none): bit 0 set when
   // A_uq = s_u A_qu^T and A_bq = s_b A_qb^T entry by entry, bit 1: s_u = -1,
   // bit 2: s_b = -1.
@@ -82,6 +83,13 @@ struct TablesHost {
   std::vector<double> fr_hm;  // [D][np][nq + nbs] (Darcy)
   std::vector<double> fr_G;   // [D][np][nq + nbs]
   std::vector<double> fr_Gt;  // [D][nq + nbs][np]
+  // The same with the potential in an orthonormal basis of the reference cell
+  // (elasticity): nodal values u = fo_P u', columns orthonormal in the reference
+  // mass Mqq; empty when Mqq has no Cholesky factor.
+  std::vector<double> Mqq;    // [nq][nq]
+  std::vector<double> fo_P;   // [nq][nq], and its transpose
+  std::vector<double> fo_Pt;
+  std::vector<double> fo_uu, fo_ub, fo_qm, fo_qq, fo_G;  // fr_uu, fr_ub, fr_qm, Fqq, fr_G
 };
 
 // Device view of the tables (pointers into one device allocation).
@@ -129,6 +137,13 @@ struct Tables {
   const double* fr_hm;
   const double* fr_G;
   const double* fr_Gt;
+  const double* fo_P;     // null: none (the potential's own basis only)
+  const double* fo_Pt;
+  const double* fo_uu;
+  const double* fo_ub;
+  const double* fo_qm;
+  const double* fo_qq;
+  const double* fo_G;
 };
 
 // Device view of a mesh for the fused element generator.
@@ -297,6 +312,13 @@ int condense_grid_options(int fam, int* gm, int max);
 size_t condense_workspace_bytes(const SysShape& sh, int fam, int64_t ncells);
 hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                 hipStream_t st, Workspace& ws, int gridmul, bool ref);
+// The potential's orthonormal basis in place of its own (elasticity's family 8,
+// whose S, g and R_uu^-1 come from there).
+bool flux_orthonormal(const Tables& T);
+// out.U and out.Y of the cells' reduced systems in the potential's own basis,
+// where the condensation worked in the orthonormal one.
+hipError_t launch_flux_factors(const Tables& T, const MeshDev& M, const CondenseOut& out,
+                               hipStream_t st);
 // Recovery after a flux-block condensation (families 8 and 10): the structured
 // solve through R_uu^-1 and C^-1 (x) M^-1, refined in FP64 against the residual
 // of the full interior system (the reduced system is worse conditioned than

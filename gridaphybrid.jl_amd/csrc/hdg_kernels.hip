@@ -3784,6 +3784,32 @@ static hipError_t launch_flux_schur(const Tables& T, const MeshDev& M, const Con
 
 #include "recover_ref.h"
 
+bool flux_orthonormal(const Tables& T) { return T.phys == kElasticity && T.fo_P && sys_shape(T).flux; }
+
+// The class's tables with the potential in the orthonormal basis (fo_P set), or
+// in its own (fo_P null).
+static Tables orthonormal_tables(const Tables& T) {
+  Tables o = T;
+  o.fr_uu = T.fo_uu;
+  o.fr_ub = T.fo_ub;
+  o.fr_qm = T.fo_qm;
+  o.Fqq = T.fo_qq;
+  o.fr_G = T.fo_G;
+  return o;
+}
+
+hipError_t launch_flux_factors(const Tables& T, const MeshDev& M, const CondenseOut& out,
+                               hipStream_t st) {
+  if (!flux_orthonormal(T) || !out.U || !out.Y || out.u_stride < (int64_t)factor_slot(sys_shape(T)) ||
+      out.y_stride < (int64_t)(T.nb + 1) * (T.ni - T.na))
+    return hipErrorInvalidValue;
+  if (M.ncells <= 0) return hipSuccess;
+  Tables own = T;
+  own.fo_P = nullptr;
+  return T.D == 2 ? launch_tile_ref<kElasticity, 2>(own, M, out, st, 0)
+                  : launch_tile_ref<kElasticity, 3>(own, M, out, st, 0);
+}
+
 hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                 hipStream_t st, Workspace& ws, int gridmul, bool ref) {
   const SysShape sh = sys_shape(T);
@@ -3799,6 +3825,12 @@ hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const Condens
   CondenseOut o = out;
   if (out.keep_uu) o.Auu = out.U + fs.auu;
   o.Rinv = out.U + fs.ri;
+  if (flux_orthonormal(T)) {  // (U: launch_flux_factors)
+    o.U = nullptr;
+    const Tables To = orthonormal_tables(T);
+    return T.D == 2 ? launch_tile_ref<kElasticity, 2>(To, M, o, st, gridmul)
+                    : launch_tile_ref<kElasticity, 3>(To, M, o, st, gridmul);
+  }
   if (T.phys == kDarcy)
     return T.D == 2 ? launch_tile_ref<kDarcy, 2>(T, M, o, st, gridmul)
                     : launch_tile_ref<kDarcy, 3>(T, M, o, st, gridmul);
@@ -4079,7 +4111,18 @@ __global__ void __launch_bounds__(256)
     }
     wave_sync_lds();
 #pragma unroll
-    for (int t = 0; t < KU; ++t) cu[t] = lane + 64 * t < nu ? uv[lane + 64 * t] : 0.0;
+    for (int t = 0; t < KU; ++t) {
+      const int r = lane + 64 * t;
+      cu[t] = r < nu ? uv[r] : 0.0;
+      if (PHYS != kDarcy && T.fo_P && r < nu) {  // P^T c_u: the steps are in that basis
+        const int d = r / nq;
+        const double* const pc = T.fo_P + (r - d * nq);
+        double x = 0.0;
+#pragma unroll 4
+        for (int j = 0; j < nq; ++j) x = fma(pc[j * nq], uv[d * nq + j], x);
+        cu[t] = x;
+      }
+    }
     // ---- the structured solve of c, then of the residuals of the full interior system
 #pragma unroll 1
     for (int it = 0; it <= kFluxRefineSteps; ++it) {
@@ -4217,7 +4260,17 @@ __global__ void __launch_bounds__(256)
       const int r = lane + 64 * t;
       if (r < na) out[cell * na + r] = xq[r];
     }
-    for (int r = lane; r < nu; r += 64) out[ncells * na + cell * nu + r] = xuv[r];
+    for (int r = lane; r < nu; r += 64) {
+      double x = xuv[r];
+      if (PHYS != kDarcy && T.fo_P) {  // x_u = P x_u'
+        const int d = r / nq;
+        const double* const pr = T.fo_Pt + (r - d * nq);
+        x = 0.0;
+#pragma unroll 4
+        for (int j = 0; j < nq; ++j) x = fma(pr[j * nq], xuv[d * nq + j], x);
+      }
+      out[ncells * na + cell * nu + r] = x;
+    }
     wave_sync_lds();
   }
 }
@@ -4257,10 +4310,11 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
     const bool g_lds = ref && base + gbytes <= 64 * 1024;
     const size_t lds = base + (g_lds ? gbytes : 0);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
+    const Tables Tr = flux_orthonormal(T) ? orthonormal_tables(T) : T;
     ClockScope clk_(st, "recover_flux");
 #define HDG_RF(P_, K_, U_, R_)                                                                  \
   hipLaunchKernelGGL((recover_flux_kernel<P_, K_, U_, R_>), dim3(grid), dim3(64 * kRecWaves),   \
-                     lds, st, FusedGen<P_>{T, M}, rs, cell_dofs, lam_free, lam_dir, out, g_lds)
+                     lds, st, FusedGen<P_>{Tr, M}, rs, cell_dofs, lam_free, lam_dir, out, g_lds)
     if (T.phys == kDarcy) {
       if (ref) {
         // (one row tile, or 2D: at most 98 + 64 rows)

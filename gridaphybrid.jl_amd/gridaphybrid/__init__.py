@@ -448,7 +448,8 @@ class HybridAffineFEOperator:
         """(U, Y) host copies: U (ncells, m, m) upper factor in LAPACK row order,
         Y (ncells, m, nb+1) = L^-1 P [B b] of the system the recovery
         back-substitutes: A_ii (m = ni) for the elimination families, the
-        reduced system after the flux block (m = ni - n_flux) for flux_schur."""
+        reduced system after the flux block (m = ni - n_flux) for flux_schur and
+        flux_ref."""
         U, Y = C.c_void_p(), C.c_void_p()
         check(lib().hdg_local_factors(self.mesh, C.byref(U), C.byref(Y)), self.ctx.h, "factors")
         nc, nb = self.info.ncells, self.info.nb

@@ -342,11 +342,15 @@ int hdg_cell_blocks(hdg_mesh* mesh, const double** S, const double** g,
  * Y [ncells][nb+1][ni] = L^-1 P [A_ib b_i] in LAPACK row order.  The pivot
  * sequence is getrf's (largest magnitude, first position on ties).  After a
  * mixed-precision condensation *U is NULL and Y holds W = A_ii^-1 [A_ib b_i]
- * in natural interior order.  After a flux-block condensation (family 8) U
- * and Y are the factors of the reduced system of the m = ni - n_flux
- * non-flux interior unknowns, at the start of each cell's slot (the rest of
- * the slot holds the recovery's kept blocks and the inverse of the reduced
- * interior block; not part of this interface).  Cell c's slots start at c * u_stride and c * y_stride
+ * in natural interior order.  After a flux-block condensation (families 8 and
+ * 10, the defaults of the larger classes: query hdg_mesh_factor_layout) U and Y
+ * are the factors of the reduced system of the m = ni - n_flux non-flux interior
+ * unknowns, at the start of each cell's slot (the rest of the slot holds the
+ * recovery's kept blocks and the inverse of the reduced interior block; not part
+ * of this interface).  Elasticity's family 8 works in another basis of the
+ * displacement and forms U and Y when this is called; from then on every
+ * condensation of the mesh forms them too, so the pointers' contents stay
+ * current.  Cell c's slots start at c * u_stride and c * y_stride
  * (hdg_mesh_factor_layout). */
 int hdg_local_factors(hdg_mesh* mesh, const double** U, const double** Y);
 /* Layout of the resident factors: rows m of the factored system (ni, or
