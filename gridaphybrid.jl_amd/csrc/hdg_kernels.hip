@@ -2548,7 +2548,9 @@ __global__ void __launch_bounds__(256) cell_rhs_kernel(Tables T, MeshDev M) {
       dbl4 acc[kRhsTiles];
 #pragma unroll
       for (int j = 0; j < kRhsTiles; ++j) acc[j] = zero;
-      for (int p0 = 0; p0 < nqc; p0 += kRhsPoints) {
+      // (elasticity's flux rows have no load: a pass of theirs stores zeros)
+      const int np_end = PHYS == kDarcy || t0 < nu ? nqc : 0;
+      for (int p0 = 0; p0 < np_end; p0 += kRhsPoints) {
         const int pn = min(kRhsPoints, nqc - p0), pn4 = (pn + 3) & ~3;
         bool flux = false;
         for (int p = tid >> 4; p < pn4; p += 16) {
