@@ -3922,6 +3922,14 @@ __device__ inline double flux_cinv_entry(const double* alpha, int D, int a, int 
   return a == b ? 1.0 / ks : 0.0;
 }
 
+// A column (stride ld) of P or its transpose times v.
+__device__ inline double p_column(const double* p, int ld, const double* v, int n) {
+  double x = 0.0;
+#pragma unroll 4
+  for (int j = 0; j < n; ++j) x = fma(p[j * ld], v[j], x);
+  return x;
+}
+
 // REF (the reference decomposition): A_qu and A_uq are not read from the slot
 // but applied from the reference matrices G_e (potential columns) and the
 // cell's cofactors c_ea,
@@ -3929,13 +3937,13 @@ __device__ inline double flux_cinv_entry(const double* alpha, int D, int a, int 
 //   elasticity: (A_qu v)[(s, i)] = sum over the components d of s = (p, q) of
 //               sum_e c_e,partner t_de[i],  t_de = G_e v_d;
 // and A_uq = -A_qu^T; A_uu is kept for one potential component.  G_e is staged
-// in LDS once per workgroup (g_lds), or, where it does not fit (2D Darcy k=6),
+// in LDS once per workgroup (g_lds; p_lds: the orthonormal basis as well), or, where it does not fit (2D Darcy k=6),
 // read from the table, which every cell shares (L2-resident).
 template <int PHYS, int KQ, int KU, bool REF>
 __global__ void __launch_bounds__(256)
     recover_flux_kernel(FusedGen<PHYS> gen, RecSlot rs, const int32_t* __restrict__ cell_dofs,
                         const double* __restrict__ lam_free, const double* __restrict__ lam_dir,
-                        double* __restrict__ out, bool g_lds) {
+                        double* __restrict__ out, bool g_lds, bool p_lds) {
   constexpr int WPB = kRecWaves;
   // M^-1 and M transposed ([col][row]: lane i reads row i at stride 1, free of
   // bank conflicts for any np), (REF with g_lds: G_e [D][np][nq]), then the
@@ -3952,7 +3960,10 @@ __global__ void __launch_bounds__(256)
   // G_e[i][c] at gsrc[(e * np + i) * gld + c]
   const double* gsrc = g_lds ? s_gu : T.fr_G;
   const int gld = g_lds ? nq : nq + T.nF * T.nm;
-  double* alpha = s_m + 2 * np * np + gsz + (int64_t)w * rec_wave_lds(na, nu, nb, REF ? ng : 0);
+  const bool orth = REF && PHYS != kDarcy && T.fo_P;  // the steps are in that basis
+  const int psz = orth && p_lds ? nq * nq : 0;
+  double* const s_p = s_gu + gsz;  // p_lds: fo_P [j][i]
+  double* alpha = s_m + 2 * np * np + gsz + psz + (int64_t)w * rec_wave_lds(na, nu, nb, REF ? ng : 0);
   double* c6 = alpha + kMaxAlpha;  // C, then C^-1 [2][36]
   double* lam = c6 + 72;           // [nb]
   double* xq = lam + nb;           // x_q [na]
@@ -3973,6 +3984,7 @@ __global__ void __launch_bounds__(256)
       const int k = t / nq, c = t - k * nq;
       s_gu[t] = T.fr_G[(size_t)k * (nq + T.nF * T.nm) + c];
     }
+  for (int t = threadIdx.x; t < psz; t += 64 * WPB) s_p[t] = T.fo_P[t];
   __syncthreads();
   const double* Minv = s_m;
   const double* Mm = s_m + np * np;
@@ -4116,13 +4128,10 @@ __global__ void __launch_bounds__(256)
     for (int t = 0; t < KU; ++t) {
       const int r = lane + 64 * t;
       cu[t] = r < nu ? uv[r] : 0.0;
-      if (PHYS != kDarcy && T.fo_P && r < nu) {  // P^T c_u: the steps are in that basis
+      if (orth && r < nu) {  // P^T c_u
         const int d = r / nq;
-        const double* const pc = T.fo_P + (r - d * nq);
-        double x = 0.0;
-#pragma unroll 4
-        for (int j = 0; j < nq; ++j) x = fma(pc[j * nq], uv[d * nq + j], x);
-        cu[t] = x;
+        cu[t] = psz ? p_column(s_p + (r - d * nq), nq, uv + d * nq, nq)
+                    : p_column(T.fo_P + (r - d * nq), nq, uv + d * nq, nq);
       }
     }
     // ---- the structured solve of c, then of the residuals of the full interior system
@@ -4264,12 +4273,10 @@ __global__ void __launch_bounds__(256)
     }
     for (int r = lane; r < nu; r += 64) {
       double x = xuv[r];
-      if (PHYS != kDarcy && T.fo_P) {  // x_u = P x_u'
+      if (orth) {  // x_u = P x_u'
         const int d = r / nq;
-        const double* const pr = T.fo_Pt + (r - d * nq);
-        x = 0.0;
-#pragma unroll 4
-        for (int j = 0; j < nq; ++j) x = fma(pr[j * nq], xuv[d * nq + j], x);
+        x = psz ? p_column(s_p + (r - d * nq) * nq, 1, xuv + d * nq, nq)
+                : p_column(T.fo_Pt + (r - d * nq), nq, xuv + d * nq, nq);
       }
       out[ncells * na + cell * nu + r] = x;
     }
@@ -4310,13 +4317,16 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
     const size_t gbytes = (size_t)T.D * T.np * T.nq * sizeof(double);
     // G_e in LDS while two workgroups still fit a CU
     const bool g_lds = ref && base + gbytes <= 64 * 1024;
-    const size_t lds = base + (g_lds ? gbytes : 0);
+    const size_t pbytes = flux_orthonormal(T) ? (size_t)T.nq * T.nq * sizeof(double) : 0;
+    const bool p_lds = g_lds && base + gbytes + pbytes <= 64 * 1024;
+    const size_t lds = base + (g_lds ? gbytes : 0) + (p_lds ? pbytes : 0);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     const Tables Tr = flux_orthonormal(T) ? orthonormal_tables(T) : T;
     ClockScope clk_(st, "recover_flux");
 #define HDG_RF(P_, K_, U_, R_)                                                                  \
   hipLaunchKernelGGL((recover_flux_kernel<P_, K_, U_, R_>), dim3(grid), dim3(64 * kRecWaves),   \
-                     lds, st, FusedGen<P_>{Tr, M}, rs, cell_dofs, lam_free, lam_dir, out, g_lds)
+                     lds, st, FusedGen<P_>{Tr, M}, rs, cell_dofs, lam_free, lam_dir, out, g_lds,  \
+                     p_lds)
     if (T.phys == kDarcy) {
       if (ref) {
         // (one row tile, or 2D: at most 98 + 64 rows)
