@@ -148,19 +148,8 @@ struct RefGen {
     const double* al = M.alpha + cell * kMaxAlpha;
     const double* b = M.srcq + cell * srcq_stride(T);
     for (int t = tid; t < kMaxAlpha; t += nthreads) sh.alpha[t] = al[t];
-    if (PHYS != kDarcy && T.fo_P) {  // P^T b_u, a component after the other
-      const int nq = T.nq;
-      for (int t = tid; t < nr; t += nthreads) {
-        const int c = (sh.idx[t] & 0xffff) * 8, d = sh.idx[t] >> 16;
-        double x = 0.0;
-        if (t < nu)
-#pragma unroll 8
-          for (int j = 0; j < nq; ++j) x = fma(table_at(T.fo_P + j * nq, c), b[na + d * nq + j], x);
-        sh.rhs[t] = x;
-      }
-    } else {
-      for (int t = tid; t < nr; t += nthreads) sh.rhs[t] = t < nu ? b[na + t] : 0.0;
-    }
+    const double* bu = b + (T.fo_P ? T.ni : na);  // in the basis of the tables
+    for (int t = tid; t < nr; t += nthreads) sh.rhs[t] = t < nu ? bu[t] : 0.0;
     int load = 0;  // the flux equation's load (none: its terms are skipped)
     if (PHYS == kDarcy)
       for (int t = tid; t < na; t += nthreads) load |= b[t] != 0.0;

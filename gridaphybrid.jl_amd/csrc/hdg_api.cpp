@@ -119,8 +119,8 @@ struct hdg_mesh {
   // its grid; the family of the last condensation decides the recovery
   int family = -1, gridmul = 0;
   int used_family = -1;
-  // (family 8, elasticity) U and Y have been asked for: every condensation forms
-  // them, in the potential's own basis
+  // (family 10 and elasticity's 8) U and Y have been asked for: every condensation
+  // forms them, in the potential's own basis
   bool want_factors = false;
   bool rec_group = false;  // (family 10) the recovery's kernel, by which the condensation kept A_uu
   DevBuf d_fptr, d_pptr, d_pfacet, d_pcell, d_plpos, d_gcell, d_glpos;
@@ -183,7 +183,7 @@ struct CellLayout {
         U(factor_slot(sys_shape(t))),
         Y((size_t)(t.nb + 1) * t.ni),
         alpha(72),
-        srcq((size_t)t.ni) {}  // interior right-hand side b_i
+        srcq((size_t)t.ni + (t.fo_P.empty() ? 0 : t.ni - t.na)) {}  // b_i, P^T b_u
 };
 
 // After a condensation by `family`, the mesh recovers 16 cells a workgroup.
@@ -219,7 +219,9 @@ hipError_t own_cell_state(hdg_mesh* m) {
 // U and Y of the last condensation where it left them out (launch_flux_factors);
 // the other families write them themselves.
 int form_factors(hdg_mesh* m) {
-  if (m->mixed || m->used_family != kFamilyFluxSchur || !flux_orthonormal(m->tdev)) return HDG_OK;
+  const bool ref = m->used_family == kFamilyFluxRef;
+  if (m->mixed || !(ref || m->used_family == kFamilyFluxSchur) || !flux_principal(m->tdev, ref))
+    return HDG_OK;
   hdg_ctx* ctx = m->ctx;
   PoolScope pool_(ctx->pool);
   HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
@@ -770,7 +772,7 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
                                                    &th.fr_bb, &th.fr_qm, &th.fr_mm, &th.fr_hm,
                                                    &th.fr_G, &th.fr_Gt, &th.fo_P, &th.fo_Pt,
                                                    &th.fo_uu, &th.fo_ub, &th.fo_qm, &th.fo_qq,
-                                                   &th.fo_G};
+                                                   &th.fo_hm, &th.fo_G, &th.fo_Gt, &th.fo_Bq};
     size_t nd = 0;
     for (auto* v : dv) nd += v->size();
     size_t bytes = nd * sizeof(double) + th.prog_val.size() * sizeof(double) +
@@ -856,7 +858,7 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
                              &T.Fmm, &T.Bp,  &T.Bq,  &T.xq,  &T.fb_minv, &T.fr_uu, &T.fr_ub,
                              &T.fr_bb, &T.fr_qm, &T.fr_mm, &T.fr_hm, &T.fr_G, &T.fr_Gt,
                              &T.fo_P, &T.fo_Pt, &T.fo_uu, &T.fo_ub, &T.fo_qm, &T.fo_qq,
-                             &T.fo_G};
+                             &T.fo_hm, &T.fo_G, &T.fo_Gt, &T.fo_Bq};
     for (size_t i = 0; i < dv.size(); ++i) *ptrs[i] = reinterpret_cast<const double*>(base + offs[i]);
     T.pmask = reinterpret_cast<const uint8_t*>(base + off_pm);
     T.qmask = reinterpret_cast<const uint8_t*>(base + off_qm);
@@ -878,6 +880,7 @@ int hdg_mesh_create(hdg_ctx* ctx, const hdg_problem* prob, const hdg_mesh_desc* 
     std::memcpy(T.fb_cid, th.fb_cid, sizeof(T.fb_cid));
     if (th.fb_minv.empty()) T.fb_minv = nullptr;
     if (th.fo_P.empty()) T.fo_P = nullptr;
+    T.nbo = th.fo_P.empty() ? 0 : th.ni - th.na;
     T.fr_npair = th.fr_npair;
   }
   m->x0.assign(desc->x0, desc->x0 + nc * D);

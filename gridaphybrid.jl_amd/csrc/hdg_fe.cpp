@@ -871,21 +871,29 @@ void detect_flux_sym(TablesHost& t) {
 //   fr_hm  (Darcy) H_e = M^-1 G_e [e][i][column], for a flux right-hand side;
 //   fr_G   G_e, [e][i][column]; fr_Gt  the same as [e][column][i].
 //
-// Elasticity has them twice.  The nodal basis of P_(k+1) on the cube (nodes on a
-// simplex, extrapolated) makes R_uu worse conditioned than the problem is: 1.9e8
-// for 3D k=3, where with the potential in a basis orthonormal in the reference
-// mass it is 27.  S and g do not depend on that basis, their rounding does: S of
-// 3D k=3 was 7.0e-12 of its largest entry off with R in the nodal basis, 1.6e-12
-// after a dense elimination of all 225 rows, and is 6.5e-13 off with the
-// orthonormal one; of k=2 2.0e-13, 4.9e-14 and 2.1e-14 (against extended
-// precision; what is left is the rounding of the nodal tables).  fo_*: the tables
-// of that basis, u = fo_P u'; any fo_P is exact, the tables being formed from its
-// rounded entries.  Darcy's R_uu gains nothing (2D k=3: condition 2e5 and 2e4, S
-// 1.8e-15 and 1.6e-15).
-// P with P^T M P = I up to rounding (the transposed inverse of M's Cholesky
-// factor); false if M is not positive definite.
-static bool orthonormal_basis(int n, const std::vector<double>& M, std::vector<double>& P) {
-  std::vector<long double> C((size_t)n * n, 0.0L), X((size_t)n * n, 0.0L);
+// And once more with the potential in a principal basis u = fo_P u' (fo_*):
+// orthonormal in the reference mass and diagonal in sum_e G_e^T M^-1 G_e, which
+// leaves the functions that no flux sees (Darcy Q_k: one; elasticity P_(k+1):
+// those orthogonal to P_(k-1)) as its last ones, with zero columns of G.  S and g
+// do not depend on the basis; their rounding, and R_uu^-1, do:
+//  - R_uu has entries of the order of the coefficient (kappa, E) on the functions
+//    a flux sees, and the stabilisation alone on the others.  In the nodal basis
+//    the two mix, and from kappa = 1e5 on (2D k=3, 20^2 cells; with h = 1/211 from
+//    1e4) the recovery through R_uu^-1 lost its values altogether (errors of order
+//    1 at 1e6).  Here they are entries of their own: 9e-9 at 1e6, 2e-7 at 1e8,
+//    which LAPACK's solve of A_ii has too (1e-8, 8e-7).
+//  - the nodal basis of P_(k+1) on the cube (nodes on a simplex, extrapolated)
+//    gives elasticity's R_uu a condition of 1.9e8 for 3D k=3, here 27: S was
+//    7.0e-12 of its largest entry off, 1.6e-12 after a dense elimination of all
+//    225 rows, and is 8.0e-13 off; k=2 2.0e-13, 4.9e-14 and 2.9e-14; Darcy 2D
+//    k=3, 211 x 77 cells, 4.7e-15, 1.1e-15 and 2.6e-15 (against extended
+//    precision; what is left is the rounding of the nodal tables).
+// Any fo_P is exact, the tables being formed from its rounded entries.
+// P with P^T M P = I and P^T K P diagonal, descending (Cholesky of M, cyclic
+// Jacobi on C^-1 K C^-T); false if M is not positive definite.
+static bool principal_basis(int n, const std::vector<double>& M, const std::vector<long double>& K,
+                            std::vector<double>& P) {
+  std::vector<long double> C((size_t)n * n, 0.0L), A = K, V((size_t)n * n, 0.0L);
   for (int j = 0; j < n; ++j) {
     long double d = M[(size_t)j * n + j];
     for (int k = 0; k < j; ++k) d -= C[(size_t)j * n + k] * C[(size_t)j * n + k];
@@ -898,21 +906,69 @@ static bool orthonormal_basis(int n, const std::vector<double>& M, std::vector<d
       C[(size_t)i * n + j] = v / C[(size_t)j * n + j];
     }
   }
+  // A = C^-1 K C^-T: rows, then columns
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int c = 0; c < n; ++c)
+      for (int i = 0; i < n; ++i) {
+        long double v = A[(size_t)i * n + c];
+        for (int k = 0; k < i; ++k) v -= C[(size_t)i * n + k] * A[(size_t)k * n + c];
+        A[(size_t)i * n + c] = v / C[(size_t)i * n + i];
+      }
+    for (int i = 0; i < n; ++i)
+      for (int j = 0; j < i; ++j) std::swap(A[(size_t)i * n + j], A[(size_t)j * n + i]);
+  }
+  for (int i = 0; i < n; ++i) V[(size_t)i * n + i] = 1.0L;
+  for (int sweep = 0; sweep < 30; ++sweep) {
+    long double off = 0.0L, dia = 0.0L;
+    for (int i = 0; i < n; ++i)
+      for (int j = 0; j < n; ++j)
+        (i == j ? dia : off) += A[(size_t)i * n + j] * A[(size_t)i * n + j];
+    if (off <= 1e-38L * dia) break;  // (V: eigenvectors in rows)
+    for (int p = 0; p < n; ++p)
+      for (int q = p + 1; q < n; ++q) {
+        const long double apq = A[(size_t)p * n + q];
+        if (apq * apq <= 1e-42L * dia) continue;
+        const long double th = (A[(size_t)q * n + q] - A[(size_t)p * n + p]) / (2.0L * apq);
+        const long double t =
+            (th >= 0.0L ? 1.0L : -1.0L) / (std::fabs(th) + std::sqrt(th * th + 1.0L));
+        const long double c = 1.0L / std::sqrt(t * t + 1.0L), sn = t * c;
+        for (int k = 0; k < n; ++k) {
+          const long double u = V[(size_t)p * n + k], w = V[(size_t)q * n + k];
+          V[(size_t)p * n + k] = c * u - sn * w;
+          V[(size_t)q * n + k] = sn * u + c * w;
+          if (k == p || k == q) continue;
+          const long double x = A[(size_t)p * n + k], y = A[(size_t)q * n + k];
+          A[(size_t)k * n + p] = A[(size_t)p * n + k] = c * x - sn * y;
+          A[(size_t)k * n + q] = A[(size_t)q * n + k] = sn * x + c * y;
+        }
+        A[(size_t)p * n + p] -= t * apq;
+        A[(size_t)q * n + q] += t * apq;
+        A[(size_t)p * n + q] = A[(size_t)q * n + p] = 0.0L;
+      }
+  }
+  std::vector<int> at(n);
+  for (int j = 0; j < n; ++j) at[j] = j;
+  std::sort(at.begin(), at.end(), [&](int i, int j) {
+    return A[(size_t)i * n + i] > A[(size_t)j * n + j];
+  });
   P.assign((size_t)n * n, 0.0);
-  for (int c = 0; c < n; ++c)  // X = C^-1 by columns, P = X^T
-    for (int i = c; i < n; ++i) {
-      long double v = i == c ? 1.0L : 0.0L;
-      for (int k = c; k < i; ++k) v -= C[(size_t)i * n + k] * X[(size_t)k * n + c];
-      X[(size_t)i * n + c] = v / C[(size_t)i * n + i];
-      P[(size_t)c * n + i] = (double)X[(size_t)i * n + c];
+  std::vector<long double> x(n);
+  for (int j = 0; j < n; ++j) {  // C^T x = v
+    for (int i = n - 1; i >= 0; --i) {
+      long double v = V[(size_t)at[j] * n + i];
+      for (int k = i + 1; k < n; ++k) v -= C[(size_t)k * n + i] * x[k];
+      x[i] = v / C[(size_t)i * n + i];
     }
+    for (int i = 0; i < n; ++i) P[(size_t)i * n + j] = (double)x[i];
+  }
   return true;
 }
 
 void build_flux_ref(TablesHost& t) {
   t.fr_npair = 0;
   for (auto* v : {&t.fr_uu, &t.fr_ub, &t.fr_bb, &t.fr_qm, &t.fr_mm, &t.fr_hm, &t.fr_G,
-                  &t.fr_Gt, &t.fo_P, &t.fo_Pt, &t.fo_uu, &t.fo_ub, &t.fo_qm, &t.fo_qq, &t.fo_G})
+                  &t.fr_Gt, &t.fo_P, &t.fo_Pt, &t.fo_uu, &t.fo_ub, &t.fo_qm, &t.fo_qq, &t.fo_hm, &t.fo_G,
+                  &t.fo_Gt, &t.fo_Bq})
     v->clear();
   const int D = t.D, np = t.np, nq = t.nq, nm = t.nm, nF = t.nF, nbs = nF * nm;
   const bool darcy = t.phys == kDarcy;
@@ -960,10 +1016,19 @@ void build_flux_ref(TablesHost& t) {
           for (int c = 0; c < nr; ++c)
             H[((size_t)e * np + i) * nr + c] += m * G[((size_t)e * np + k) * nr + c];
         }
-    auto dot = [&](int e, int r, int e2, int c) {
-      long double v = 0.0L;
+    std::vector<long double> Gc(G.size()), Hc(G.size());  // by columns
+    for (int e = 0; e < D; ++e)
       for (int i = 0; i < np; ++i)
-        v += G[((size_t)e * np + i) * nr + r] * H[((size_t)e2 * np + i) * nr + c];
+        for (int c = 0; c < nr; ++c) {
+          const size_t from = ((size_t)e * np + i) * nr + c, to = ((size_t)e * nr + c) * np + i;
+          Gc[to] = G[from];
+          Hc[to] = H[from];
+        }
+    auto dot = [&](int e, int r, int e2, int c) {
+      const long double* const x = &Gc[((size_t)e * nr + r) * np];
+      const long double* const y = &Hc[((size_t)e2 * nr + c) * np];
+      long double v = 0.0L;
+      for (int i = 0; i < np; ++i) v += x[i] * y[i];
       return v;
     };
     uu.assign((size_t)t.fr_npair * nq * nq, 0.0);
@@ -1004,7 +1069,12 @@ void build_flux_ref(TablesHost& t) {
     for (int i = 0; i < np; ++i)
       for (int c = 0; c < nr; ++c)
         t.fr_Gt[((size_t)e * nr + c) * np + i] = t.fr_G[((size_t)e * np + i) * nr + c];
-  if (darcy || !orthonormal_basis(nq, t.Mqq, t.fo_P)) return;
+  // K = sum_e G_e^T M^-1 G_e
+  std::vector<long double> K((size_t)nq * nq, 0.0L);
+  for (size_t r = 0; r < (size_t)D * np; ++r)
+    for (int i = 0; i < nq; ++i)
+      for (int j = 0; j < nq; ++j) K[(size_t)i * nq + j] += G[r * nr + i] * H[r * nr + j];
+  if (!principal_basis(nq, t.Mqq, K, t.fo_P)) return;
   t.fo_Pt.assign((size_t)nq * nq, 0.0);
   for (int i = 0; i < nq; ++i)
     for (int j = 0; j < nq; ++j) t.fo_Pt[(size_t)j * nq + i] = t.fo_P[(size_t)i * nq + j];
@@ -1014,11 +1084,33 @@ void build_flux_ref(TablesHost& t) {
     for (int k = 0; k < nq; ++k) v += b[k] * t.fo_P[(size_t)k * nq + j];
     return v;
   };
+  std::vector<long double> bq(nq);
+  t.fo_Bq.assign(t.Bq.size(), 0.0);
+  for (size_t q = 0; q < (size_t)t.nqc; ++q) {
+    for (int k = 0; k < nq; ++k) bq[k] = t.Bq[q * nq + k];
+    for (int j = 0; j < nq; ++j) t.fo_Bq[q * nq + j] = (double)times_p(bq.data(), j);
+  }
   std::vector<long double> Go = G;
   for (size_t r = 0; r < (size_t)D * np; ++r)
     for (int j = 0; j < nq; ++j) Go[r * nr + j] = times_p(&G[r * nr], j);
+  // the functions no flux sees: their columns are zero but for rounding
+  long double top = 0.0L;
+  for (int j = 0; j < nq; ++j)
+    for (size_t r = 0; r < (size_t)D * np; ++r) top = std::max(top, std::fabs(Go[r * nr + j]));
+  for (int j = 0; j < nq; ++j) {
+    long double own = 0.0L;
+    for (size_t r = 0; r < (size_t)D * np; ++r) own = std::max(own, std::fabs(Go[r * nr + j]));
+    if (own < 1e-11L * top)
+      for (size_t r = 0; r < (size_t)D * np; ++r) Go[r * nr + j] = 0.0L;
+  }
   products(Go, H, t.fo_uu, t.fo_ub);
+  if (darcy) t.fo_hm.assign(H.begin(), H.end());
   t.fo_G.assign(Go.begin(), Go.end());
+  t.fo_Gt.assign(Go.size(), 0.0);
+  for (int e = 0; e < D; ++e)
+    for (int i = 0; i < np; ++i)
+      for (int c = 0; c < nr; ++c)
+        t.fo_Gt[((size_t)e * nr + c) * np + i] = t.fo_G[((size_t)e * np + i) * nr + c];
   t.fo_qm.assign((size_t)nq * nbs, 0.0);
   std::vector<long double> row(nq), B((size_t)nq * nq);
   for (int b = 0; b < nbs; ++b) {

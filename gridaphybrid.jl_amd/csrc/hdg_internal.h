@@ -83,13 +83,14 @@ struct TablesHost {
   std::vector<double> fr_hm;  // [D][np][nq + nbs] (Darcy)
   std::vector<double> fr_G;   // [D][np][nq + nbs]
   std::vector<double> fr_Gt;  // [D][nq + nbs][np]
-  // The same with the potential in an orthonormal basis of the reference cell
-  // (elasticity): nodal values u = fo_P u', columns orthonormal in the reference
-  // mass Mqq; empty when Mqq has no Cholesky factor.
+  // The same with the potential in the principal basis of the reference cell,
+  // nodal values u = fo_P u'; empty when Mqq has no Cholesky factor.
   std::vector<double> Mqq;    // [nq][nq]
   std::vector<double> fo_P;   // [nq][nq], and its transpose
   std::vector<double> fo_Pt;
-  std::vector<double> fo_uu, fo_ub, fo_qm, fo_qq, fo_G;  // fr_uu, fr_ub, fr_qm, Fqq, fr_G
+  // (fr_uu, fr_ub, fr_qm, Fqq, fr_hm, fr_G, fr_Gt there)
+  std::vector<double> fo_uu, fo_ub, fo_qm, fo_qq, fo_hm, fo_G, fo_Gt;
+  std::vector<double> fo_Bq;  // Bq fo_P [nqc][nq]
 };
 
 // Device view of the tables (pointers into one device allocation).
@@ -143,7 +144,11 @@ struct Tables {
   const double* fo_ub;
   const double* fo_qm;
   const double* fo_qq;
+  const double* fo_hm;
   const double* fo_G;
+  const double* fo_Gt;
+  const double* fo_Bq;
+  int nbo;  // potential rows of the right-hand side in that basis, behind b_i
 };
 
 // Device view of a mesh for the fused element generator.
@@ -155,7 +160,7 @@ struct MeshDev {
   const double* coef;      // [ncells] kappa or nu
   const double* src;       // [ncells][nqc][ncomp] or null (user source values)
   double* alpha;           // [ncells][72] per-cell entry-program coefficients (scratch)
-  double* srcq;            // [ncells][ni] interior right-hand side b_i (scratch)
+  double* srcq;            // [ncells][ni + nbo] interior right-hand side b_i, P^T b_u (scratch)
   int source;              // hdg_source
   double tau;
   double young;
@@ -312,11 +317,11 @@ int condense_grid_options(int fam, int* gm, int max);
 size_t condense_workspace_bytes(const SysShape& sh, int fam, int64_t ncells);
 hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                 hipStream_t st, Workspace& ws, int gridmul, bool ref);
-// The potential's orthonormal basis in place of its own (elasticity's family 8,
-// whose S, g and R_uu^-1 come from there).
-bool flux_orthonormal(const Tables& T);
+// The potential's principal basis in place of its own: family 10 and elasticity's
+// family 8, whose S, g and R_uu^-1 come from there.
+bool flux_principal(const Tables& T, bool ref);
 // out.U and out.Y of the cells' reduced systems in the potential's own basis,
-// where the condensation worked in the orthonormal one.
+// where the condensation worked in the principal one.
 hipError_t launch_flux_factors(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                hipStream_t st);
 // Recovery after a flux-block condensation (families 8 and 10): the structured

@@ -186,9 +186,10 @@ constexpr int kMaxAlpha = 72;
 // build_program in hdg_fe.cpp).  One thread per cell computes its
 // coefficients into LDS; the wavefront then stores its 64 cells' rows as one
 // contiguous, coalesced range.
-// Per-cell stride of the right-hand-side scratch: the interior b_i [ni].
+// Per-cell stride of the right-hand-side scratch: the interior b_i [ni], and its
+// potential rows in the principal basis [nbo].
 __device__ __host__ inline int64_t srcq_stride(const Tables& T) {
-  return (int64_t)T.ni;
+  return (int64_t)T.ni + T.nbo;
 }
 
 constexpr int kPrepCells = 64;  // cells (threads) per prep workgroup
@@ -2527,7 +2528,7 @@ bool condense_supported(int n) {
 // lane per row: 64^3 k=2 1,550 -> 384 us, 512^2 k=2 354 -> 105, 24^3 k=3 229 ->
 // 74, elasticity of 5,814 cells k=2 54 -> 28; 1,728 cells k=3 57 -> 74.)
 constexpr int kRhsPoints = 32;
-constexpr int kRhsTiles = 4;  // output tiles of a wavefront in one pass over the points
+constexpr int kRhsTiles = 5;  // output tiles of a wavefront in one pass over the points
 
 template <int PHYS, int D>
 __global__ void __launch_bounds__(256) cell_rhs_kernel(Tables T, MeshDev M) {
@@ -2536,10 +2537,11 @@ __global__ void __launch_bounds__(256) cell_rhs_kernel(Tables T, MeshDev M) {
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int i16 = lane & 15, q4 = lane >> 4;
   const int np = T.np, nq = T.nq, na = T.na, nqc = T.nqc;
-  // output tiles: the potential components, then the flux components (elasticity: 0)
+  // output tiles: the potential components, the same in the principal basis
+  // (nbo), then the flux components (elasticity: 0)
   const int tq = (nq + 15) >> 4, tp = (np + 15) >> 4;
   constexpr int NC = PHYS == kDarcy ? D : D * (D + 1) / 2;
-  const int nu = (PHYS == kDarcy ? 1 : D) * tq, nt = nu + NC * tp;
+  const int n1 = (PHYS == kDarcy ? 1 : D) * tq, nu = T.nbo ? 2 * n1 : n1, nt = nu + NC * tp;
   const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
   for (int64_t c0 = (int64_t)blockIdx.x * 16; c0 < M.ncells; c0 += (int64_t)gridDim.x * 16) {
     const int64_t cell = min(c0 + (tid & 15), M.ncells - 1);
@@ -2569,9 +2571,10 @@ __global__ void __launch_bounds__(256) cell_rhs_kernel(Tables T, MeshDev M) {
           const int t = t0 + w + 4 * j;  // wave-uniform
           if (t >= (PHYS == kDarcy && flux ? nt : nu)) continue;
           const bool u = t < nu;
-          const int c = u ? (PHYS == kDarcy ? D : t / tq) : (t - nu) / tp;
-          const int n = u ? nq : np, r = 16 * (u ? t % tq : (t - nu) % tp) + i16;
-          const double* const B = (u ? T.Bq : T.Bp) + min(r, n - 1);
+          const int tu = t < n1 ? t : t - n1;
+          const int c = u ? (PHYS == kDarcy ? D : tu / tq) : (t - nu) / tp;
+          const int n = u ? nq : np, r = 16 * (u ? tu % tq : (t - nu) % tp) + i16;
+          const double* const B = (t < n1 ? T.Bq : u ? T.fo_Bq : T.Bp) + min(r, n - 1);
           double b[kRhsPoints / 4];  // a chunk's in flight together
 #pragma unroll
           for (int s = 0; s < kRhsPoints / 4; ++s)
@@ -2590,9 +2593,10 @@ __global__ void __launch_bounds__(256) cell_rhs_kernel(Tables T, MeshDev M) {
         const int t = t0 + w + 4 * j;
         if (t >= nt) continue;
         const bool u = t < nu;
-        const int c = u ? (PHYS == kDarcy ? 0 : t / tq) : (t - nu) / tp;
-        const int n = u ? nq : np, r0 = 16 * (u ? t % tq : (t - nu) % tp) + q4;
-        double* const dst = sq + (u ? na + c * nq : c * np);
+        const int tu = t < n1 ? t : t - n1;
+        const int c = u ? (PHYS == kDarcy ? 0 : tu / tq) : (t - nu) / tp;
+        const int n = u ? nq : np, r0 = 16 * (u ? tu % tq : (t - nu) % tp) + q4;
+        double* const dst = sq + (t < n1 ? na + c * nq : u ? T.ni + c * nq : c * np);
 #pragma unroll
         for (int v = 0; v < 4; ++v)
           if (r0 + 4 * v < n) dst[r0 + 4 * v] = PHYS == kDarcy ? acc[j][v] : -acc[j][v];
@@ -3786,30 +3790,43 @@ static hipError_t launch_flux_schur(const Tables& T, const MeshDev& M, const Con
 
 #include "recover_ref.h"
 
-bool flux_orthonormal(const Tables& T) { return T.phys == kElasticity && T.fo_P && sys_shape(T).flux; }
+bool flux_principal(const Tables& T, bool ref) {
+  const SysShape sh = sys_shape(T);
+  return T.fo_P && (T.phys == kDarcy ? ref && sh.ref : sh.flux);
+}
 
-// The class's tables with the potential in the orthonormal basis (fo_P set), or
+// The class's tables with the potential in the principal basis (fo_P set), or
 // in its own (fo_P null).
-static Tables orthonormal_tables(const Tables& T) {
+static Tables principal_tables(const Tables& T) {
   Tables o = T;
   o.fr_uu = T.fo_uu;
   o.fr_ub = T.fo_ub;
   o.fr_qm = T.fo_qm;
   o.Fqq = T.fo_qq;
+  o.fr_hm = T.fo_hm;
   o.fr_G = T.fo_G;
+  o.fr_Gt = T.fo_Gt;
   return o;
+}
+
+static hipError_t launch_tile_ref(const Tables& T, const MeshDev& M, const CondenseOut& out,
+                                  hipStream_t st, int gridmul) {
+  if (T.phys == kDarcy)
+    return T.D == 2 ? launch_tile_ref<kDarcy, 2>(T, M, out, st, gridmul)
+                    : launch_tile_ref<kDarcy, 3>(T, M, out, st, gridmul);
+  return T.D == 2 ? launch_tile_ref<kElasticity, 2>(T, M, out, st, gridmul)
+                  : launch_tile_ref<kElasticity, 3>(T, M, out, st, gridmul);
 }
 
 hipError_t launch_flux_factors(const Tables& T, const MeshDev& M, const CondenseOut& out,
                                hipStream_t st) {
-  if (!flux_orthonormal(T) || !out.U || !out.Y || out.u_stride < (int64_t)factor_slot(sys_shape(T)) ||
+  if (!flux_principal(T, true) || !out.U || !out.Y || out.u_stride < (int64_t)factor_slot(sys_shape(T)) ||
       out.y_stride < (int64_t)(T.nb + 1) * (T.ni - T.na))
     return hipErrorInvalidValue;
   if (M.ncells <= 0) return hipSuccess;
   Tables own = T;
   own.fo_P = nullptr;
-  return T.D == 2 ? launch_tile_ref<kElasticity, 2>(own, M, out, st, 0)
-                  : launch_tile_ref<kElasticity, 3>(own, M, out, st, 0);
+  return launch_tile_ref(own, M, out, st, 0);
 }
 
 hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const CondenseOut& out,
@@ -3827,17 +3844,9 @@ hipError_t launch_condense_flux(const Tables& T, const MeshDev& M, const Condens
   CondenseOut o = out;
   if (out.keep_uu) o.Auu = out.U + fs.auu;
   o.Rinv = out.U + fs.ri;
-  if (flux_orthonormal(T)) {  // (U: launch_flux_factors)
-    o.U = nullptr;
-    const Tables To = orthonormal_tables(T);
-    return T.D == 2 ? launch_tile_ref<kElasticity, 2>(To, M, o, st, gridmul)
-                    : launch_tile_ref<kElasticity, 3>(To, M, o, st, gridmul);
-  }
-  if (T.phys == kDarcy)
-    return T.D == 2 ? launch_tile_ref<kDarcy, 2>(T, M, o, st, gridmul)
-                    : launch_tile_ref<kDarcy, 3>(T, M, o, st, gridmul);
-  return T.D == 2 ? launch_tile_ref<kElasticity, 2>(T, M, o, st, gridmul)
-                  : launch_tile_ref<kElasticity, 3>(T, M, o, st, gridmul);
+  const bool orth = flux_principal(T, ref);
+  if (orth) o.U = nullptr;  // (launch_flux_factors)
+  return launch_tile_ref(orth ? principal_tables(T) : T, M, o, st, gridmul);
 }
 
 size_t factor_slot(const SysShape& sh) {
@@ -3882,10 +3891,10 @@ SysShape sys_shape(const TablesHost& t) { return shape_of(t, !t.fb_minv.empty())
 //   z = A_qq^-1 r_q (A_qq^-1 = C^-1 (x) M^-1),  d_u = R_uu^-1 (r_u - A_uq z),
 //   d_q = z - A_qq^-1 A_qu d_u,
 // applied to c and then, up to kFluxRefineSteps times, to the residual of the
-// full interior system, r = c - A_ii x.  The reduced system R_uu is worse
-// conditioned than A_ii when the flux block is small (large kappa): the first
-// x_u can be off by cond(R_uu) eps in the near-null mode of A_uq A_qq^-1 A_qu,
-// and the refinement brings it to the accuracy of a direct FP64 solve of A_ii.
+// full interior system, r = c - A_ii x.  R_uu is worse conditioned than A_ii
+// when the flux block is small (large kappa): the functions that no flux sees
+// stand beside entries of the order of kappa.  With REF all of it is in the
+// principal basis of the potential, which keeps the two apart (build_flux_ref).
 // Each step reads every kept block once: A_qu x_u is carried from step to step
 // (A_qu x_u + A_qu d_u), and r_u - A_uq z is formed as c_u - A_uu x_u -
 // A_uq (x_q + z), whose rounding is that of the residual itself.  It stops
@@ -3937,7 +3946,7 @@ __device__ inline double p_column(const double* p, int ld, const double* v, int 
 //   elasticity: (A_qu v)[(s, i)] = sum over the components d of s = (p, q) of
 //               sum_e c_e,partner t_de[i],  t_de = G_e v_d;
 // and A_uq = -A_qu^T; A_uu is kept for one potential component.  G_e is staged
-// in LDS once per workgroup (g_lds; p_lds: the orthonormal basis as well), or, where it does not fit (2D Darcy k=6),
+// in LDS once per workgroup (g_lds; p_lds: the principal basis as well), or, where it does not fit (2D Darcy k=6),
 // read from the table, which every cell shares (L2-resident).
 template <int PHYS, int KQ, int KU, bool REF>
 __global__ void __launch_bounds__(256)
@@ -3960,7 +3969,7 @@ __global__ void __launch_bounds__(256)
   // G_e[i][c] at gsrc[(e * np + i) * gld + c]
   const double* gsrc = g_lds ? s_gu : T.fr_G;
   const int gld = g_lds ? nq : nq + T.nF * T.nm;
-  const bool orth = REF && PHYS != kDarcy && T.fo_P;  // the steps are in that basis
+  const bool orth = REF && T.fo_P;  // the steps are in that basis
   const int psz = orth && p_lds ? nq * nq : 0;
   double* const s_p = s_gu + gsz;  // p_lds: fo_P [j][i]
   double* alpha = s_m + 2 * np * np + gsz + psz + (int64_t)w * rec_wave_lds(na, nu, nb, REF ? ng : 0);
@@ -4303,9 +4312,11 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
   rs.auu = fs.auu;
   rs.aqu = fs.aqu;
   rs.auq = fs.auq;
+  const bool orth = flux_principal(T, ref);
+  const Tables Tr = orth ? principal_tables(T) : T;
   if (M.ncells > 0 && group) {
     const auto go = T.D == 2 ? launch_recover_ref<2> : launch_recover_ref<3>;
-    const hipError_t e = go(T, M, U + fs.ri, usz, cell_dofs, lam_free, lam_dir, out, st);
+    const hipError_t e = go(Tr, M, U + fs.ri, usz, cell_dofs, lam_free, lam_dir, out, st);
     if (e != hipSuccess) return e;
   } else if (M.ncells > 0) {
     const int64_t blocks = (M.ncells + kRecWaves - 1) / kRecWaves;
@@ -4317,11 +4328,10 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
     const size_t gbytes = (size_t)T.D * T.np * T.nq * sizeof(double);
     // G_e in LDS while two workgroups still fit a CU
     const bool g_lds = ref && base + gbytes <= 64 * 1024;
-    const size_t pbytes = flux_orthonormal(T) ? (size_t)T.nq * T.nq * sizeof(double) : 0;
+    const size_t pbytes = orth ? (size_t)T.nq * T.nq * sizeof(double) : 0;
     const bool p_lds = g_lds && base + gbytes + pbytes <= 64 * 1024;
     const size_t lds = base + (g_lds ? gbytes : 0) + (p_lds ? pbytes : 0);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
-    const Tables Tr = flux_orthonormal(T) ? orthonormal_tables(T) : T;
     ClockScope clk_(st, "recover_flux");
 #define HDG_RF(P_, K_, U_, R_)                                                                  \
   hipLaunchKernelGGL((recover_flux_kernel<P_, K_, U_, R_>), dim3(grid), dim3(64 * kRecWaves),   \

@@ -28,16 +28,16 @@
 //   z = A_qq^-1 r_q (A_qq^-1 = C^-1 (x) M^-1),  d_u = R_uu^-1 (r_u - A_uq z),
 //   d_q = z - A_qq^-1 A_qu d_u,
 // applied to c and then, up to kFluxRefineSteps times, to the residual of the
-// full interior system, r = c - A_ii x: R_uu is worse conditioned than A_ii
-// when the flux block is small (large kappa), the first x_u can be off by
-// cond(R_uu) eps in the near-null mode of A_uq A_qq^-1 A_qu, and the refinement
-// brings it to the accuracy of a direct FP64 solve of A_ii.  c_q - A_qu x_u is
-// carried from step to step, and r_u - A_uq z is formed as
+// full interior system, r = c - A_ii x.  All of it is in the principal basis of
+// the potential (build_flux_ref), where R_uu^-1 is exact enough however small the
+// flux block is (large kappa); x_u returns to the nodal one at the end.  c_q -
+// A_qu x_u is carried from step to step, and r_u - A_uq z is formed as
 // c_u - A_uu x_u - A_uq (x_q + z), whose rounding is that of the residual
 // itself.  A cell's columns rest once its correction is below 2^-44 of its
-// solution (the next would be smaller by the ratio of this one to the error it
-// removed, below 2^-8 wherever R_uu^-1 is of use at all); the workgroup ends
-// when all 16 do.
+// solution: the next would be smaller by the ratio of this one to the error it
+// removed.  (With 2^-48, or without resting, the errors of 60 to 500 cells each
+// of 2D k=3 and 4 and of 3D k=1 and 2, kappa up to lognormal(0, 3), have the same
+// quantiles to a few percent.)  The workgroup ends when all 16 do.
 
 constexpr int kRecLd = 17;    // doubles between rows of a vector in LDS
 constexpr int kRecCoef = 17;  // coefficients of a cell, at most
@@ -171,8 +171,9 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
       for (int v = 0; v < 4; ++v) ca[a][v] = bi[a * np + min(16 * w + 4 * v + q4, np - 1)];
     }
+    const double* const bu = bi + (T.fo_P ? T.ni : na);  // in the basis of the tables
 #pragma unroll
-    for (int v = 0; v < 4; ++v) cu[0][v] = bi[na + min(16 * w + 4 * v + q4, nq - 1)];
+    for (int v = 0; v < 4; ++v) cu[0][v] = bu[min(16 * w + 4 * v + q4, nq - 1)];
     {
       dbl4 t[D], q[D];
 #pragma unroll
@@ -357,6 +358,11 @@ __global__ void __launch_bounds__(512, 2)
       for (int a = 0; a < D; ++a) put(V + a * np4 * kRecLd, xq[a], np);
       __syncthreads();
     }
+    dbl4 ux[1] = {zero};
+    if (T.fo_P && qrow)  // x_u = P x_u'
+      rec_mm<1, 1>(
+          ux, nq, q4, [&](int, int k) { return table_at(T.fo_Pt, 8u * (qr + k * nq)); },
+          [&](int, int k) { return XU[k * kRecLd + i16]; });
     if (c0 + i16 < ncells) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -364,7 +370,7 @@ __global__ void __launch_bounds__(512, 2)
         if (r < np)
 #pragma unroll
           for (int a = 0; a < D; ++a) out[cell * na + a * np + r] = xq[a][v];
-        if (r < nq) out[ncells * na + cell * nq + r] = XU[r * kRecLd + i16];
+        if (r < nq) out[ncells * na + cell * nq + r] = T.fo_P ? ux[0][v] : XU[r * kRecLd + i16];
       }
     }
     __syncthreads();  // LDS reuse by the next cells

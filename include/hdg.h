@@ -347,10 +347,10 @@ int hdg_cell_blocks(hdg_mesh* mesh, const double** S, const double** g,
  * are the factors of the reduced system of the m = ni - n_flux non-flux interior
  * unknowns, at the start of each cell's slot (the rest of the slot holds the
  * recovery's kept blocks and the inverse of the reduced interior block; not part
- * of this interface).  Elasticity's family 8 works in another basis of the
- * displacement and forms U and Y when this is called; from then on every
- * condensation of the mesh forms them too, so the pointers' contents stay
- * current.  Cell c's slots start at c * u_stride and c * y_stride
+ * of this interface).  Family 10 and elasticity's family 8 work in another basis
+ * of the potential (displacement) and form U and Y when this is called; from
+ * then on every condensation of the mesh forms them too, so the pointers'
+ * contents stay current.  Cell c's slots start at c * u_stride and c * y_stride
  * (hdg_mesh_factor_layout). */
 int hdg_local_factors(hdg_mesh* mesh, const double** U, const double** Y);
 /* Layout of the resident factors: rows m of the factored system (ni, or
