@@ -1612,8 +1612,8 @@ int recover_facet_major(hdg_mesh* m, const double* lam_free, double* free_values
   }
   if (m->used_family == kFamilyFluxSchur || m->used_family == kFamilyFluxRef) {
     const CellLayout L(m->th);
-    HIP_TRY(ctx, launch_recover_flux(m->tdev, m->meshdev(), m->pU, (int64_t)L.U,
-                                     m->used_family == kFamilyFluxRef, m->rec_group,
+    HIP_TRY(ctx, launch_recover_flux(m->tdev, m->meshdev(), m->pU, m->pY, (int64_t)L.U,
+                                     (int64_t)L.Y, m->used_family == kFamilyFluxRef, m->rec_group,
                                      m->d_cell_dofs.as<int32_t>(), lam_free,
                                      m->d_lam_dir.as<double>(), free_values, m->nfree,
                                      ctx->stream),

@@ -332,9 +332,9 @@ hipError_t launch_flux_factors(const Tables& T, const MeshDev& M, const Condense
 // decides with recover_by_group on the cells of one recovery and keeps the
 // answer for it.
 bool recover_by_group(const Tables& T, int64_t ncells);
-hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, int64_t usz,
-                               bool ref, bool group, const int32_t* cell_dofs,
-                               const double* lam_free,
+hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, const double* Y,
+                               int64_t usz, int64_t ysz, bool ref, bool group,
+                               const int32_t* cell_dofs, const double* lam_free,
                                const double* lam_dir, double* out, int64_t nfree,
                                hipStream_t st);
 constexpr int kFluxRefineSteps = 2;  // FP64 refinement steps of the flux recovery (at most)

@@ -3894,7 +3894,10 @@ SysShape sys_shape(const TablesHost& t) { return shape_of(t, !t.fb_minv.empty())
 // full interior system, r = c - A_ii x.  R_uu is worse conditioned than A_ii
 // when the flux block is small (large kappa): the functions that no flux sees
 // stand beside entries of the order of kappa.  With REF all of it is in the
-// principal basis of the potential, which keeps the two apart (build_flux_ref).
+// principal basis of the potential, which keeps the two apart (build_flux_ref);
+// without, the first d_u is back-substituted, x_u = U^-1 (y - Y lambda): its
+// error stays with those functions, where that of R_uu^-1 t reaches all (3D k=1,
+// 5^3 cells, kappa up to 1e8: errors of 6e-8 and 2e-1).
 // Each step reads every kept block once: A_qu x_u is carried from step to step
 // (A_qu x_u + A_qu d_u), and r_u - A_uq z is formed as c_u - A_uu x_u -
 // A_uq (x_q + z), whose rounding is that of the residual itself.  It stops
@@ -3911,6 +3914,8 @@ struct RecSlot {
   const double* slot;  // per-cell slots, stride usz
   int64_t usz;
   int64_t ri, auu, aqu, auq;  // R_uu^-1 [col][row], A_uu, A_qu, A_uq (offsets in the slot)
+  const double* y;            // Y, stride ysz (not REF)
+  int64_t ysz;
 };
 
 // C^-1 (6 x 6, row-major) of a cell's flux block C (x) M, one entry per lane:
@@ -4234,6 +4239,20 @@ __global__ void __launch_bounds__(256)
 #pragma unroll 4
           for (int j = 0; j < nu; ++j) du[t] = fma(Ri[(int64_t)j * nu + r], uv[j], du[t]);
       }
+      if (!REF && it == 0) {  // x_u = U^-1 (y - Y lambda): KU = 1
+        const double* const Yc = rs.y + cell * rs.ysz + min(lane, nu - 1);
+        double x = Yc[(int64_t)nb * nu];
+#pragma unroll 4
+        for (int j = 0; j < nb; ++j) x = fma(-Yc[(int64_t)j * nu], lam[j], x);
+#pragma unroll 4
+        for (int c = nu - 1; c >= 0; --c) {
+          const double uc = base[c * (c + 1) / 2 + min(lane, c)];
+          const double p = wave_readlane_f64(uc, c), v = wave_readlane_f64(x, c);
+          const double xc = p != 0.0 ? v / p : 0.0;
+          x = lane < c ? fma(-uc, xc, x) : lane == c ? xc : x;
+        }
+        du[0] = lane < nu ? x : 0.0;
+      }
       wave_sync_lds();
 #pragma unroll
       for (int t = 0; t < KU; ++t)
@@ -4293,10 +4312,11 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, int64_t usz,
-                               bool ref, bool group, const int32_t* cell_dofs,
-                               const double* lam_free, const double* lam_dir, double* out,
-                               int64_t nfree, hipStream_t st) {
+hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* U, const double* Y,
+                               int64_t usz, int64_t ysz, bool ref, bool group,
+                               const int32_t* cell_dofs, const double* lam_free,
+                               const double* lam_dir, double* out, int64_t nfree,
+                               hipStream_t st) {
   const int na = T.na, nu = T.ni - na, nb = T.nb;
   const SysShape sh = sys_shape(T);
   ref = ref || T.phys != kDarcy;
@@ -4306,6 +4326,8 @@ hipError_t launch_recover_flux(const Tables& T, const MeshDev& M, const double* 
   RecSlot rs;
   rs.slot = U;
   rs.usz = usz;
+  rs.y = Y;
+  rs.ysz = ysz;
   const FluxSlot fs = flux_slot(sh.flux_keep, nu);
   if (usz < fs.size) return hipErrorInvalidValue;
   rs.ri = fs.ri;

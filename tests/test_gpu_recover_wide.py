@@ -67,6 +67,36 @@ def test_darcy_large_permeabilities(ctx, D, k, cells, space):
     op.close()
 
 
+# Darcy's family 8 (both products per cell) and reflected cells, which it serves
+@pytest.mark.parametrize("D,k,n", [(2, 3, 9), (3, 1, 5), (3, 2, 4)])
+@pytest.mark.parametrize("reflect", [False, True])
+def test_darcy_large_permeabilities_products_per_cell(ctx, D, k, n, reflect):
+    import gridaphybrid as gh
+    import meshgen
+    print(f"large permeabilities, family 8, D={D} k={k} reflected={reflect}", flush=True)
+    nc = n ** D
+    kappa = 10.0 ** (np.arange(nc) % 9)
+    if reflect:
+        x0, J, cf, nf, perm, _ = meshgen.sheared_rotated_mesh(D, n, seed=14, frac=0.0)
+        c, f = nc // 2, (2, 3) if D == 2 else (4, 5)   # xi_0 -> 1 - xi_0
+        x0[c] = x0[c] + J[c][:, 0]
+        J[c][:, 0] = -J[c][:, 0]
+        cf[c][list(f)] = cf[c][list(f[::-1])]
+        perm[:] = 0
+        perm[c] = [1, 1, 0, 0] if D == 2 else [2, 2, 2, 2, 0, 0]
+        model = gh.AffineDiscreteModel(x0=x0, J=J, cell_facets=cf, nfacets=nf, facet_perm=perm)
+    else:
+        model = gh.CartesianDiscreteModel((0.0, 1.0) * D, (n,) * D)
+    X = gh.HDGSpaces.darcy_baseline(model, k)
+    op = gh.HybridAffineFEOperator(gh.DarcyHDG(tau=1.0, kappa=kappa, source=0), X, X, [1, 2], [3],
+                                   ctx=ctx, assemble=False)
+    op.set_family(8)
+    op.assemble()
+    _check(op, 1 + 0.1 * np.random.default_rng(2).standard_normal(op.info.nfree), nc // 2,
+           min(9, nc - nc // 2))
+    op.close()
+
+
 @pytest.mark.parametrize("D,k,E", [(3, 1, 1e4), (3, 1, 1e8), (3, 2, 1e6), (2, 4, 1e8)])
 def test_elasticity_large_moduli(ctx, D, k, E):
     import gridaphybrid as gh
