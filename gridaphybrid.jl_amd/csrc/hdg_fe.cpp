@@ -871,29 +871,92 @@ void detect_flux_sym(TablesHost& t) {
 //   fr_hm  (Darcy) H_e = M^-1 G_e [e][i][column], for a flux right-hand side;
 //   fr_G   G_e, [e][i][column]; fr_Gt  the same as [e][column][i].
 //
-// And once more with the potential in a principal basis u = fo_P u' (fo_*):
-// orthonormal in the reference mass and diagonal in sum_e G_e^T M^-1 G_e, which
-// leaves the functions that no flux sees (Darcy Q_k: one; elasticity P_(k+1):
-// those orthogonal to P_(k-1)) as its last ones, with zero columns of G.  S and g
-// do not depend on the basis; their rounding, and R_uu^-1, do:
+// And once more with the potential in a principal basis u = fo_P u' (fo_*): the
+// functions that no flux sees (zero columns of G; Darcy Q_k: one, elasticity
+// P_(k+1): those orthogonal to P_(k-1)) last, those that no facet sees (zero in
+// Fqq and Fqm) before them, each orthonormal in the reference mass, and an
+// orthonormal rest.  S and g do not depend on the basis; their rounding, and
+// R_uu^-1, do:
 //  - R_uu has entries of the order of the coefficient (kappa, E) on the functions
 //    a flux sees, and the stabilisation alone on the others.  In the nodal basis
 //    the two mix, and from kappa = 1e5 on (2D k=3, 20^2 cells; with h = 1/211 from
 //    1e4) the recovery through R_uu^-1 lost its values altogether (errors of order
 //    1 at 1e6).  Here they are entries of their own: 9e-9 at 1e6, 2e-7 at 1e8,
-//    which LAPACK's solve of A_ii has too (1e-8, 8e-7).
+//    which LAPACK's solve of A_ii has too (1e-8, 8e-7).  At small coefficients it
+//    is the stabilisation that is large, on all but the functions inside the
+//    cell (without their zeros 4e-7 at 1e-12, 211 x 77 cells; with them 9e-16).
 //  - the nodal basis of P_(k+1) on the cube (nodes on a simplex, extrapolated)
 //    gives elasticity's R_uu a condition of 1.9e8 for 3D k=3, here 27: S was
 //    7.0e-12 of its largest entry off, 1.6e-12 after a dense elimination of all
 //    225 rows, and is 8.0e-13 off; k=2 2.0e-13, 4.9e-14 and 2.9e-14; Darcy 2D
-//    k=3, 211 x 77 cells, 4.7e-15, 1.1e-15 and 2.6e-15 (against extended
+//    k=3, 211 x 77 cells, 4.6e-15, 1.1e-15 and 3.5e-15 (against extended
 //    precision; what is left is the rounding of the nodal tables).
 // Any fo_P is exact, the tables being formed from its rounded entries.
-// P with P^T M P = I and P^T K P diagonal, descending (Cholesky of M, cyclic
-// Jacobi on C^-1 K C^-T); false if M is not positive definite.
-static bool principal_basis(int n, const std::vector<double>& M, const std::vector<long double>& K,
-                            std::vector<double>& P) {
-  std::vector<long double> C((size_t)n * n, 0.0L), A = K, V((size_t)n * n, 0.0L);
+namespace {
+using LVec = std::vector<long double>;
+
+// Orthogonalises the columns v (stored one after the other, length n) from
+// column `first` on against all before them, twice, and normalises them; false
+// if one is dependent.
+bool orthonormalise(int n, LVec& v, int first) {
+  const int m = (int)(v.size() / n);
+  for (int j = first; j < m; ++j) {
+    long double len0 = 0.0L, len = 0.0L;
+    for (int i = 0; i < n; ++i) len0 += v[(size_t)j * n + i] * v[(size_t)j * n + i];
+    for (int pass = 0; pass < 2; ++pass)
+      for (int k = 0; k < j; ++k) {
+        long double d = 0.0L;
+        for (int i = 0; i < n; ++i) d += v[(size_t)k * n + i] * v[(size_t)j * n + i];
+        for (int i = 0; i < n; ++i) v[(size_t)j * n + i] -= d * v[(size_t)k * n + i];
+      }
+    for (int i = 0; i < n; ++i) len += v[(size_t)j * n + i] * v[(size_t)j * n + i];
+    if (!(len > 1e-6L * len0)) return false;
+    for (int i = 0; i < n; ++i) v[(size_t)j * n + i] /= std::sqrt(len);
+  }
+  return true;
+}
+
+// Orthonormal basis of the null space of A (symmetric, positive semidefinite up
+// to its entries' rounding): Cholesky with diagonal pivoting, whose rest below
+// 1e-11 of the largest pivot is taken as zero.
+LVec null_space(int n, const LVec& A0) {
+  LVec A = A0;
+  std::vector<int> at(n);
+  for (int i = 0; i < n; ++i) at[i] = i;
+  long double top = 0.0L;
+  int r = 0;
+  for (; r < n; ++r) {
+    int p = r;
+    for (int i = r + 1; i < n; ++i)
+      if (A[(size_t)at[i] * n + at[i]] > A[(size_t)at[p] * n + at[p]]) p = i;
+    const long double d = A[(size_t)at[p] * n + at[p]];
+    if (r == 0) top = d;
+    if (!(d > 1e-11L * top)) break;
+    std::swap(at[r], at[p]);
+    for (int i = r + 1; i < n; ++i) {  // the pivot's row of the factor stays in A
+      const long double l = A[(size_t)at[i] * n + at[r]] / d;
+      for (int j = r + 1; j < n; ++j)
+        A[(size_t)at[i] * n + at[j]] -= l * A[(size_t)at[r] * n + at[j]];
+    }
+  }
+  LVec v((size_t)(n - r) * n, 0.0L);
+  for (int j = r; j < n; ++j) {  // A_r,r x = -A_r,j
+    long double* const x = &v[(size_t)(j - r) * n];
+    x[at[j]] = 1.0L;
+    for (int i = r - 1; i >= 0; --i) {
+      long double s = A[(size_t)at[i] * n + at[j]];
+      for (int k = i + 1; k < r; ++k) s += A[(size_t)at[i] * n + at[k]] * x[at[k]];
+      x[at[i]] = -s / A[(size_t)at[i] * n + at[i]];
+    }
+  }
+  return orthonormalise(n, v, 0) ? v : LVec();
+}
+
+// The basis P of build_flux_ref from the reference mass M, K = sum_e G_e^T M^-1
+// G_e and the sum of the facet masses T; false if M is not positive definite.
+bool principal_basis(int n, const std::vector<double>& M, const LVec& K, const LVec& T,
+                     std::vector<double>& P) {
+  LVec C((size_t)n * n, 0.0L);
   for (int j = 0; j < n; ++j) {
     long double d = M[(size_t)j * n + j];
     for (int k = 0; k < j; ++k) d -= C[(size_t)j * n + k] * C[(size_t)j * n + k];
@@ -906,63 +969,59 @@ static bool principal_basis(int n, const std::vector<double>& M, const std::vect
       C[(size_t)i * n + j] = v / C[(size_t)j * n + j];
     }
   }
-  // A = C^-1 K C^-T: rows, then columns
-  for (int pass = 0; pass < 2; ++pass) {
-    for (int c = 0; c < n; ++c)
+  auto reduced = [&](LVec A) {  // C^-1 A C^-T: rows, then columns
+    for (int pass = 0; pass < 2; ++pass) {
       for (int i = 0; i < n; ++i) {
-        long double v = A[(size_t)i * n + c];
-        for (int k = 0; k < i; ++k) v -= C[(size_t)i * n + k] * A[(size_t)k * n + c];
-        A[(size_t)i * n + c] = v / C[(size_t)i * n + i];
+        for (int k = 0; k < i; ++k)
+          for (int c = 0; c < n; ++c)
+            A[(size_t)i * n + c] -= C[(size_t)i * n + k] * A[(size_t)k * n + c];
+        for (int c = 0; c < n; ++c) A[(size_t)i * n + c] /= C[(size_t)i * n + i];
       }
-    for (int i = 0; i < n; ++i)
-      for (int j = 0; j < i; ++j) std::swap(A[(size_t)i * n + j], A[(size_t)j * n + i]);
+      for (int i = 0; i < n; ++i)
+        for (int j = 0; j < i; ++j) std::swap(A[(size_t)i * n + j], A[(size_t)j * n + i]);
+    }
+    return A;
+  };
+  const LVec unseen = null_space(n, reduced(K));
+  LVec inside = null_space(n, reduced(T));
+  LVec all = inside;
+  all.insert(all.end(), unseen.begin(), unseen.end());
+  if (!orthonormalise(n, all, (int)(inside.size() / n))) {  // (not independent)
+    inside.clear();
+    all = unseen;
   }
-  for (int i = 0; i < n; ++i) V[(size_t)i * n + i] = 1.0L;
-  for (int sweep = 0; sweep < 30; ++sweep) {
-    long double off = 0.0L, dia = 0.0L;
-    for (int i = 0; i < n; ++i)
-      for (int j = 0; j < n; ++j)
-        (i == j ? dia : off) += A[(size_t)i * n + j] * A[(size_t)i * n + j];
-    if (off <= 1e-38L * dia) break;  // (V: eigenvectors in rows)
-    for (int p = 0; p < n; ++p)
-      for (int q = p + 1; q < n; ++q) {
-        const long double apq = A[(size_t)p * n + q];
-        if (apq * apq <= 1e-42L * dia) continue;
-        const long double th = (A[(size_t)q * n + q] - A[(size_t)p * n + p]) / (2.0L * apq);
-        const long double t =
-            (th >= 0.0L ? 1.0L : -1.0L) / (std::fabs(th) + std::sqrt(th * th + 1.0L));
-        const long double c = 1.0L / std::sqrt(t * t + 1.0L), sn = t * c;
-        for (int k = 0; k < n; ++k) {
-          const long double u = V[(size_t)p * n + k], w = V[(size_t)q * n + k];
-          V[(size_t)p * n + k] = c * u - sn * w;
-          V[(size_t)q * n + k] = sn * u + c * w;
-          if (k == p || k == q) continue;
-          const long double x = A[(size_t)p * n + k], y = A[(size_t)q * n + k];
-          A[(size_t)k * n + p] = A[(size_t)p * n + k] = c * x - sn * y;
-          A[(size_t)k * n + q] = A[(size_t)q * n + k] = sn * x + c * y;
-        }
-        A[(size_t)p * n + p] -= t * apq;
-        A[(size_t)q * n + q] += t * apq;
-        A[(size_t)p * n + q] = A[(size_t)q * n + p] = 0.0L;
-      }
+  // the rest: the unit vectors furthest from what is there, one after the other
+  LVec rest;
+  LVec far(n, 1.0L);  // 1 - |projection of e_i|^2
+  auto take = [&](const long double* q) {
+    for (int i = 0; i < n; ++i) far[i] -= q[i] * q[i];
+  };
+  for (size_t j = 0; j < all.size(); j += n) take(&all[j]);
+  while ((int)(all.size() / n) < n) {
+    const int i = (int)(std::max_element(far.begin(), far.end()) - far.begin());
+    all.resize(all.size() + n, 0.0L);
+    const size_t last = all.size() - n;
+    all[last + i] = 1.0L;
+    if (!orthonormalise(n, all, (int)(last / n))) return false;
+    take(&all[last]);
+    rest.insert(rest.end(), all.begin() + last, all.end());
   }
-  std::vector<int> at(n);
-  for (int j = 0; j < n; ++j) at[j] = j;
-  std::sort(at.begin(), at.end(), [&](int i, int j) {
-    return A[(size_t)i * n + i] > A[(size_t)j * n + j];
-  });
+  LVec v = rest;
+  v.insert(v.end(), inside.begin(), inside.end());
+  v.insert(v.end(), unseen.begin(), unseen.end());
   P.assign((size_t)n * n, 0.0);
-  std::vector<long double> x(n);
-  for (int j = 0; j < n; ++j) {  // C^T x = v
+  LVec x(n);
+  for (int j = 0; j < n; ++j) {  // C^T x = v_j
     for (int i = n - 1; i >= 0; --i) {
-      long double v = V[(size_t)at[j] * n + i];
-      for (int k = i + 1; k < n; ++k) v -= C[(size_t)k * n + i] * x[k];
-      x[i] = v / C[(size_t)i * n + i];
+      long double s = v[(size_t)j * n + i];
+      for (int k = i + 1; k < n; ++k) s -= C[(size_t)k * n + i] * x[k];
+      x[i] = s / C[(size_t)i * n + i];
     }
     for (int i = 0; i < n; ++i) P[(size_t)i * n + j] = (double)x[i];
   }
   return true;
 }
+}  // namespace
 
 void build_flux_ref(TablesHost& t) {
   t.fr_npair = 0;
@@ -1074,7 +1133,10 @@ void build_flux_ref(TablesHost& t) {
   for (size_t r = 0; r < (size_t)D * np; ++r)
     for (int i = 0; i < nq; ++i)
       for (int j = 0; j < nq; ++j) K[(size_t)i * nq + j] += G[r * nr + i] * H[r * nr + j];
-  if (!principal_basis(nq, t.Mqq, K, t.fo_P)) return;
+  std::vector<long double> Ts((size_t)nq * nq, 0.0L);
+  for (size_t k = 0; k < t.Fqq.size(); ++k)
+    Ts[k % ((size_t)nq * nq)] += t.Fqq[k];
+  if (!principal_basis(nq, t.Mqq, K, Ts, t.fo_P)) return;
   t.fo_Pt.assign((size_t)nq * nq, 0.0);
   for (int i = 0; i < nq; ++i)
     for (int j = 0; j < nq; ++j) t.fo_Pt[(size_t)j * nq + i] = t.fo_P[(size_t)i * nq + j];
@@ -1126,6 +1188,18 @@ void build_flux_ref(TablesHost& t) {
     for (int j = 0; j < nq; ++j)
       for (int i = 0; i < nq; ++i)
         t.fo_qq[((size_t)f * nq + i) * nq + j] = (double)times_p(&B[(size_t)j * nq], i);
+  }
+  // and the functions no facet sees: their facet masses and couplings
+  double big = 0.0;
+  for (const double v : t.fo_qq) big = std::max(big, std::fabs(v));
+  for (int j = 0; j < nq; ++j) {
+    double own = 0.0;
+    for (int f = 0; f < nF; ++f) own = std::max(own, std::fabs(t.fo_qq[((size_t)f * nq + j) * nq + j]));
+    if (own >= 1e-11 * big) continue;
+    for (int f = 0; f < nF; ++f)
+      for (int i = 0; i < nq; ++i)
+        t.fo_qq[((size_t)f * nq + i) * nq + j] = t.fo_qq[((size_t)f * nq + j) * nq + i] = 0.0;
+    for (int b = 0; b < nbs; ++b) t.fo_qm[(size_t)j * nbs + b] = 0.0;
   }
 }
 

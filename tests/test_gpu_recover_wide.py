@@ -1,5 +1,5 @@
-"""Recovery where the flux block is small: permeabilities (Young's moduli for
-elasticity) of up to 1e8.  The reduced interior block then has entries of the
+"""Recovery where the flux block is small or large: permeabilities from 1e-8 to 1e8
+(Young's moduli of up to 1e8 for elasticity).  The reduced interior block then has entries of the
 order of the coefficient beside the functions that no flux sees, which only the
 stabilisation holds, and its inverse has to keep both apart.
 
@@ -51,15 +51,16 @@ def _check(op, lam, first, cnt):
     (2, 3, (10, 9), 0), (2, 3, (48, 47), 0), (2, 4, (10, 9), 0), (2, 4, (33, 33), 0),
     (3, 1, (5, 5, 4), 0), (3, 1, (13, 13, 13), 0), (3, 2, (4, 4, 4), 0), (3, 3, (3, 3, 3), 0),
     (2, 3, (10, 9), 1), (3, 2, (13, 13, 13), 1)])
-def test_darcy_large_permeabilities(ctx, D, k, cells, space):
+@pytest.mark.parametrize("power", [1, -1])
+def test_darcy_wide_permeabilities(ctx, D, k, cells, space, power):
     import gridaphybrid as gh
-    print(f"large permeabilities D={D} k={k} cells={cells} space={space}", flush=True)
+    print(f"wide permeabilities D={D} k={k} cells={cells} space={space} power={power}", flush=True)
     nc = int(np.prod(cells))
     model = gh.CartesianDiscreteModel((0.0, 1.0) * D, cells)
     X = gh.HDGSpaces(model, k, k, k, space)
     op = gh.HybridAffineFEOperator(
-        gh.DarcyHDG(tau=1.0, kappa=10.0 ** (np.arange(nc) % 9), source=3), X, X, [1, 2], [3],
-        ctx=ctx, assemble=False)
+        gh.DarcyHDG(tau=1.0, kappa=10.0 ** (power * (np.arange(nc) % 9)), source=3), X, X,
+        [1, 2], [3], ctx=ctx, assemble=False)
     op.set_family(10)
     op.assemble()
     _check(op, 1 + 0.1 * np.random.default_rng(2).standard_normal(op.info.nfree), nc // 2,
