@@ -45,12 +45,13 @@ def f_rec(ni, nb):
     return 2 * ni * nb + 2 * ni * ni
 
 
-def kernel_model(kname, info, D, sweeps, family=None, nqc=0):
+def kernel_model(kname, info, D, sweeps, family=None, nqc=0, elasticity=False):
     """Roofline model of one kernel, per cell: (bound, algorithmic quantity,
     unit).  HBM-bound kernels count the compulsory bytes of their inputs and
     outputs (8-byte values, 4-byte ids); compute-bound ones the algorithmic
     flops.  ni, nb: interior and skeleton sizes; na: flux unknowns; nu = ni -
-    na; nr = nu + nb rows of the reduced system; nqc: cell quadrature points."""
+    na; nr = nu + nb rows of the reduced system; nqc: cell quadrature points;
+    elasticity: D displacement components (Darcy otherwise)."""
     ni, nb, na = info.ni, info.nb, info.n_flux
     nu, nr = ni - na, ni - na + nb
     nc = max(int(info.ncells), 1)
@@ -64,20 +65,25 @@ def kernel_model(kname, info, D, sweeps, family=None, nqc=0):
         return "hbm", 8 * (D + D * D + 1 + 72) + 2 * D, "byte"
     if kname == "prep_rhs":
         # reads the cell's origin, Jacobian and coefficient (the built-in
-        # source is evaluated at the quadrature points); writes b_i
-        return "hbm", 8 * (D + D * D + 1 + ni), "byte"
+        # source is evaluated at the quadrature points); writes b_i and its
+        # potential rows in the principal basis
+        return "hbm", 8 * (D + D * D + 1 + ni + nu), "byte"
     if kname == "condense_tile":
-        # the tile elimination of the flux families' reduced systems: reads the
-        # cell coefficients (72) and b_i; writes S, g, U (packed), R_uu^-1, Y and
-        # (but for Darcy's reference products) A_uu of one potential component
-        nq = 0 if family == 10 else nu // (1 if nu * D == na else D)
-        return "hbm", 8 * (72 + ni + nb * nb + nb + nu * (nu + 1) // 2 + nq * nq + nu * nu
-                           + (nb + 1) * nu), "byte"
+        # the tile elimination of the flux families' reduced systems writes S, g,
+        # R_uu^-1 and Y; from reference products it reads the cell coefficients
+        # (72) and b_i and keeps elasticity's A_uu of one component; after
+        # flux_schur (Darcy's family 8) it reads R and writes U (packed)
+        out = nb * nb + nb + nu * nu + (nb + 1) * nu
+        if family == SCHUR_FAMILY and not elasticity:
+            return "hbm", 8 * (nr * (nr + 1) + nu * (nu + 1) // 2 + out), "byte"
+        return "hbm", 8 * (72 + ni + (nu // D) ** 2 * elasticity + out), "byte"
     if kname == "recover_flux":
-        # reads R_uu^-1 (and, for the MFMA-product family, the kept A_uu, A_qu
-        # and A_uq), the cell coefficients and b_i, the cell's trace values and
-        # ids; writes (q, u)
-        kept = 0 if family == 10 else nu * nu + 2 * na * nu
+        # reads R_uu^-1, the cell coefficients and b_i, the cell's trace values and
+        # ids; elasticity A_uu of one component; Darcy's family 8 A_uu, A_qu, A_uq,
+        # U and Y; writes (q, u)
+        kept = (nu // D) ** 2 * elasticity
+        if family == SCHUR_FAMILY and not elasticity:
+            kept = nu * nu + 2 * na * nu + nu * (nu + 1) // 2 + (nb + 1) * nu
         return "hbm", 8 * (nu * nu + kept + 72 + ni + nb + ni) + 4 * nb, "byte"
     if kname == "assemble":
         # reads every S block once; writes the CSC values
@@ -689,7 +695,7 @@ def main():
             t_launch = run["kernels_ms_per_launch"][k]
             cpl = nc / (t_step / t_launch)
             bound, q, unit = kernel_model(k, info, 3, sweeps, run.get("family"),
-                                          (args.order + 2) ** 3)
+                                          (args.order + 2) ** 3, args.physics == "elasticity")
             rate = q * cpl / (t_launch * 1e-3)
             if bound == "hbm":
                 out[k] = dict(bound="hbm", achieved=rate / 1e9, peak=PEAK_HBM_GBS, unit="GB/s",
