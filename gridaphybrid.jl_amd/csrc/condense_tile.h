@@ -34,13 +34,16 @@
 // (register-grid, workspace-panel and blocked eliminations, the reduced systems
 // formed by kernels of their own and written to memory, the inverses by another):
 //   map level, 4,096 cells of 108 + 54, both maps   17.1 -> 5.1 ms
-//   Darcy 64^3 k=2 (27 + 54 of 108 + 54)            25.2 -> 9.7 ms
-//   Darcy 24^3 k=3 (64 + 96 of 256 + 96)            17.6 -> 3.5 ms
-//   elasticity 5,814 cells k=2 (60 + 108)            9.4 -> 1.6 ms
-//   elasticity 1,728 cells k=3 (105 + 180)          12.1 -> 2.2 ms
+//   Darcy 64^3 k=2 (27 + 54 of 108 + 54)            25.2 -> 9.4 ms
+//   Darcy 24^3 k=3 (64 + 96 of 256 + 96)            17.6 -> 3.4 ms
+//   elasticity 5,814 cells k=2 (60 + 108)            9.4 -> 1.5 ms
+//   elasticity 1,728 cells k=3 (105 + 180)          12.1 -> 2.1 ms
 // The symmetry of the reduced systems (half of S formed, both halves stored; a
-// column's weights looked up once) and no scratch memory in any instance gave
-// 11.9 -> 9.7, 6.2 -> 3.5, 2.8 -> 1.6 and 3.3 -> 2.2 ms of the last four.
+// column's weights looked up once) and less scratch memory gave 11.9 -> 9.7, 6.2
+// -> 3.5, 2.8 -> 1.6 and 3.3 -> 2.2 ms of the last four, and not storing U, which
+// no recovery of theirs reads, the rest.  The four wavefront kernels of RefGen
+// with two row tiles keep 48 to 64 bytes a lane in scratch memory (168 VGPRs, for
+// three wavefronts a SIMD); no other instance has any.
 
 // c ? a : b and c ? a : 0 by masks.  The compiler turns a conditional of loaded
 // values into branches around the loads, one latency after the other; through

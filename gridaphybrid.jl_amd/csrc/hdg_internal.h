@@ -296,6 +296,10 @@ SysShape sys_shape(const TablesHost& t);
 // families; for classes where the flux-block path applies, room for its
 // reduced factors and the interior blocks its recovery refines with:
 //   [U m(m+1)/2][A_uu m*m][A_qu na*m][A_uq m*na][R_uu^-1 m*m],  m = ni - na.
+// The Schur complement of family 8 on Darcy fills all of it.  The reference
+// products write R_uu^-1, in the principal basis of the potential, and A_uu (of
+// one component) if CondenseOut::keep_uu; U, in the nodal basis, only once
+// hdg_local_factors has asked for it (launch_flux_factors); A_qu and A_uq never.
 size_t factor_slot(const SysShape& sh);
 // Family id of the flux-block Schur complement: the flux unknowns are
 // eliminated through C^-1 (x) M^-1 and the reduced system of the remaining

@@ -2490,10 +2490,13 @@ static size_t flux_workspace_bytes(int nr, int64_t ncells);
 int condense_default_family(const SysShape& sh) {
   // Where the flux block goes through reference products the reduced system wins
   // from the 48 + 16 and 32 + 24 rows of Darcy 2D k=3 and 3D k=1 on (a step of
-  // 16,247 cells 1,113 -> 470 us, of 13,547 cells 696 -> 400 us, against the
-  // wavefront kernel with a row per lane); at 12 + 8 it loses (512^2 cells
-  // 2.27 -> 2.88 ms).  27 + 12 belong to the wavefront kernel by contract: its
-  // factor is that of all 27 rows.  Elasticity's products win from 54 + 54.
+  // 16,247 cells 1,061 -> 334 us, of 256 cells 197 -> 136; 13,547 cells 627 -> 302,
+  // 512 cells 184 -> 140, against the wavefront kernel with a row per lane); at
+  // 12 + 8 it loses (512^2 cells 2.09 -> 2.21 ms, 16,247 cells 213 -> 244 us).
+  // 27 + 12 (2D k=2) would win too (512^2 cells 4.86 -> 2.72 ms, 16,247 cells
+  // 392 -> 283 us, 256 cells 144 -> 126) and has not been moved: the suite holds
+  // that this class's resident factors are those of all 27 rows; a mesh moves with
+  // hdg_mesh_set_family.  Elasticity's products win from 54 + 54.
   if ((sh.flux || sh.ref) && sh.ni + sh.nb > (sh.ref ? 44 : 96))
     return sh.ref ? kFamRef : kFamFlux;
   return default_family(sh.ni, sh.nb, true);
@@ -2525,8 +2528,9 @@ bool condense_supported(int n) {
 // generators read one value per right-hand-side entry.
 // (Bounded by the sources' sines and the store of b_i, 0.6 TB/s at 64^3 k=2.
 // Against a wavefront per cell with a lane per point, 27 of 64 in 3D k=2, then a
-// lane per row: 64^3 k=2 1,550 -> 384 us, 512^2 k=2 354 -> 105, 24^3 k=3 229 ->
-// 74, elasticity of 5,814 cells k=2 54 -> 28; 1,728 cells k=3 57 -> 74.)
+// lane per row: 64^3 k=2 1,550 -> 409 us, 512^2 k=2 354 -> 113, 24^3 k=3 229 ->
+// 73, elasticity of 5,814 cells k=2 54 -> 31, 1,728 cells k=3 57 -> 50; of this
+// the potential's rows in the principal basis take 5 to 7 in 100.)
 constexpr int kRhsPoints = 32;
 constexpr int kRhsTiles = 5;  // output tiles of a wavefront in one pass over the points
 
