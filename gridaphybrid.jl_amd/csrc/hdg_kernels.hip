@@ -2494,9 +2494,9 @@ int condense_default_family(const SysShape& sh) {
   // 512 cells 184 -> 140, against the wavefront kernel with a row per lane); at
   // 12 + 8 it loses (512^2 cells 2.09 -> 2.21 ms, 16,247 cells 213 -> 244 us).
   // 27 + 12 (2D k=2) would win too (512^2 cells 4.86 -> 2.72 ms, 16,247 cells
-  // 392 -> 283 us, 256 cells 144 -> 126) and has not been moved: the suite holds
-  // that this class's resident factors are those of all 27 rows; a mesh moves with
-  // hdg_mesh_set_family.  Elasticity's products win from 54 + 54.
+  // 392 -> 283 us, 256 cells 144 -> 126) and has not been moved yet: the rule goes
+  // by class, and a test holds the factors of a 4 x 4 mesh to those of all 27 rows;
+  // hdg_mesh_set_family moves a mesh.  Elasticity's products win from 54 + 54.
   if ((sh.flux || sh.ref) && sh.ni + sh.nb > (sh.ref ? 44 : 96))
     return sh.ref ? kFamRef : kFamFlux;
   return default_family(sh.ni, sh.nb, true);
