@@ -34,16 +34,18 @@
 // (register-grid, workspace-panel and blocked eliminations, the reduced systems
 // formed by kernels of their own and written to memory, the inverses by another):
 //   map level, 4,096 cells of 108 + 54, both maps   17.1 -> 5.1 ms
-//   Darcy 64^3 k=2 (27 + 54 of 108 + 54)            25.2 -> 9.4 ms
-//   Darcy 24^3 k=3 (64 + 96 of 256 + 96)            17.6 -> 3.4 ms
+//   Darcy 64^3 k=2 (27 + 54 of 108 + 54)            25.2 -> 9.2 ms
+//   Darcy 24^3 k=3 (64 + 96 of 256 + 96)            17.6 -> 3.3 ms
 //   elasticity 5,814 cells k=2 (60 + 108)            9.4 -> 1.5 ms
 //   elasticity 1,728 cells k=3 (105 + 180)          12.1 -> 2.1 ms
 // The symmetry of the reduced systems (half of S formed, both halves stored; a
-// column's weights looked up once) and less scratch memory gave 11.9 -> 9.7, 6.2
-// -> 3.5, 2.8 -> 1.6 and 3.3 -> 2.2 ms of the last four, and not storing U, which
-// no recovery of theirs reads, the rest.  The four wavefront kernels of RefGen
-// with two row tiles keep 48 to 64 bytes a lane in scratch memory (168 VGPRs, for
-// three wavefronts a SIMD); no other instance has any.
+// column's weights looked up once) and no scratch memory gave 11.9 -> 9.7, 6.2 ->
+// 3.5, 2.8 -> 1.6 and 3.3 -> 2.2 ms of the last four; not storing U, which no
+// recovery of theirs reads, the rest.  No instance uses scratch memory: the
+// addresses of a generator's tables, hoisted out of the cell loop, had cost the
+// wavefront kernels of two row tiles 36 to 64 bytes a lane, and those of one tile
+// the fourth wavefront a SIMD (RefGen::begin; 64^3 k=2 9.43 -> 9.24 ms, 2D k=3,
+// 16,247 cells, 161 -> 141 us, 3D k=1, 13,547 cells, 127 -> 115 us).
 
 // c ? a : b and c ? a : 0 by masks.  The compiler turns a conditional of loaded
 // values into branches around the loads, one latency after the other; through
@@ -61,6 +63,18 @@ __device__ inline double pick(bool c, double a, double b) {
 __device__ inline double keep_if(bool c, double a) {
   const int m = lane_mask(c);
   return __hiloint2double(__double2hiint(a) & m, __double2loint(a) & m);
+}
+
+// A copy of v the compiler cannot see through: what is built on it (bounds,
+// masks, addresses) stays in the loop or phase that uses it, where hoisted out
+// of the cell loop it spills.
+__device__ inline int opaque_v(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+__device__ inline int opaque_s(int v) {
+  asm volatile("" : "+s"(v));
+  return v;
 }
 
 // Where a generator's entries go: rows and columns of the four blocks, and the
@@ -146,7 +160,8 @@ struct RefGen {
     return PHYS == kDarcy ? -sh.alpha[1 + e * D + a] : sh.alpha[36 + e * D + a];
   }
   __device__ void begin(int64_t cell, Shared& sh) const {
-    const int tid = threadIdx.x, nthreads = blockDim.x;
+    // (opaque: what begin() addresses, kept for the next cell, spills)
+    const int tid = opaque_v(threadIdx.x), nthreads = blockDim.x;
     const int na = T.na, nu = ND * T.nq, nr = nu + T.nb;
     const double* al = M.alpha + cell * kMaxAlpha;
     const double* b = M.srcq + cell * srcq_stride(T);
@@ -336,18 +351,6 @@ __device__ inline void tile_start(const RefGen<PHYS, D, MAXNR, MAXZ>& g,
                                   int nthreads) {
   g.start(sh, tid, nthreads);
   __syncthreads();
-}
-
-// A copy of v the compiler cannot see through: what is built on it (bounds,
-// masks, addresses) stays in the loop or phase that uses it, where hoisted out
-// of the cell loop it spills.
-__device__ inline int opaque_v(int v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-__device__ inline int opaque_s(int v) {
-  asm volatile("" : "+s"(v));
-  return v;
 }
 
 // The factored interior block F of one cell in LDS and the products with it.
