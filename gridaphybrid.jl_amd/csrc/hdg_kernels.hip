@@ -2490,13 +2490,13 @@ static size_t flux_workspace_bytes(int nr, int64_t ncells);
 int condense_default_family(const SysShape& sh) {
   // Where the flux block goes through reference products the reduced system wins
   // from the 48 + 16 and 32 + 24 rows of Darcy 2D k=3 and 3D k=1 on (a step of
-  // 16,247 cells 1,061 -> 334 us, of 256 cells 197 -> 136; 13,547 cells 627 -> 302,
-  // 512 cells 184 -> 140, against the wavefront kernel with a row per lane); at
-  // 12 + 8 it loses (512^2 cells 2.09 -> 2.21 ms, 16,247 cells 213 -> 244 us).
-  // 27 + 12 (2D k=2) would win too (512^2 cells 4.86 -> 2.72 ms, 16,247 cells
-  // 392 -> 283 us, 256 cells 144 -> 126) and has not been moved yet: the rule goes
-  // by class, and a test holds the factors of a 4 x 4 mesh to those of all 27 rows;
-  // hdg_mesh_set_family moves a mesh.  Elasticity's products win from 54 + 54.
+  // 16,247 cells 1,074 -> 322 us, of 256 cells 207 -> 143; 13,547 cells 637 -> 298,
+  // 512 cells 192 -> 150, against the wavefront kernel with a row per lane); at
+  // 12 + 8 it does on many cells only (512^2 2.10 -> 1.99 ms, 16,247 cells 225 ->
+  // 241 us).  27 + 12 (2D k=2) would win too (512^2 cells 4.88 -> 2.46 ms, 16,247
+  // cells 390 -> 268 us, 256 cells 150 -> 133) and has not been moved yet: the rule
+  // goes by class, and a test holds the factors of a 4 x 4 mesh to those of all 27
+  // rows; hdg_mesh_set_family moves a mesh.  Elasticity's products win from 54 + 54.
   if ((sh.flux || sh.ref) && sh.ni + sh.nb > (sh.ref ? 44 : 96))
     return sh.ref ? kFamRef : kFamFlux;
   return default_family(sh.ni, sh.nb, true);
