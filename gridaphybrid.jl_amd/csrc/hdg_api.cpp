@@ -1415,9 +1415,9 @@ int hdg_cell_blocks(hdg_mesh* m, const double** S, const double** g, const int32
 int hdg_local_factors(hdg_mesh* m, const double** U, const double** Y) {
   if (!m) return HDG_ERR_ARG;
   if (!m->want_factors) {
-    m->want_factors = true;
     if (m->condensed)
       if (const int rc = form_factors(m)) return rc;
+    m->want_factors = true;
   }
   if (U) *U = m->mixed ? nullptr : m->pU;
   if (Y) *Y = m->pY;
